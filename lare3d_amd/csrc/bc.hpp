@@ -5,109 +5,147 @@
 // span the full extent of the other two axes (so corners wrap); on a
 // BC_USER axis the MPI exchange is a no-op and the user mirrors / zero
 // walls of boundary.f90 apply.  The reference runs all exchanges (x, y, z)
-// before all user fills (x, y, z); the host launches one kernel per axis in
-// that order.  One launch handles up to 8 fields so that a whole
-// boundary_conditions call is at most three launches.  A BC_OPEN side
-// (openboundary.f90) gets no fill at all: the MPI exchange is a no-op there
-// and the user fills of boundary.f90 apply to BC_USER sides only, so the
-// ghosts keep the far-field values until open_bcs sets the first layer.
+// before all user fills (x, y, z).  A BC_OPEN side (openboundary.f90) gets
+// no fill at all: the MPI exchange is a no-op there and the user fills of
+// boundary.f90 apply to BC_USER sides only, so the ghosts keep the far-field
+// values until open_bcs sets the first layer.
+//
+// All axes of all fields of a call are filled in one launch (k_halo).  Each
+// of the reference's passes copies whole layers, over the full extent of
+// the other two axes, so the value left at a point after the sequence is the
+// old value at (mx(i), my(j), mz(k)), where m of an axis maps a filled layer
+// to its source layer and every other index to itself -- whatever the order
+// of the passes; and it is zero if any wall that zeroes its layers covers
+// the point.  A source layer is never filled itself, so a point that is read
+// is never written and the launch needs no order among its threads.
+//
+// Why one launch: it is bound by launch and load latency on small grids and
+// by the 8-byte stores at both ends of every row on large ones.  A pass per
+// axis (and per sweep one for dm) took 24 launches of about 6.5 us, 164 us
+// of a 16^3 step's 540; the 6 here take 26 us.  At 256^3 the fills of a step
+// went from 0.72 to 0.51 ms.
 
-enum BcOp {
-  BC_NONE = 0,
-  BC_PER_CELL,   // (n+1:n+2) <- (1:2), (-1:0) <- (n-1:n)      cell_xface
-  BC_PER_FACE,   // (n+1:n+2) <- (1:2), (-2:0) <- (n-2:n)      bx_xface / bx_xface1
-  BC_PER_NODE,   // (n:n+2) <- (0:2), (-2:-1) <- (n-2:n-1)     node_xface1 / node_xface
-  BC_MIR_CELL,   // 0 <- 1, -1 <- 2, n+1 <- n, n+2 <- n-1     boundary.f90:134-160 etc.
-  BC_MIR_FACE,   // -1 <- 1, -2 <- 2, n+1 <- n-1, n+2 <- n-2  boundary.f90:68-69,77-78
-  BC_ZERO_NODE,  // -2..0 = 0, n..n+2 = 0                      boundary.f90:260-292
-  BC_DM_CLAMP,   // dm(n+1) <- dm(n), dm(-1) <- dm(0) over transverse 0..n+1 (xremap.f90:906-915)
-  BC_PHI_NEU     // 0 <- 1, -1 <- 1, n+1 <- n, n+2 <- n     phi_mpi walls (initial_conditions.f90:276-291)
+// Layers that a fill may write on one axis: -2, -1, 0, n, n+1, n+2.
+#define HALO_LAYERS 6
+__device__ __forceinline__ int halo_layer(int q, int n) { return q < 3 ? q - 2 : n + q - 3; }
+
+// Source of index c on an axis of n cells for the three staggerings along
+// that axis: cell centres, faces (the normal axis of a face field), nodes.
+// nodez: the wall zeroes the node layer instead (boundary.f90:260-292).
+struct HaloMap {
+  int cell, face, node;
+  bool nodez;
 };
-
-#define BC_MAXF 8
-struct BcSet {
-  void *f[BC_MAXF];
-  int op[BC_MAXF];
-  int wide[BC_MAXF];  // 1: FP64 array, 0: FP32 array
-  int nf;
-  int skip_lo, skip_hi;  // leave the low / high side alone (a BC_OPEN side)
-};
-
-template <class T>
-__device__ __forceinline__ void bc_line(T *a, int op, int base, int st, int n, bool dm_ok, bool lo, bool hi) {
-  switch (op) {
-    case BC_PER_CELL:
-      a[base + (n + 1) * st] = a[base + 1 * st];
-      a[base + (n + 2) * st] = a[base + 2 * st];
-      a[base - 1 * st] = a[base + (n - 1) * st];
-      a[base + 0 * st] = a[base + n * st];
-      break;
-    case BC_PER_FACE:
-      a[base + (n + 1) * st] = a[base + 1 * st];
-      a[base + (n + 2) * st] = a[base + 2 * st];
-      a[base - 2 * st] = a[base + (n - 2) * st];
-      a[base - 1 * st] = a[base + (n - 1) * st];
-      a[base + 0 * st] = a[base + n * st];
-      break;
-    case BC_PER_NODE: {
-      const T v0 = a[base], v1 = a[base + st], v2 = a[base + 2 * st];
-      a[base + n * st] = v0;
-      a[base + (n + 1) * st] = v1;
-      a[base + (n + 2) * st] = v2;
-      a[base - 2 * st] = a[base + (n - 2) * st];
-      a[base - 1 * st] = a[base + (n - 1) * st];
-      break;
+__device__ __forceinline__ HaloMap halo_map(int c, int n, int periodic, int open_lo, int open_hi) {
+  HaloMap m = {c, c, c, false};
+  if (c > 0 && c < n) return m;
+  if (periodic) {
+    // cells: (n+1:n+2) <- (1:2), (-1:0) <- (n-1:n)   cell_xface
+    // faces: the same and -2 <- n-2                  bx_xface / bx_xface1
+    // nodes: (n:n+2) <- (0:2), (-2:-1) <- (n-2:n-1)  node_xface1 / node_xface
+    if (c <= 0) {
+      if (c >= -1) m.cell = c + n;
+      m.face = c + n;
+      if (c < 0) m.node = c + n;
+    } else {
+      if (c > n) m.cell = m.face = c - n;
+      m.node = c - n;
     }
-    case BC_MIR_CELL:
-      if (lo) {
-        a[base + 0 * st] = a[base + 1 * st];
-        a[base - 1 * st] = a[base + 2 * st];
-      }
-      if (hi) {
-        a[base + (n + 1) * st] = a[base + n * st];
-        a[base + (n + 2) * st] = a[base + (n - 1) * st];
-      }
-      break;
-    case BC_MIR_FACE:
-      if (lo) {
-        a[base - 1 * st] = a[base + 1 * st];
-        a[base - 2 * st] = a[base + 2 * st];
-      }
-      if (hi) {
-        a[base + (n + 1) * st] = a[base + (n - 1) * st];
-        a[base + (n + 2) * st] = a[base + (n - 2) * st];
-      }
-      break;
-    case BC_ZERO_NODE:
-      if (lo) {
-        a[base - 2 * st] = (T)0;
-        a[base - 1 * st] = (T)0;
-        a[base + 0 * st] = (T)0;
-      }
-      if (hi) {
-        a[base + n * st] = (T)0;
-        a[base + (n + 1) * st] = (T)0;
-        a[base + (n + 2) * st] = (T)0;
-      }
-      break;
-    case BC_PHI_NEU:
-      a[base + 0 * st] = a[base + 1 * st];
-      a[base - 1 * st] = a[base + 1 * st];
-      a[base + (n + 1) * st] = a[base + n * st];
-      a[base + (n + 2) * st] = a[base + n * st];
-      break;
-    case BC_DM_CLAMP:
-      if (dm_ok) {
-        a[base + (n + 1) * st] = a[base + n * st];
-        a[base - 1 * st] = a[base + 0 * st];
-      }
-      break;
-    default:
-      break;
+    return m;
   }
+  if (c <= 0 ? open_lo : open_hi) return m;
+  // walls: cells 0 <- 1, -1 <- 2, n+1 <- n, n+2 <- n-1 (boundary.f90:134-160);
+  // faces -1 <- 1, -2 <- 2, n+1 <- n-1, n+2 <- n-2 (:68-69, :77-78)
+  m.nodez = true;
+  if (c <= 0) {
+    if (c >= -1) m.cell = 1 - c;
+    if (c < 0) m.face = -c;
+  } else if (c > n) {
+    m.cell = 2 * n + 1 - c;
+    m.face = 2 * n - c;
+  }
+  return m;
 }
 
-__global__ __launch_bounds__(64) void k_bc_axis(Geo g, BcSet s, int axis) {
+// Fields of one fill: the face field (NB = 1: b[0..2]), NC cell fields and
+// NN node fields (0 or 3).
+struct HaloSet {
+  double *b[3];
+  real *cell[2];
+  real *node[3];
+};
+
+// One thread per point of the shell: the z layers over the whole (x, y)
+// extent, the y layers over k = 1..n-1, the x layers over j, k = 1..n-1.  All
+// loads of a point are issued before its stores.
+template <int NB, int NC, int NN>
+__global__ __launch_bounds__(256) void k_halo(Geo g, HaloSet s) {
+  const unsigned t = blockIdx.x * 256u + threadIdx.x;
+  const unsigned wx = (unsigned)g.nx + 5u, wy = (unsigned)g.ny + 5u;
+  const unsigned my = (unsigned)g.ny - 1u, mz = (unsigned)g.nz - 1u;
+  const unsigned nzl = HALO_LAYERS * wx * wy, nyl = HALO_LAYERS * wx * mz, nxl = HALO_LAYERS * my * mz;
+  int i, j, k;
+  if (t < nzl) {
+    const unsigned r = t / wx, l = r / wy;
+    i = (int)(t - r * wx) - 2;
+    j = (int)(r - l * wy) - 2;
+    k = halo_layer((int)l, g.nz);
+  } else if (t < nzl + nyl) {
+    const unsigned u = t - nzl, r = u / wx, l = r / mz;
+    i = (int)(u - r * wx) - 2;
+    j = halo_layer((int)l, g.ny);
+    k = (int)(r - l * mz) + 1;
+  } else if (t < nzl + nyl + nxl) {
+    const unsigned u = t - nzl - nyl, r = u / HALO_LAYERS, q = r / my;
+    i = halo_layer((int)(u - r * HALO_LAYERS), g.nx);
+    j = (int)(r - q * my) + 1;
+    k = (int)q + 1;
+  } else {
+    return;
+  }
+  const HaloMap mx = halo_map(i, g.nx, g.per[0], g.open_lo[0], g.open_hi[0]);
+  const HaloMap my_ = halo_map(j, g.ny, g.per[1], g.open_lo[1], g.open_hi[1]);
+  const HaloMap mz_ = halo_map(k, g.nz, g.per[2], g.open_lo[2], g.open_hi[2]);
+  const int c = g.idx(i, j, k);
+  const bool z = mx.nodez || my_.nodez || mz_.nodez;
+  const int sx = g.idx(mx.face, my_.cell, mz_.cell), sy = g.idx(mx.cell, my_.face, mz_.cell),
+            sz = g.idx(mx.cell, my_.cell, mz_.face), sc = g.idx(mx.cell, my_.cell, mz_.cell),
+            sn = g.idx(mx.node, my_.node, mz_.node);
+  double vb[3] = {0.0, 0.0, 0.0};
+  real vc[2] = {0, 0}, vn[3] = {0, 0, 0};
+  if constexpr (NB) {
+    vb[0] = s.b[0][sx];
+    vb[1] = s.b[1][sy];
+    vb[2] = s.b[2][sz];
+  }
+#pragma unroll
+  for (int q = 0; q < NC; ++q) vc[q] = s.cell[q][sc];
+#pragma unroll
+  for (int q = 0; q < NN; ++q) vn[q] = s.node[q][sn];
+  if constexpr (NB) {
+    if (sx != c) s.b[0][c] = vb[0];
+    if (sy != c) s.b[1][c] = vb[1];
+    if (sz != c) s.b[2][c] = vb[2];
+  }
+  if (NC > 0 && sc != c)
+#pragma unroll
+    for (int q = 0; q < NC; ++q) s.cell[q][c] = vc[q];
+  if (NN > 0 && (z || sn != c))
+#pragma unroll
+    for (int q = 0; q < NN; ++q) s.node[q][c] = z ? (real)0 : vn[q];
+}
+static inline unsigned halo_blocks(const Geo &g) {
+  const long wx = g.nx + 5, wy = g.ny + 5, my = g.ny - 1, mz = g.nz - 1;
+  return (unsigned)((HALO_LAYERS * (wx * wy + wx * mz + my * mz) + 255) / 256);
+}
+
+// Line fills of the potential phi (phi_mpi, initial_conditions.f90:268-291),
+// whose walls copy the first interior layer into both ghost layers.
+enum BcOp {
+  BC_PER_CELL,   // (n+1:n+2) <- (1:2), (-1:0) <- (n-1:n)
+  BC_PHI_NEU     // 0 <- 1, -1 <- 1, n+1 <- n, n+2 <- n
+};
+__global__ __launch_bounds__(64) void k_bc_axis(Geo g, double *__restrict__ a, int op, int axis) {
   // plane coordinates: u runs along the contiguous axis where possible
   const int u = axis == 0 ? 1 : 0;
   const int w = axis == 2 ? 1 : 2;
@@ -121,105 +159,11 @@ __global__ __launch_bounds__(64) void k_bc_axis(Geo g, BcSet s, int axis) {
   c[u] = iu;
   c[w] = iw;
   const int base = g.idx(c[0], c[1], c[2]);  // index of layer 0 on this line
-  const bool dm_ok = iu >= 0 && iu <= g.n(u) + 1 && iw >= 0 && iw <= g.n(w) + 1;
-  const bool lo = !s.skip_lo, hi = !s.skip_hi;
-  for (int q = 0; q < s.nf; ++q) {
-    if (s.wide[q]) bc_line((double *)s.f[q], s.op[q], base, st, n, dm_ok, lo, hi);
-    else bc_line((float *)s.f[q], s.op[q], base, st, n, dm_ok, lo, hi);
-  }
-}
-
-// The x-axis fill with the work spread over the ghost slots of each line:
-// thread (line, slot) does the slot-th (destination <- source) copy of the
-// operation, slots 0..7, lines over the full (y, z) extent -2..n+2.  The
-// copies of one operation touch disjoint destination and source layers
-// (n >= 4), so doing them in parallel gives the sequential result, and the
-// eight lanes of a line share its two end cache lines.
-// Destination and source offsets (along the line) of one slot of a fill.
-struct BcMove {
-  int dst, src;
-  bool zero, act;
-};
-__device__ __forceinline__ BcMove bc_slot(int op, int n, int slot, bool dm_ok) {
-  int dst = 0, src = 0;
-  bool zero = false, act = false;
-  switch (op) {
-    case BC_PER_CELL: {
-      const int d[4] = {n + 1, n + 2, -1, 0}, r[4] = {1, 2, n - 1, n};
-      if (slot < 4) { dst = d[slot]; src = r[slot]; act = true; }
-      break;
-    }
-    case BC_PER_FACE: {
-      const int d[5] = {n + 1, n + 2, -2, -1, 0}, r[5] = {1, 2, n - 2, n - 1, n};
-      if (slot < 5) { dst = d[slot]; src = r[slot]; act = true; }
-      break;
-    }
-    case BC_PER_NODE: {
-      const int d[5] = {n, n + 1, n + 2, -2, -1}, r[5] = {0, 1, 2, n - 2, n - 1};
-      if (slot < 5) { dst = d[slot]; src = r[slot]; act = true; }
-      break;
-    }
-    case BC_MIR_CELL: {
-      const int d[4] = {0, -1, n + 1, n + 2}, r[4] = {1, 2, n, n - 1};
-      if (slot < 4) { dst = d[slot]; src = r[slot]; act = true; }
-      break;
-    }
-    case BC_MIR_FACE: {
-      const int d[4] = {-1, -2, n + 1, n + 2}, r[4] = {1, 2, n - 1, n - 2};
-      if (slot < 4) { dst = d[slot]; src = r[slot]; act = true; }
-      break;
-    }
-    case BC_ZERO_NODE: {
-      const int d[6] = {-2, -1, 0, n, n + 1, n + 2};
-      if (slot < 6) { dst = d[slot]; zero = true; act = true; }
-      break;
-    }
-    case BC_PHI_NEU: {
-      const int d[4] = {0, -1, n + 1, n + 2}, r[4] = {1, 1, n, n};
-      if (slot < 4) { dst = d[slot]; src = r[slot]; act = true; }
-      break;
-    }
-    case BC_DM_CLAMP: {
-      const int d[2] = {n + 1, -1}, r[2] = {n, 0};
-      if (slot < 2 && dm_ok) { dst = d[slot]; src = r[slot]; act = true; }
-      break;
-    }
-    default:
-      break;
-  }
-  BcMove m = {dst, src, zero, act};
-  return m;
-}
-// the slot's move, unless it writes a side that is left alone
-__device__ __forceinline__ BcMove bc_slot_side(int op, int n, int slot, bool dm_ok, const BcSet &s) {
-  BcMove m = bc_slot(op, n, slot, dm_ok);
-  if (m.act && (m.dst <= 0 ? s.skip_lo : s.skip_hi)) m.act = false;
-  return m;
-}
-
-__global__ __launch_bounds__(256) void k_bc_x(Geo g, BcSet s) {
-  const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  const int slot = t & 7, line = t >> 3;
-  const int ly = g.ny + 5;
-  if (line >= ly * (g.nz + 5)) return;
-  const int j = -2 + line % ly, k = -2 + line / ly;
-  const int base = g.idx(0, j, k);
-  const bool dm_ok = j >= 0 && j <= g.ny + 1 && k >= 0 && k <= g.nz + 1;
-  // The fields are distinct arrays, so all loads are issued before any
-  // store (values pass through double, which is exact for FP32 too).
-  BcMove mv[BC_MAXF];
-  double v[BC_MAXF];
-#pragma unroll
-  for (int q = 0; q < BC_MAXF; ++q) {
-    mv[q] = q < s.nf ? bc_slot_side(s.op[q], g.nx, slot, dm_ok, s) : BcMove{0, 0, false, false};
-    v[q] = 0.0;
-    if (mv[q].act && !mv[q].zero)
-      v[q] = s.wide[q] ? ((const double *)s.f[q])[base + mv[q].src] : (double)((const float *)s.f[q])[base + mv[q].src];
-  }
-#pragma unroll
-  for (int q = 0; q < BC_MAXF; ++q) {
-    if (!mv[q].act) continue;
-    if (s.wide[q]) ((double *)s.f[q])[base + mv[q].dst] = v[q];
-    else ((float *)s.f[q])[base + mv[q].dst] = (float)v[q];
-  }
+  const bool per = op == BC_PER_CELL;
+  const double l1 = a[base + (per ? n : 1) * st], l2 = a[base + (per ? n - 1 : 1) * st];
+  const double h1 = a[base + (per ? 1 : n) * st], h2 = a[base + (per ? 2 : n) * st];
+  a[base] = l1;
+  a[base - st] = l2;
+  a[base + (n + 1) * st] = h1;
+  a[base + (n + 2) * st] = h2;
 }

@@ -548,6 +548,23 @@ __device__ __forceinline__ void vl_cell(acc v_advect, double fm, double fi, doub
   Di = vl_di<acc>(dfi, dfu, sign_v, dci, dcu, dbu, phi);
 }
 
+// dm of sweep coordinate m (0..n) at index c, and the halo layers along the
+// sweep that take its value: on a periodic axis (n+1:n+2) <- (1:2) and
+// (-1:0) <- (n-1:n), so the flux formed at 0 itself is not kept; otherwise
+// the clamps dm(n+1) <- dm(n), dm(-1) <- dm(0) (xremap.f90:906-915).  A fill
+// launch of its own took 3 to 7 us per sweep at any size.
+__device__ __forceinline__ void store_dm(real *__restrict__ dm, int c, int MS, int m, int n, int periodic, real v) {
+  if (periodic) {
+    if (m > 0) dm[c] = v;
+    if (m == 1 || m == 2) dm[c + n * MS] = v;
+    if (m >= n - 1) dm[c - n * MS] = v;
+  } else {
+    dm[c] = v;
+    if (m == 0) dm[c - MS] = v;
+    if (m == n) dm[c + MS] = v;
+  }
+}
+
 // Mass flux (x_mass_flux, xremap.f90:474-533), energy flux (x_energy_flux,
 // :539-601) and the density and energy updates (:174-196) of the y and z
 // sweeps (M = 1, 2) in one pass, marching along the sweep axis.  The launch
@@ -558,10 +575,9 @@ __device__ __forceinline__ void vl_cell(acc v_advect, double fm, double fi, doub
 // 1..n, the flux and dm at m-1 carried from the previous point (rounded to
 // the storage type, as stored values are).  A chunk that starts at m0 > 0
 // first forms the fluxes of m0-1, whose dm the chunk below stores.  On a
-// periodic sweep axis the dm halo fill that follows overwrites dm(0) with
-// dm(n), and the energy flux at 0 and the update at 1 take dm(0) after that
-// fill, so there the first chunk forms dm(n) from its own window at n and
-// uses it at 0.  The new density goes to rho_new and the new energy to
+// periodic sweep axis dm(0) takes the value of dm(n) (store_dm), and so do the
+// energy flux at 0 and the update at 1, so there the first chunk forms dm(n)
+// from its own window at n and uses it at 0.  The new density goes to rho_new and the new energy to
 // e_new, since neighbouring chunks still read the old energy; only cells
 // 1..n are written (the halo refresh after the sweep fills the rest).
 template <int M>
@@ -627,7 +643,7 @@ __global__ __launch_bounds__(BX * BY) void k_mass_rho_energy_m(Geo g, Box b, con
     acc vad_p, vad_m, dbu, fu, Di, phi;
     vl_cell(v_advect, r[0], r[1], r[2], r[3], dcm, dci, dcp, d[1], d[2], tdt, vad_p, vad_m, dbu, fu, Di, phi);
     const real dm_own = (fu + Di * ((acc)1.0 - phi)) * v_advect * tdt * area;
-    if (m >= m0) dm[c] = dm_own;
+    if (m >= m0) store_dm(dm, c, MS, m, g.n(M), periodic, dm_own);
     if (!inner) continue;
     const real dmc = (periodic && m == 0) ? dm_wrap : dm_own;
     vl_cell(v_advect, e[0], e[1], e[2], e[3], dcm, dci, dcp, d[1], d[2], tdt, vad_p, vad_m, dbu, fu, Di, phi);
@@ -653,8 +669,7 @@ __global__ __launch_bounds__(BX * BY) void k_mass_rho_energy_m(Geo g, Box b, con
 // one; lanes 1..REX_OUT own their points.  Every point forms dm and its
 // owner stores it; points with transverse 1..n also form the energy flux,
 // and those at x >= 1 update rho and energy.  On a periodic x axis the
-// lanes at x = 0 form dm(n) as well and use it, as the dm halo fill would
-// have made them.
+// lanes at x = 0 form dm(n) as well and use it, the value that dm(0) takes.
 #define REX_OUT 63
 __device__ __forceinline__ acc mass_flux_x(const Geo &g, const real *__restrict__ rho, const real *__restrict__ vel,
                                           const real *__restrict__ db1, int c, int i, int j, int k, acc dt) {
@@ -686,7 +701,7 @@ __global__ __launch_bounds__(BX * BY) void k_mass_rho_energy_x(Geo g, Box b, con
   const int c = g.idx(i, j, k);
   const acc tdt = (acc)dt;
   const real dm_own = mass_flux_x(g, rho1, vel, db1, c, i, j, k, tdt);
-  if (valid && lane >= 1) dm[c] = dm_own;
+  if (valid && lane >= 1) store_dm(dm, c, 1, i, g.nx, periodic, dm_own);
   const bool inner = j >= 1 && j <= g.ny && k >= 1 && k <= g.nz;
   real dmc = dm_own, F = 0;
   if (inner) {

@@ -259,72 +259,27 @@ int read_scalars(int slot, int count, double *out) {
 // ----------------------------------------------------------------------------
 enum FieldKind { FK_CELL, FK_NODE, FK_BX, FK_BY, FK_BZ };
 
-struct BcField {
-  void *a;
-  FieldKind kind;
-};
-
-// FP64 storage: face B (and predictor B); everything else in `real`
-bool wide_kind(FieldKind k) { return k == FK_BX || k == FK_BY || k == FK_BZ || sizeof(real) == sizeof(double); }
-
-int op_for(FieldKind k, int axis, bool periodic) {
-  switch (k) {
-    case FK_CELL: return periodic ? BC_PER_CELL : BC_MIR_CELL;
-    case FK_NODE: return periodic ? BC_PER_NODE : BC_ZERO_NODE;
-    case FK_BX: return axis == 0 ? (periodic ? BC_PER_FACE : BC_MIR_FACE) : (periodic ? BC_PER_CELL : BC_MIR_CELL);
-    case FK_BY: return axis == 1 ? (periodic ? BC_PER_FACE : BC_MIR_FACE) : (periodic ? BC_PER_CELL : BC_MIR_CELL);
-    case FK_BZ: return axis == 2 ? (periodic ? BC_PER_FACE : BC_MIR_FACE) : (periodic ? BC_PER_CELL : BC_MIR_CELL);
-  }
-  return BC_NONE;
-}
-
-int launch_bc_axis(const BcSet &s, int axis, const char *name) {
-  if (axis == 0) {
-    const int lines = (S.n[1] + 5) * (S.n[2] + 5);
-    LAUNCH(name, k_bc_x, dim3((unsigned)((lines * 8 + 255) / 256)), dim3(256), S.g, s);
-    return 0;
-  }
-  const int u = axis == 0 ? 1 : 0, w = axis == 2 ? 1 : 2;
-  dim3 grid((unsigned)((S.n[u] + 5 + 63) / 64), (unsigned)(S.n[w] + 5));
-  LAUNCH(name, k_bc_axis, grid, dim3(64), S.g, s, axis);
-  return 0;
-}
-
-// exchanges on periodic axes (x, y, z), then user fills (x, y, z)
-int apply_bcs(const BcField *f, int nf, const char *name) {
-  for (int pass = 0; pass < 2; ++pass)
-    for (int ax = 0; ax < 3; ++ax) {
-      const bool periodic = S.per[ax];
-      if ((pass == 0) != periodic) continue;
-      BcSet s = {};
-      s.nf = nf;
-      for (int q = 0; q < nf; ++q) {
-        s.f[q] = f[q].a;
-        s.op[q] = op_for(f[q].kind, ax, periodic);
-        s.wide[q] = wide_kind(f[q].kind) ? 1 : 0;
-      }
-      s.skip_lo = S.bc[2 * ax] == LARE_BC_OPEN;
-      s.skip_hi = S.bc[2 * ax + 1] == LARE_BC_OPEN;
-      if (s.skip_lo && s.skip_hi) continue;
-      int rc = launch_bc_axis(s, ax, name);
-      if (rc) return rc;
-    }
+// the fields of h that NB, NC and NN say, every axis at once
+template <int NB, int NC, int NN>
+int fill_halo(const HaloSet &h, const char *name) {
+  LAUNCH(name, (k_halo<NB, NC, NN>), dim3(halo_blocks(S.g)), dim3(256), S.g, h);
   return 0;
 }
 
 int bfield_bcs(double *bx, double *by, double *bz) {
-  BcField f[3] = {{bx, FK_BX}, {by, FK_BY}, {bz, FK_BZ}};
-  return apply_bcs(f, 3, "bc_bfield");
+  return fill_halo<1, 0, 0>({{bx, by, bz}, {nullptr, nullptr}, {nullptr, nullptr, nullptr}}, "bc_bfield");
 }
 int energy_bcs() {
-  BcField f[1] = {{S.energy, FK_CELL}};
-  return apply_bcs(f, 1, "bc_energy");
+  return fill_halo<0, 1, 0>({{nullptr, nullptr, nullptr}, {S.energy, nullptr}, {nullptr, nullptr, nullptr}},
+                            "bc_energy");
 }
-int boundary_conditions() {
-  BcField f[8] = {{S.bx, FK_BX},     {S.by, FK_BY},   {S.bz, FK_BZ},   {S.energy, FK_CELL},
-                  {S.rho, FK_CELL},  {S.vx, FK_NODE}, {S.vy, FK_NODE}, {S.vz, FK_NODE}};
-  return apply_bcs(f, 8, "bc_all");
+int node_bcs(real *ux, real *uy, real *uz, const char *name) {
+  return fill_halo<0, 0, 3>({{nullptr, nullptr, nullptr}, {nullptr, nullptr}, {ux, uy, uz}}, name);
 }
+HaloSet state_halo() {
+  return {{S.bx, S.by, S.bz}, {S.energy, S.rho}, {S.vx, S.vy, S.vz}};
+}
+int boundary_conditions() { return fill_halo<1, 2, 3>(state_halo(), "bc_all"); }
 
 // ----------------------------------------------------------------------------
 // conduction
@@ -594,15 +549,6 @@ int sweep_full(double dt, double pass[3], bool first, bool last) {
     LAUNCH("rho_energy", k_mass_rho_energy_m<AX>, zchunk_grid(march_box(mb, AX)), box_block(), S.g, mb, S.energy,
            S.rho, vel, S.db1, S.dm, S.cv1, S.cv2, S.rho_alt, S.Fe, dt, S.per[AX] ? 1 : 0);
   }
-  {
-    BcSet s = {};
-    s.nf = 1;
-    s.f[0] = S.dm;
-    s.op[0] = S.per[AX] ? BC_PER_CELL : BC_DM_CLAMP;
-    s.wide[0] = wide_kind(FK_CELL) ? 1 : 0;
-    rc = launch_bc_axis(s, AX, "bc_dm");
-    if (rc) return rc;
-  }
   if (S.any_open) {
     // the new energy and density cover cells 1..n; the ghosts of a BC_OPEN
     // side keep their values (no fill there)
@@ -663,9 +609,9 @@ int eulerian_remap(int step, bool predictor) {
   // The B -> face flux scaling (remap.f90:44-67) happens inside the first
   // sweep's CT kernels and the scaling back (remap.f90:102-125) inside the
   // last sweep's update.  In the full remap the last sweep's halo refresh
-  // then runs on B instead of on face fluxes; the B halos it writes are
-  // written again from the same interior by the bfield_bcs that follows the
-  // scaling back in the reference, and nothing reads them in between.
+  // then runs on B instead of on face fluxes, which leaves the halos that the
+  // bfield_bcs after the scaling back in the reference writes from the same
+  // interior.
   if (predictor) {
     for (int q = 0; q < 3; ++q) {
       const int ax = kStrang[c][q];
@@ -686,7 +632,7 @@ int eulerian_remap(int step, bool predictor) {
                      : (ax == 1 ? sweep_full<1>(dt, pass, first, last) : sweep_full<2>(dt, pass, first, last));
     if (rc) return rc;
   }
-  return bfield_bcs(S.bx, S.by, S.bz);
+  return 0;
 }
 
 // ----------------------------------------------------------------------------
@@ -985,8 +931,7 @@ int lagrangian_step() {
       tb = S.bx; S.bx = S.fxr; S.fxr = tb;
       tb = S.by; S.by = S.fyr; S.fyr = tb;
       tb = S.bz; S.bz = S.fzr; S.fzr = tb;
-      BcField f[4] = {{S.bx, FK_BX}, {S.by, FK_BY}, {S.bz, FK_BZ}, {S.energy, FK_CELL}};
-      rc = apply_bcs(f, 4, "bc_resistive");
+      rc = fill_halo<1, 1, 0>(state_halo(), "bc_resistive");
       if (rc) return rc;
     }
     S.dt = actual_dt;
@@ -1032,11 +977,8 @@ int lagrangian_step() {
            S.bpx, S.bpy, S.bpz, S.rho_v, S.al1, S.al2, S.al3, S.gamma_boris, S.vx1, S.vy1, S.vz1, S.dt2, S.cv1,
            nullptr, nullptr, nullptr);
   }
-  {
-    BcField f[3] = {{S.vx1, FK_NODE}, {S.vy1, FK_NODE}, {S.vz1, FK_NODE}};
-    rc = apply_bcs(f, 3, "bc_v1");
-    if (rc) return rc;
-  }
+  rc = node_bcs(S.vx1, S.vy1, S.vz1, "bc_v1");
+  if (rc) return rc;
   if (S.any_open) {
     // v1 = v over the whole array before the predictor remap
     // (lagran.F90:1051-1053); the forces then set nodes 0..n and
@@ -1081,20 +1023,13 @@ int lagrangian_step() {
   if (S.any_open) {
     // velocity_bcs, open_bcs, then (with the end of lagrangian_step)
     // energy_bcs and density_bcs (lagran.F90:408-412, :196-198)
-    BcField fv[3] = {{S.vx, FK_NODE}, {S.vy, FK_NODE}, {S.vz, FK_NODE}};
-    rc = apply_bcs(fv, 3, "bc_lagrangian");
+    rc = node_bcs(S.vx, S.vy, S.vz, "bc_lagrangian");
     if (rc) return rc;
     rc = open_bcs();
     if (rc) return rc;
-    BcField fc[2] = {{S.energy, FK_CELL}, {S.rho, FK_CELL}};
-    return apply_bcs(fc, 2, "bc_lagrangian");
+    return fill_halo<0, 2, 0>(state_halo(), "bc_lagrangian");
   }
-  {
-    BcField f[5] = {{S.energy, FK_CELL}, {S.rho, FK_CELL}, {S.vx, FK_NODE}, {S.vy, FK_NODE}, {S.vz, FK_NODE}};
-    rc = apply_bcs(f, 5, "bc_lagrangian");
-    if (rc) return rc;
-  }
-  return 0;
+  return fill_halo<0, 2, 3>(state_halo(), "bc_lagrangian");
 }
 
 // ----------------------------------------------------------------------------
@@ -2150,25 +2085,19 @@ int api_potential_field(const lare_potential *pf, int32_t *iterations, double *r
   auto phi_bcs = [&]() -> int {
     // phi_mpi: exchanges on periodic axes, the z boundaries, then the
     // zero-gradient x and y walls
+    auto line = [&](int ax, int op) -> int {
+      const int u = ax == 0 ? 1 : 0, wa = ax == 2 ? 1 : 2;
+      LAUNCH("bc_phi", k_bc_axis, dim3((unsigned)((S.n[u] + 5 + 63) / 64), (unsigned)(S.n[wa] + 5)), dim3(64), S.g,
+             phi, op, ax);
+      return 0;
+    };
     for (int ax = 0; ax < 3; ++ax) {
-      if (!S.per[ax]) continue;
-      BcSet b = {};
-      b.nf = 1;
-      b.f[0] = phi;
-      b.op[0] = BC_PER_CELL;
-      b.wide[0] = 1;
-      int rc = launch_bc_axis(b, ax, "bc_phi");
+      int rc = S.per[ax] ? line(ax, BC_PER_CELL) : 0;
       if (rc) return rc;
     }
     LAUNCH("phi_zbc", k_phi_zbc, box_grid(zb), box_block(), S.g, zb, phi, flux0);
     for (int ax = 0; ax < 2; ++ax) {
-      if (S.per[ax]) continue;
-      BcSet b = {};
-      b.nf = 1;
-      b.f[0] = phi;
-      b.op[0] = BC_PHI_NEU;
-      b.wide[0] = 1;
-      int rc = launch_bc_axis(b, ax, "bc_phi");
+      int rc = S.per[ax] ? 0 : line(ax, BC_PHI_NEU);
       if (rc) return rc;
     }
     return 0;

@@ -31,9 +31,11 @@ struct Geo {
   __device__ __forceinline__ double cv(int i, int j, int k) const { return dxb[i] * dyb[j] * dzb[k]; }
 };
 
-// Index box [lo, hi] inclusive per axis.
+// Index box [lo, hi] inclusive per axis; zc: points per block along the march
+// axis of a marching launch (1 .. ZCHUNK, march_chunk).
 struct Box {
   int x0, x1, y0, y1, z0, z1;
+  int zc;
 };
 
 #define BX 64
@@ -73,9 +75,29 @@ static inline unsigned plane_blocks(const Box &b) {
 }
 static inline dim3 box_grid(const Box &b) { return dim3(plane_blocks(b), 1, (unsigned)(b.z1 - b.z0 + 1)); }
 static inline dim3 box_block() { return dim3(BX, BY, 1); }
+#define ZCHUNK 8  // most points a block marches over
 static inline Box mkbox(int x0, int x1, int y0, int y1, int z0, int z1) {
-  Box b = {x0, x1, y0, y1, z0, z1};
+  Box b = {x0, x1, y0, y1, z0, z1, ZCHUNK};
   return b;
+}
+
+// Points a block marches over, for a launch of per_plane blocks on each of
+// `points` march positions: the longest chunk (each chunk re-reads the
+// planes before it) that still launches MARCH_BLOCKS blocks, two for each of
+// the 256 CUs.  Below that a launch is bound by the serial chain of loads of
+// its march, not by bandwidth: with chunks of 8 a marching kernel took 14 to
+// 25 us at 16^3 and at 64^3 alike, and with this rule 4 to 6 and 7 to 10 us.
+// Steps of the resistive sheet (FP64, ms) with chunks of 8 | targets of 256 |
+// 512 | 1024 | 2048 blocks:
+//   16^3 0.34 | 0.205 | 0.200 | 0.197 | 0.197    64^3 0.47 | 0.403 | 0.365 | 0.394 | 0.406
+//   96^3 0.79 | 0.774 | 0.729 | 0.739 | 0.823   128^3 1.55 | 1.545 | 1.545 | 1.548 | 1.528
+#ifndef MARCH_BLOCKS
+#define MARCH_BLOCKS 512
+#endif
+static inline int march_chunk(unsigned per_plane, int points) {
+  int c = ZCHUNK;
+  while (c > 1 && (long)per_plane * ((points + c - 1) / c) < MARCH_BLOCKS) c >>= 1;
+  return c;
 }
 
 __device__ __forceinline__ double dmin(double a, double b) { return a < b ? a : b; }
@@ -122,22 +144,21 @@ __device__ __forceinline__ void block_reduce_store(double (&v)[NV], const int *o
 }
 
 // Columns of a z-marching launch: thread (i, j) of the flattened plane tile
-// blockIdx.x walks planes k0 .. k1 of its chunk (ZCHUNK planes per block).
-#define ZCHUNK 8
+// blockIdx.x walks planes k0 .. k1 of its chunk (b.zc planes per block).
 #define ZRANGE(b, k0, k1)                                             \
-  const int k0 = (b).z0 + (int)blockIdx.z * ZCHUNK;                    \
-  const int k1 = k0 + ZCHUNK - 1 < (b).z1 ? k0 + ZCHUNK - 1 : (b).z1;
+  const int k0 = (b).z0 + (int)blockIdx.z * (b).zc;                    \
+  const int k1 = k0 + (b).zc - 1 < (b).z1 ? k0 + (b).zc - 1 : (b).z1;
 #define ZCOLUMN(b, i, j, k0, k1) \
   PLANE_POS(b, i, j)             \
   ZRANGE(b, k0, k1)              \
   if (j > (b).y1) return;
 
-// Columns of a launch that marches along axis M (1 = y, 2 = z) for ZCHUNK
+// Columns of a launch that marches along axis M (1 = y, 2 = z) for b.zc
 // points: the flattened tile covers x and the other transverse axis, whose
 // index is p; MJ/MK give j and k at march coordinate m.  The grid is the
 // zchunk grid of the box with its y and z ranges swapped when M = 1.
 #define MCOLUMN(M, b, i, p, m0, m1)                                                         \
-  const Box pb_ = (M) == 2 ? (b) : Box{(b).x0, (b).x1, (b).z0, (b).z1, (b).y0, (b).y1};   \
+  const Box pb_ = (M) == 2 ? (b) : Box{(b).x0, (b).x1, (b).z0, (b).z1, (b).y0, (b).y1, (b).zc};   \
   PLANE_POS(pb_, i, p)                                                                     \
   ZRANGE(pb_, m0, m1)                                                                      \
   if (p > pb_.y1) return;

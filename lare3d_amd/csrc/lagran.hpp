@@ -581,7 +581,7 @@ struct EPlane {
 // (:1270-1288, cells 1..n) takes curlb of the same eight nodes, rounded to
 // the storage type as stored values are, and energy = MAX(energy, 0)
 // (:1305) follows over the cell box -1..n+2.  A block is a tile of RS_ROWS rows of
-// 64 nodes marching in z over ZCHUNK planes (plus plane k0-1 for the EMFs of
+// 64 nodes marching in z over b.zc planes (plus plane k0-1 for the EMFs of
 // plane k-1); lane 0 and row 0 only supply neighbour EMFs, which pass through
 // LDS, so a tile writes RS_OUT_X x RS_OUT_Y nodes.  Neighbouring tiles still
 // read the old B, so the new B goes to bxo..bzo at every node of the launch

@@ -199,7 +199,7 @@ template <int AX> struct CtComp {
 //   t1 = t1 - F1 + F1(s-1), t2 = t2 - F2 + F2(s-1) along the sweep;
 //   a = a + F1 - F1(c - AS1) + F2 - F2(c - AS2) across the transverse axes.
 // A block is a tile of the plane across the march axis, rows of lanes along
-// x, covering a chunk of CTS_CHUNK points along the march.  It first forms
+// x, covering a chunk of mc (at most CTS_CHUNK) points along the march.  It first forms
 // the fluxes of the chunk and of the point before it into LDS, then, after
 // one barrier, writes its points, taking each flux and its neighbours along
 // the march (the previous point), along x (the lane below) and along the
@@ -212,6 +212,7 @@ template <int AX> struct CtComp {
 #ifndef CTS_CHUNK
 #define CTS_CHUNK 8
 #endif
+static_assert(ZCHUNK <= CTS_CHUNK, "march_chunk gives the CT sweeps at most ZCHUNK points");
 
 __device__ __forceinline__ bool in_box(const Box &b, int i, int j, int k) {
   return i >= b.x0 && i <= b.x1 && j >= b.y0 && j <= b.y1 && k >= b.z0 && k <= b.z1;
@@ -260,7 +261,7 @@ __device__ __forceinline__ void ct_store(const Wid &wd, int c, int i, int j, int
 // y and z sweeps (M = 1, 2).  Rows of CTM_XW lanes along x, CTM_ROWS rows
 // along the other transverse axis P (which is t2's axis, so F2a comes from
 // the row below; t1 is bx, so F1a comes from the lane below).  Two phases
-// per chunk of CTS_CHUNK points along the sweep:
+// per chunk of mc points along the sweep:
 //  1. each thread marches its column and forms the fluxes of points m0-1 ..
 //     m1 into LDS, holding the four-point stencils of db1, of both fields'
 //     widths and of their quotients field / width in registers (a quotient
@@ -282,7 +283,7 @@ __global__ __launch_bounds__(CTM_THREADS) void k_ct_sweep_m(Geo g, const double 
                                                             double *__restrict__ t2o, double *__restrict__ ao,
                                                             const real *__restrict__ vel,
                                                             const real *__restrict__ db1, int VS1, int GS1, int VS2,
-                                                            int GS2, double dt, int ntx, Box bt1, Box ba1, Box bt2,
+                                                            int GS2, double dt, int ntx, int mc, Box bt1, Box ba1, Box bt2,
                                                             Box ba2) {
   constexpr int T1 = CtComp<M>::T1, T2 = CtComp<M>::T2;
   constexpr int P = M == 2 ? 1 : 2;
@@ -294,8 +295,8 @@ __global__ __launch_bounds__(CTM_THREADS) void k_ct_sweep_m(Geo g, const double 
   const int i = -3 + tx * (CTM_XW - 1) + xl;
   const int p = -3 + ty * (CTM_ROWS - 1) + row;
   const int n = g.n(M), nx = g.nx, nP = g.n(P);
-  const int m0 = -2 + (int)blockIdx.z * CTS_CHUNK;
-  const int m1 = m0 + CTS_CHUNK - 1 < n + 2 ? m0 + CTS_CHUNK - 1 : n + 2;
+  const int m0 = -2 + (int)blockIdx.z * mc;
+  const int m1 = m0 + mc - 1 < n + 2 ? m0 + mc - 1 : n + 2;
   // a flux column lies in the flux box across the sweep; an output column
   // in the padded box, off the halo lane and row
   const bool col = i >= -1 && i <= nx + 1 && p >= -1 && p <= nP + 1;
@@ -405,7 +406,7 @@ __global__ __launch_bounds__(CTX_THREADS) void k_ct_sweep_x(Geo g, const double 
                                                             double *__restrict__ t2o, double *__restrict__ ao,
                                                             const real *__restrict__ vel,
                                                             const real *__restrict__ db1, int GS1, int VS2, double dt,
-                                                            int ntx, Box bt1, Box ba1, Box bt2, Box ba2) {
+                                                            int ntx, int mc, Box bt1, Box ba1, Box bt2, Box ba2) {
   constexpr int T1 = CtComp<0>::T1, T2 = CtComp<0>::T2;
   __shared__ real fl[CTS_CHUNK + 1][2][CTX_ROWS][64];
   const int lane = (int)threadIdx.x & 63, row = (int)threadIdx.x >> 6;
@@ -415,8 +416,8 @@ __global__ __launch_bounds__(CTX_THREADS) void k_ct_sweep_x(Geo g, const double 
   const int j = -3 + ty * (CTX_ROWS - 1) + row;
   const int nx = g.nx, ny = g.ny, nz = g.nz;
   const int Z = g.sz;
-  const int k0 = -2 + (int)blockIdx.z * CTS_CHUNK;
-  const int k1 = k0 + CTS_CHUNK - 1 < nz + 2 ? k0 + CTS_CHUNK - 1 : nz + 2;
+  const int k0 = -2 + (int)blockIdx.z * mc;
+  const int k1 = k0 + mc - 1 < nz + 2 ? k0 + mc - 1 : nz + 2;
   // quotient points x = -1..n+2 and flux points x = -1..n+1 of flux rows
   // y = -1..n+1; output points of the padded box off the halo lanes and row
   const bool qrow = j >= -1 && j <= ny + 1 && i >= -1 && i <= nx + 2;
@@ -861,7 +862,7 @@ __device__ __forceinline__ VertexV vertex_march(const Geo &g, const real *__rest
 // geometry) and the updates of xremap.f90:282-329 (nodes 0..n) in one pass.
 // Waves cover runs of 64 points of a plane of the launch box (the whole
 // padded box) flattened along x, successive waves overlapping by two, and
-// march in z over ZCHUNK planes, keeping the upper plane of vertex cells for
+// march in z over b.zc planes, keeping the upper plane of vertex cells for
 // the next node: each lane forms the vertex quantities of its node, takes
 // rho_v of node i+1 from the lane to its right and the flux and dm_v of node
 // i-1 from the lane to its left; lanes 1..MOMX_OUT write.  Every point is

@@ -170,23 +170,30 @@ Box cell_box() { return mkbox(-1, nx() + 2, -1, ny() + 2, -1, nz() + 2); }
 Box interior() { return mkbox(1, nx(), 1, ny(), 1, nz()); }
 Box nodes0n() { return mkbox(0, nx(), 0, ny(), 0, nz()); }
 
-// grid of k_resist over the padded box: tiles of RS_OUT_X x RS_OUT_Y
-// written nodes, ZCHUNK planes per block
-dim3 resist_grid(int *tiles_x) {
-  const Box fb = full_box();
-  *tiles_x = (fb.x1 - fb.x0 + RS_OUT_X) / RS_OUT_X;
-  const int tiles_y = (fb.y1 - fb.y0 + RS_OUT_Y) / RS_OUT_Y;
-  return dim3((unsigned)(*tiles_x * tiles_y), 1, (unsigned)((fb.z1 - fb.z0 + ZCHUNK) / ZCHUNK));
-}
-
-// grid of a z-marching launch: BX*BY columns, ZCHUNK planes per block
-dim3 zchunk_grid(const Box &b) {
-  return dim3(plane_blocks(b), 1, (unsigned)((b.z1 - b.z0 + 1 + ZCHUNK - 1) / ZCHUNK));
+// grid of k_resist over the padded box b: tiles of RS_OUT_X x RS_OUT_Y
+// written nodes, b.zc (set here) planes per block
+dim3 resist_grid(Box &b, int *tiles_x) {
+  *tiles_x = (b.x1 - b.x0 + RS_OUT_X) / RS_OUT_X;
+  const int tiles = *tiles_x * ((b.y1 - b.y0 + RS_OUT_Y) / RS_OUT_Y);
+  b.zc = march_chunk((unsigned)tiles, b.z1 - b.z0 + 1);
+  return dim3((unsigned)tiles, 1, (unsigned)((b.z1 - b.z0 + b.zc) / b.zc));
 }
 
 // the box whose zchunk grid a launch marching along axis M (1, 2) uses:
 // y and z ranges swapped for M = 1 (MCOLUMN)
-Box march_box(const Box &b, int M) { return M == 2 ? b : mkbox(b.x0, b.x1, b.z0, b.z1, b.y0, b.y1); }
+Box march_box(const Box &b, int M) {
+  return M == 2 ? b : Box{b.x0, b.x1, b.z0, b.z1, b.y0, b.y1, b.zc};
+}
+
+// b with the chunk of a launch of plane_blocks columns marching along axis M
+Box marched(Box b, int M = 2) {
+  const Box m = march_box(b, M);
+  b.zc = march_chunk(plane_blocks(m), m.z1 - m.z0 + 1);
+  return b;
+}
+
+// grid of a z-marching launch: BX*BY columns, b.zc planes per block
+dim3 zchunk_grid(const Box &b) { return dim3(plane_blocks(b), 1, (unsigned)((b.z1 - b.z0 + b.zc) / b.zc)); }
 
 // reduction over partials of a grid launched from index 0 on every axis
 dim3 grid_from0(int x1, int y1, int z1) { return box_grid(mkbox(0, x1, 0, y1, 0, z1)); }
@@ -318,31 +325,37 @@ int calc_s_stages() {
   return 0;
 }
 
-// grid of the z-marching stage kernels over the interior box: waves of
-// RKL_OUT cells over rows of x0-1..x1, ZCHUNK planes per block
-dim3 rkl2_grid(const Box &in) {
-  const long npts = (long)(in.x1 - in.x0 + 2) * (in.y1 - in.y0 + 1);
-  const long waves = (npts + RKL_OUT - 1) / RKL_OUT;
-  return dim3((unsigned)((waves + BY - 1) / BY), 1, (unsigned)((in.z1 - in.z0 + 1 + ZCHUNK - 1) / ZCHUNK));
+// blocks per plane of a launch of waves that own `out` points each of a plane
+// of npts points
+unsigned wave_blocks(long npts, int out) { return (unsigned)(((npts + out - 1) / out + BY - 1) / BY); }
+
+// grid of the z-marching stage kernels over the interior box (in.zc set
+// here): waves of RKL_OUT cells over rows of x0-1..x1
+dim3 rkl2_grid(Box &in) {
+  const unsigned pb = wave_blocks((long)(in.x1 - in.x0 + 2) * (in.y1 - in.y0 + 1), RKL_OUT);
+  in.zc = march_chunk(pb, in.z1 - in.z0 + 1);
+  return dim3(pb, 1, (unsigned)((in.z1 - in.z0 + in.zc) / in.zc));
 }
 // stage 1 from E0 (ghosts as stored): Lc and Y1 = E0 + mu_t1 dt Lc
 int rkl2_stage1(const real *E0, real *Yout, CondArgs ca, double mu_t1) {
-  const Box in = interior();
+  Box in = interior();
+  const dim3 gr = rkl2_grid(in);
   // the stage-1 read is direct: no ghost mapping, BC_OPEN or not
   if (ca.xi)
-    LAUNCH("rkl2_stage1", (k_rkl2_z<TMODE_DIRECT, 1, true, false>), rkl2_grid(in), box_block(), S.g, in, E0, E0, E0,
+    LAUNCH("rkl2_stage1", (k_rkl2_z<TMODE_DIRECT, 1, true, false>), gr, box_block(), S.g, in, E0, E0, E0,
            S.rho, S.bx, S.by, S.bz, S.larsen, S.Lc, Yout, ca, 0.0, 0.0, 0.0, mu_t1, 0.0);
   else
-    LAUNCH("rkl2_stage1", (k_rkl2_z<TMODE_DIRECT, 1, false, false>), rkl2_grid(in), box_block(), S.g, in, E0, E0, E0,
+    LAUNCH("rkl2_stage1", (k_rkl2_z<TMODE_DIRECT, 1, false, false>), gr, box_block(), S.g, in, E0, E0, E0,
            S.rho, S.bx, S.by, S.bz, S.larsen, S.Lc, Yout, ca, 0.0, 0.0, 0.0, mu_t1, 0.0);
   return 0;
 }
 // stage j >= 2 from Y2 (and Y1, E0, Lc) under a ghost-read mode
 int rkl2_stage(int mode, const real *Y2, const real *Y1, const real *E0, real *Yout, CondArgs ca, double mu, double nu,
                double one_m_mu_nu, double mu_t, double gam_t) {
-  const Box in = interior();
+  Box in = interior();
+  const dim3 gr = rkl2_grid(in);
 #define RKL2_STAGE(M, P, O)                                                                                       \
-  LAUNCH("rkl2_stage", (k_rkl2_z<M, 0, P, O>), rkl2_grid(in), box_block(), S.g, in, Y2, Y1, E0, S.rho, S.bx, S.by, \
+  LAUNCH("rkl2_stage", (k_rkl2_z<M, 0, P, O>), gr, box_block(), S.g, in, Y2, Y1, E0, S.rho, S.bx, S.by, \
          S.bz, S.larsen, S.Lc, Yout, ca, mu, nu, one_m_mu_nu, mu_t, gam_t)
   if (S.any_open) {
     if (mode == TMODE_STALE) {
@@ -452,32 +465,34 @@ int ct_sweep(const double *const in[3], double *const out[3], const real *vel, d
     // x sweep: va1 = z and ga2 = z (see the flux table above); tiles of
     // CTX_W points in x by CTX_ROWS - 1 rows in y, marching in z
     const int ntx = (N[0] + 5 + CTX_W - 1) / CTX_W, nty = (N[1] + 5 + CTX_ROWS - 2) / (CTX_ROWS - 1);
-    const dim3 grid((unsigned)(ntx * nty), 1, (unsigned)((N[2] + 5 + CTS_CHUNK - 1) / CTS_CHUNK));
+    const int mc = march_chunk((unsigned)(ntx * nty), N[2] + 5);
+    const dim3 grid((unsigned)(ntx * nty), 1, (unsigned)((N[2] + 4 + mc) / mc));
     if (sc > 0)
       LAUNCH("ct_sweep", k_ct_sweep_x<1>, grid, blk, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX], vel,
-             S.db1, strides(ga1), strides(va2), dt, ntx, bt1, ba1, bt2, ba2);
+             S.db1, strides(ga1), strides(va2), dt, ntx, mc, bt1, ba1, bt2, ba2);
     else if (sc < 0)
       LAUNCH("ct_sweep", k_ct_sweep_x<-1>, grid, blk, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX], vel,
-             S.db1, strides(ga1), strides(va2), dt, ntx, bt1, ba1, bt2, ba2);
+             S.db1, strides(ga1), strides(va2), dt, ntx, mc, bt1, ba1, bt2, ba2);
     else
       LAUNCH("ct_sweep", k_ct_sweep_x<0>, grid, blk, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX], vel,
-             S.db1, strides(ga1), strides(va2), dt, ntx, bt1, ba1, bt2, ba2);
+             S.db1, strides(ga1), strides(va2), dt, ntx, mc, bt1, ba1, bt2, ba2);
   } else {
     // y and z sweeps march along the sweep axis; tiles of CTM_XW - 1 points
     // in x by CTM_ROWS - 1 rows along the other transverse axis
     const int P = AX == 2 ? 1 : 2;
     const int ntx = (N[0] + 5 + CTM_XW - 2) / (CTM_XW - 1), nty = (N[P] + 5 + CTM_ROWS - 2) / (CTM_ROWS - 1);
-    const dim3 grid((unsigned)(ntx * nty), 1, (unsigned)((N[AX] + 5 + CTS_CHUNK - 1) / CTS_CHUNK));
+    const int mc = march_chunk((unsigned)(ntx * nty), N[AX] + 5);
+    const dim3 grid((unsigned)(ntx * nty), 1, (unsigned)((N[AX] + 4 + mc) / mc));
     const dim3 blkm(CTM_THREADS, 1, 1);
     if (sc > 0)
       LAUNCH("ct_sweep", (k_ct_sweep_m<AX, 1>), grid, blkm, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX],
-             vel, S.db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, bt1, ba1, bt2, ba2);
+             vel, S.db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, mc, bt1, ba1, bt2, ba2);
     else if (sc < 0)
       LAUNCH("ct_sweep", (k_ct_sweep_m<AX, -1>), grid, blkm, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX],
-             vel, S.db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, bt1, ba1, bt2, ba2);
+             vel, S.db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, mc, bt1, ba1, bt2, ba2);
     else
       LAUNCH("ct_sweep", (k_ct_sweep_m<AX, 0>), grid, blkm, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX],
-             vel, S.db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, bt1, ba1, bt2, ba2);
+             vel, S.db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, mc, bt1, ba1, bt2, ba2);
   }
   return 0;
 }
@@ -497,11 +512,12 @@ template <int AX>
 int sweep_predictor(double dt, bool first, bool last) {
   // the last pass also forms the predictor energy and pressure
   const PredP pr = {S.energy, S.rho, S.visc_heat, S.p0, S.pp, S.p.gamma, S.dt2, eos_args()};
+  const Box cb = marched(cell_box());
   if (last)
-    LAUNCH("geom", (k_geom<AX, 1>), zchunk_grid(cell_box()), box_block(), S.g, cell_box(), S.vx, S.vy, S.vz, S.cv1,
+    LAUNCH("geom", (k_geom<AX, 1>), zchunk_grid(cb), box_block(), S.g, cb, S.vx, S.vy, S.vz, S.cv1,
            S.cv2, S.db1, dt, 1.0, 1.0, 1.0, pr);
   else
-    LAUNCH("geom", (k_geom<AX, 0>), zchunk_grid(cell_box()), box_block(), S.g, cell_box(), S.vx, S.vy, S.vz, S.cv1,
+    LAUNCH("geom", (k_geom<AX, 0>), zchunk_grid(cb), box_block(), S.g, cb, S.vx, S.vy, S.vz, S.cv1,
            S.cv2, S.db1, dt, 1.0, 1.0, 1.0, pr);
   const real *vel = AX == 0 ? S.vx : (AX == 1 ? S.vy : S.vz);
   if (first) {
@@ -522,7 +538,8 @@ template <int AX>
 int sweep_full(double dt, double pass[3], bool first, bool last) {
   const int N[3] = {nx(), ny(), nz()};
   const real *vel = AX == 0 ? S.vx1 : (AX == 1 ? S.vy1 : S.vz1);
-  LAUNCH("geom", (k_geom<AX, 2>), zchunk_grid(cell_box()), box_block(), S.g, cell_box(), S.vx1, S.vy1, S.vz1, S.cv1,
+  const Box cb = marched(cell_box());
+  LAUNCH("geom", (k_geom<AX, 2>), zchunk_grid(cb), box_block(), S.g, cb, S.vx1, S.vy1, S.vz1, S.cv1,
          S.cv2, S.db1, dt, pass[0], pass[1], pass[2], PredP{});
   {
     const double *const B[3] = {S.bx, S.by, S.bz};
@@ -535,14 +552,14 @@ int sweep_full(double dt, double pass[3], bool first, bool last) {
   int hi[3] = {N[0] + 1, N[1] + 1, N[2] + 1};
   hi[AX] = N[AX];
   Box mb = mkbox(0, hi[0], 0, hi[1], 0, hi[2]);
+  if (AX != 0) mb = marched(mb, AX);
   // mass flux, energy flux and the density and energy updates in one pass
   // over the mass flux's box (updates on cells 1..n); the new energy lands
   // in the energy flux array, which then swaps roles with the energy array
   // (the new density goes to rho_alt as before)
   if constexpr (AX == 0) {
-    const long npts = (long)(mb.x1 - mb.x0 + 1) * (mb.y1 - mb.y0 + 1);
-    const long waves = (npts + REX_OUT - 1) / REX_OUT;
-    const dim3 gx((unsigned)((waves + BY - 1) / BY), 1, (unsigned)(mb.z1 - mb.z0 + 1));
+    const dim3 gx(wave_blocks((long)(mb.x1 - mb.x0 + 1) * (mb.y1 - mb.y0 + 1), REX_OUT), 1,
+                  (unsigned)(mb.z1 - mb.z0 + 1));
     LAUNCH("rho_energy", k_mass_rho_energy_x, gx, box_block(), S.g, mb, S.energy, S.rho, vel, S.db1, S.dm, S.cv1,
            S.cv2, S.rho_alt, S.Fe, dt, S.per[AX] ? 1 : 0);
   } else {
@@ -565,12 +582,12 @@ int sweep_full(double dt, double pass[3], bool first, bool last) {
     // padded box (rho1 = rho before this sweep's update, which went to
     // rho_alt); the new velocities land in the flux arrays, which then swap
     // roles with the velocity arrays
-    const Box xb = full_box();
+    Box xb = full_box();
     if constexpr (AX == 0) {
-      const long npts = (long)(xb.x1 - xb.x0 + 1) * (xb.y1 - xb.y0 + 1);
-      const long out = S.delta_ke ? MOMX_OUT_RKE : MOMX_OUT;
-      const long waves = (npts + out - 1) / out;
-      const dim3 gx((unsigned)((waves + BY - 1) / BY), 1, (unsigned)((xb.z1 - xb.z0 + ZCHUNK) / ZCHUNK));
+      const unsigned pb = wave_blocks((long)(xb.x1 - xb.x0 + 1) * (xb.y1 - xb.y0 + 1),
+                                      S.delta_ke ? MOMX_OUT_RKE : MOMX_OUT);
+      xb.zc = march_chunk(pb, xb.z1 - xb.z0 + 1);
+      const dim3 gx(pb, 1, (unsigned)((xb.z1 - xb.z0 + xb.zc) / xb.zc));
       if (S.delta_ke)
         LAUNCH("mom_remap", k_mom_remap_x<true>, gx, box_block(), S.g, xb, S.vx, S.vy, S.vz, vel, S.db1, S.rho,
                S.cv1, S.cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk);
@@ -578,6 +595,7 @@ int sweep_full(double dt, double pass[3], bool first, bool last) {
         LAUNCH("mom_remap", k_mom_remap_x<false>, gx, box_block(), S.g, xb, S.vx, S.vy, S.vz, vel, S.db1, S.rho,
                S.cv1, S.cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk);
     } else {
+      xb = marched(xb, AX);
       if (S.delta_ke)
         LAUNCH("mom_remap", (k_mom_remap_m<AX, true>), zchunk_grid(march_box(xb, AX)), box_block(), S.g, xb, S.vx,
                S.vy, S.vz, vel, S.db1, S.rho, S.cv1, S.cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk);
@@ -640,7 +658,7 @@ int eulerian_remap(int step, bool predictor) {
 // ----------------------------------------------------------------------------
 int eta_calc() {
   if (S.p.resistive_mhd) {
-    const Box eb = mkbox(-1, nx() + 1, -1, ny() + 1, -1, nz() + 1);
+    const Box eb = marched(mkbox(-1, nx() + 1, -1, ny() + 1, -1, nz() + 1));
     LAUNCH("eta", k_eta, zchunk_grid(eb), box_block(), S.g, eb, S.bx, S.by, S.bz, S.eta,
                S.p.eta_background, S.p.eta0, S.p.j_max);
   } else {
@@ -832,7 +850,7 @@ int lagrangian_step() {
   const int N0 = nx(), N1 = ny(), N2 = nz();
   LagArgs a = lag_args();  // dt = previous step's dt (Q1)
   {
-    const Box vb = mkbox(-1, N0 + 1, -1, N1 + 1, -1, N2 + 1);
+    const Box vb = marched(mkbox(-1, N0 + 1, -1, N1 + 1, -1, N2 + 1));
     const EosArgs eq = eos_args();
 #define VERTEX_PREP(GB, PI)                                                                                        \
   LAUNCH("vertex_prep", (k_vertex_prep<GB, PI>), zchunk_grid(vb), box_block(), S.g, vb, S.rho, S.energy, S.bx, S.by, \
@@ -851,11 +869,11 @@ int lagrangian_step() {
     LAUNCH_BOX("damp_apply", k_damp_apply, nodes0n(), S.vx, S.vy, S.vz, S.qx, S.qy, S.qz, S.dt);
   }
   {
-    const Box ab = mkbox(-1, N0 + 1, -1, N1 + 2, 0, N2 + 2);
+    const Box ab = marched(mkbox(-1, N0 + 1, -1, N1 + 2, 0, N2 + 2));
     LAUNCH("alpha", k_alpha, zchunk_grid(ab), box_block(), S.g, ab, S.vx, S.vy, S.vz, S.rho_v, S.cs_v, S.al1, S.al2,
            S.al3, a);
   }
-  const Box vdb = mkbox(0, N0 + 1, 0, N1 + 1, 0, N2 + 1);
+  const Box vdb = marched(mkbox(0, N0 + 1, 0, N1 + 1, 0, N2 + 1));
   dim3 gr = zchunk_grid(vdb);
   if (S.pi_eos)
     LAUNCH("visc_dt", k_visc_dt<true>, gr, box_block(), S.g, vdb, S.vx, S.vy, S.vz, S.rho, S.energy, S.bx, S.by, S.bz,
@@ -894,9 +912,9 @@ int lagrangian_step() {
     // k_resist, which writes the new B to the fxr..fzr arrays; they then
     // swap roles with bx..bz.  The B and energy halos of a substep are
     // refreshed together.
-    const Box fb = full_box();
+    Box fb = full_box();
     int tiles_x;
-    const dim3 g2 = resist_grid(&tiles_x);
+    const dim3 g2 = resist_grid(fb, &tiles_x);
     if ((size_t)g2.x * g2.y * g2.z > S.partial_cap)
       return fail(LARE_E_ARG, "resistive grid of %u blocks exceeds the partial buffer", g2.x * g2.z);
     for (int sc = 1; sc <= substeps; ++sc) {
@@ -956,13 +974,14 @@ int lagrangian_step() {
   }
 
   // predictor-corrector (lagran.F90:208-478)
+  const Box nb = marched(nodes0n()), ib = marched(interior());
   if (S.p.cauchy) {
     // the Cauchy solution for the cell-centred B1 (B1 cv1 in the spare
     // predictor-B arrays), cv1 and the predictor pressure; no predictor remap
     real *b1[3] = {(real *)S.bpx, (real *)S.bpy, (real *)S.bpz};
     LAUNCH_BOX("cauchy_b", k_cauchy_b, cell_box(), S.vx, S.vy, S.vz, S.bx, S.by, S.bz, S.cv1, b1[0], b1[1], b1[2],
                S.energy, S.rho, S.visc_heat, S.p0, S.pp, S.p.gamma, S.dt2, eos_args());
-    LAUNCH("force", k_force<true>, zchunk_grid(nodes0n()), box_block(), S.g, nodes0n(), S.vx, S.vy, S.vz, S.pp,
+    LAUNCH("force", k_force<true>, zchunk_grid(nb), box_block(), S.g, nb, S.vx, S.vy, S.vz, S.pp,
            S.bx, S.by, S.bz, S.rho_v, S.al1, S.al2, S.al3, S.gamma_boris, S.vx1, S.vy1, S.vz1, S.dt2, S.cv1, b1[0],
            b1[1], b1[2]);
   } else {
@@ -973,7 +992,7 @@ int lagrangian_step() {
     if (rc) return rc;
     // the predictor energy and pressure were formed in the predictor
     // remap's last geometry pass
-    LAUNCH("force", k_force<false>, zchunk_grid(nodes0n()), box_block(), S.g, nodes0n(), S.vx, S.vy, S.vz, S.pp,
+    LAUNCH("force", k_force<false>, zchunk_grid(nb), box_block(), S.g, nb, S.vx, S.vy, S.vz, S.pp,
            S.bpx, S.bpy, S.bpz, S.rho_v, S.al1, S.al2, S.al3, S.gamma_boris, S.vx1, S.vy1, S.vz1, S.dt2, S.cv1,
            nullptr, nullptr, nullptr);
   }
@@ -991,13 +1010,13 @@ int lagrangian_step() {
     rc = open_save();
     if (rc) return rc;
   }
-  dim3 g3 = zchunk_grid(interior());
+  dim3 g3 = zchunk_grid(ib);
   if (S.cool_v)
-    LAUNCH("shock_corr", k_shock_corr<true>, g3, box_block(), S.g, interior(), S.vx, S.vy, S.vz, S.vx1, S.vy1, S.vz1,
+    LAUNCH("shock_corr", k_shock_corr<true>, g3, box_block(), S.g, ib, S.vx, S.vy, S.vz, S.vx1, S.vy1, S.vz1,
            S.al1, S.al2, S.al3, S.pp, S.energy, S.rho, S.visc_dep, S.Fx, S.Fy, S.Fz, S.cool_v, S.p.alpha_av,
            S.partial, S.dt);
   else
-    LAUNCH("shock_corr", k_shock_corr<false>, g3, box_block(), S.g, interior(), S.vx, S.vy, S.vz, S.vx1, S.vy1, S.vz1,
+    LAUNCH("shock_corr", k_shock_corr<false>, g3, box_block(), S.g, ib, S.vx, S.vy, S.vz, S.vx1, S.vy1, S.vz1,
            S.al1, S.al2, S.al3, S.pp, S.energy, S.rho, S.visc_dep, S.Fx, S.Fy, S.Fz, S.cool_v, S.p.alpha_av,
            S.partial, S.dt);
   rc = final_reduce(g3, 1, 0, 8, 1);
@@ -1265,7 +1284,8 @@ int api_init(const lare_grid *grid, const lare_params *params) {
   dim3 gr = grid_from0(n[0] + 2, n[1] + 2, n[2] + 2);
   S.partial_cap = (size_t)gr.x * gr.y * gr.z * 4;
   int tiles_x;
-  const dim3 grs = resist_grid(&tiles_x);
+  Box rb = full_box();
+  const dim3 grs = resist_grid(rb, &tiles_x);
   if ((size_t)grs.x * grs.y * grs.z > S.partial_cap) S.partial_cap = (size_t)grs.x * grs.y * grs.z;
   // + RED_ROWS x RED_MAXV level-1 results after the per-block partials
   HIPCHK(hipMalloc((void **)&S.partial, sizeof(double) * (S.partial_cap + RED_ROWS * RED_MAXV)));

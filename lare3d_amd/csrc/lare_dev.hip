@@ -19,6 +19,7 @@
 #include <string.h>
 
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/lare3d_dev.h"

@@ -1054,10 +1054,12 @@ int lagrangian_step() {
 // ----------------------------------------------------------------------------
 // memory
 // ----------------------------------------------------------------------------
+#include "transfer.hpp"
 void sur_free();
 void free_all() {
   sur_free();
   if (S.stream) (void)hipStreamSynchronize(S.stream);
+  xfer_free();
   for (void *p : S.allocs) (void)hipFree(p);
   S.allocs.clear();
   if (S.metric) (void)hipFree(S.metric);
@@ -1097,32 +1099,33 @@ void lower_of(FieldKind k, int lo[3]) {
   if (k == FK_BZ) lo[2] = -2;
 }
 
-// host staging buffer of one element type
+// adds the transfer of one device box to or from a host Fortran array (FP64,
+// reference bounds); a NULL array is left out
 template <class T>
-std::vector<T> &stage_buf() {
-  static std::vector<T> v;
-  return v;
+void xfer_add(XferSet &s, T *dev, double *host, FieldKind k) {
+  if (!host) return;
+  XferField &f = s.f[s.nf++];
+  f.dev = dev;
+  f.host = host;
+  f.wide = sizeof(T) == sizeof(double);
+  lower_of(k, f.lo);
+  f.first = s.total;
+  s.total += (unsigned long)(nx() + 3 - f.lo[0]) * (ny() + 3 - f.lo[1]) * (nz() + 3 - f.lo[2]);
 }
-
-// copy one field between a host Fortran array (FP64, reference bounds) and
-// its padded device box, converting to the device storage type
-template <class T>
-int xfer(T *dev, double *host, FieldKind k, bool to_dev) {
-  int lo[3];
-  lower_of(k, lo);
-  const long ex = nx() + 2 - lo[0] + 1, ey = ny() + 2 - lo[1] + 1;
-  std::vector<T> &st = stage_buf<T>();
-  if (st.size() != S.ntot) st.assign(S.ntot, (T)0);
-  HIPCHK(hipMemcpy(st.data(), dev, sizeof(T) * S.ntot, hipMemcpyDeviceToHost));
-  for (int kk = lo[2]; kk <= nz() + 2; ++kk)
-    for (int jj = lo[1]; jj <= ny() + 2; ++jj)
-      for (int ii = lo[0]; ii <= nx() + 2; ++ii) {
-        const long h = ((long)(kk - lo[2]) * ey + (jj - lo[1])) * ex + (ii - lo[0]);
-        if (to_dev) st[S.g.idx(ii, jj, kk)] = (T)host[h];
-        else host[h] = (double)st[S.g.idx(ii, jj, kk)];
-      }
-  if (to_dev) HIPCHK(hipMemcpy(dev, st.data(), sizeof(T) * S.ntot, hipMemcpyHostToDevice));
-  return 0;
+XferSet state_xfer(const lare_fields *f) {
+  XferSet s = {};
+  xfer_add(s, S.rho, f->rho, FK_CELL);
+  xfer_add(s, S.energy, f->energy, FK_CELL);
+  xfer_add(s, S.vx, f->vx, FK_NODE);
+  xfer_add(s, S.vy, f->vy, FK_NODE);
+  xfer_add(s, S.vz, f->vz, FK_NODE);
+  xfer_add(s, S.bx, f->bx, FK_BX);
+  xfer_add(s, S.by, f->by, FK_BY);
+  xfer_add(s, S.bz, f->bz, FK_BZ);
+  xfer_add(s, S.eta, f->eta, FK_CELL);
+  xfer_add(s, S.visc_dep, f->visc_dep, FK_CELL);
+  xfer_add(s, S.ohmic_dep, f->ohmic_dep, FK_CELL);
+  return s;
 }
 
 // ============================================================================
@@ -1307,20 +1310,10 @@ int api_upload(const lare_fields *f) {
     return fail(LARE_E_ARG, "lare_dev_upload: missing field");
   if (S.p.use_viscous_damping && !f->visc3) return fail(LARE_E_ARG, "visc3 required with viscous damping");
   HIPCHK(hipStreamSynchronize(S.stream));
-  int rc = 0;
-  rc |= xfer(S.rho, f->rho, FK_CELL, true);
-  rc |= xfer(S.energy, f->energy, FK_CELL, true);
-  rc |= xfer(S.vx, f->vx, FK_NODE, true);
-  rc |= xfer(S.vy, f->vy, FK_NODE, true);
-  rc |= xfer(S.vz, f->vz, FK_NODE, true);
-  rc |= xfer(S.bx, f->bx, FK_BX, true);
-  rc |= xfer(S.by, f->by, FK_BY, true);
-  rc |= xfer(S.bz, f->bz, FK_BZ, true);
-  if (f->visc3) rc |= xfer(S.visc3, f->visc3, FK_NODE, true);
-  if (f->eta) rc |= xfer(S.eta, f->eta, FK_CELL, true);
-  if (f->visc_dep) rc |= xfer(S.visc_dep, f->visc_dep, FK_CELL, true);
-  if (f->ohmic_dep) rc |= xfer(S.ohmic_dep, f->ohmic_dep, FK_CELL, true);
-  if (rc) return fail(LARE_E_STATE, "upload failed: %s", g_err);
+  XferSet x = state_xfer(f);
+  xfer_add(x, S.visc3, f->visc3, FK_NODE);
+  int rc = transfer(x, true);
+  if (rc) return rc;
   S.loaded = true;
   return 0;
 }
@@ -1329,20 +1322,7 @@ int api_download(lare_fields *f) {
   if (!S.loaded) return fail(LARE_E_STATE, "lare_dev_download before lare_dev_upload");
   if (!f) return fail(LARE_E_ARG, "lare_dev_download: NULL");
   HIPCHK(hipStreamSynchronize(S.stream));
-  int rc = 0;
-  if (f->rho) rc |= xfer(S.rho, f->rho, FK_CELL, false);
-  if (f->energy) rc |= xfer(S.energy, f->energy, FK_CELL, false);
-  if (f->vx) rc |= xfer(S.vx, f->vx, FK_NODE, false);
-  if (f->vy) rc |= xfer(S.vy, f->vy, FK_NODE, false);
-  if (f->vz) rc |= xfer(S.vz, f->vz, FK_NODE, false);
-  if (f->bx) rc |= xfer(S.bx, f->bx, FK_BX, false);
-  if (f->by) rc |= xfer(S.by, f->by, FK_BY, false);
-  if (f->bz) rc |= xfer(S.bz, f->bz, FK_BZ, false);
-  if (f->eta) rc |= xfer(S.eta, f->eta, FK_CELL, false);
-  if (f->visc_dep) rc |= xfer(S.visc_dep, f->visc_dep, FK_CELL, false);
-  if (f->ohmic_dep) rc |= xfer(S.ohmic_dep, f->ohmic_dep, FK_CELL, false);
-  if (rc) return fail(LARE_E_STATE, "download failed: %s", g_err);
-  return 0;
+  return transfer(state_xfer(f), false);
 }
 
 int api_get_scalars(lare_scalars *o) {
@@ -1433,11 +1413,12 @@ int api_get_neutral(double *xi_h, double *ep_h) {
   if ((xi_h && !S.xi) || (ep_h && !S.eta_perp))
     return fail(LARE_E_STATE, "get_neutral: the partially ionised arrays are off");
   HIPCHK(hipStreamSynchronize(S.stream));
-  int rc = 0;
-  if (xi_h) rc = xfer(S.xi, xi_h, FK_CELL, false);
-  if (!rc && ep_h) {
-    rc = xfer(S.eta_perp, ep_h, FK_CELL, false);
-    if (rc) return rc;
+  XferSet x = {};
+  xfer_add(x, S.xi, xi_h, FK_CELL);
+  xfer_add(x, S.eta_perp, ep_h, FK_CELL);
+  int rc = transfer(x, false);
+  if (rc) return rc;
+  if (ep_h) {
     // the array exists at nodes 0..n only (neutral.f90:73-131)
     const long ex = nx() + 4, ey = ny() + 4, ez = nz() + 4;
     for (long k = 0; k < ez; ++k)

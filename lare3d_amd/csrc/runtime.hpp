@@ -2078,20 +2078,18 @@ int api_potential_field(const lare_potential *pf, int32_t *iterations, double *r
   HIPCHK(hipStreamSynchronize(S.stream));
   HIPCHK(hipMemcpy(flux0, pf->flux0, sizeof(double) * (size_t)N0 * N1, hipMemcpyHostToDevice));
   LAUNCH_BOX("fill", k_fill64, full_box(), phi, 0.0);
-  LAUNCH("sor_reset", k_sor_reset, dim3(1), dim3(64), S.dscal);
   const int ncol = (N0 + 1) / 2;
-  const dim3 gs((unsigned)(((long)ncol * N1 + BX * BY - 1) / (BX * BY)));
+  const dim3 gs((unsigned)(((long)ncol * N1 + 63) / 64));
   const Box zb = mkbox(-1, N0 + 2, -1, N1 + 2, 0, 0);
-  const double w = pf->omega, dx1 = pf->dx1, dy1 = pf->dy1, dz1 = pf->dz1;
+  auto line = [&](int ax, int op) -> int {
+    const int u = ax == 0 ? 1 : 0, wa = ax == 2 ? 1 : 2;
+    LAUNCH("bc_phi", k_bc_axis, dim3((unsigned)((S.n[u] + 5 + 63) / 64), (unsigned)(S.n[wa] + 5)), dim3(64), S.g, phi,
+           op, ax);
+    return 0;
+  };
   auto phi_bcs = [&]() -> int {
     // phi_mpi: exchanges on periodic axes, the z boundaries, then the
     // zero-gradient x and y walls
-    auto line = [&](int ax, int op) -> int {
-      const int u = ax == 0 ? 1 : 0, wa = ax == 2 ? 1 : 2;
-      LAUNCH("bc_phi", k_bc_axis, dim3((unsigned)((S.n[u] + 5 + 63) / 64), (unsigned)(S.n[wa] + 5)), dim3(64), S.g,
-             phi, op, ax);
-      return 0;
-    };
     for (int ax = 0; ax < 3; ++ax) {
       int rc = S.per[ax] ? line(ax, BC_PER_CELL) : 0;
       if (rc) return rc;
@@ -2103,26 +2101,44 @@ int api_potential_field(const lare_potential *pf, int32_t *iterations, double *r
     }
     return 0;
   };
-  const int batch = 32;
-  double h[5] = {0, 0, 0, 0, 0};
-  for (;;) {
-    for (int q = 0; q < batch; ++q) {
-      for (int z1 = 1; z1 <= 2; ++z1) {
-        LAUNCH("sor", k_sor_pass, gs, box_block(), S.g, phi, z1, w, dx1, dy1, dz1, S.dscal + 12, S.partial);
-        int rc = final_reduce(gs, 1, 1, 9 + z1, 0);
-        if (rc) return rc;
-        rc = phi_bcs();
-        if (rc) return rc;
-      }
-      LAUNCH("sor_check", k_sor_check, dim3(1), dim3(64), S.dscal, pf->fractional_error, pf->max_iterations);
-    }
-    int rc = read_scalars(10, 5, h);
-    if (rc) return rc;
-    if (h[2] != 0.0) break;
+  // the batch state lives in the level-1 rows of the reductions
+  static_assert(sizeof(SorBatch) <= sizeof(double) * RED_ROWS * RED_MAXV, "batch state");
+  SorBatch *const sb = (SorBatch *)(S.partial + S.partial_cap);
+  SorBatch hb;
+  SorArgs sa = {pf->omega, pf->dx1, pf->dy1, pf->dz1, pf->fractional_error, 0, 0, 0, 1};
+  int *const maps[2] = {&sa.mapx, &sa.mapy};
+  bool ghost[2] = {false, false};  // periodic with an odd number of points
+  for (int ax = 0; ax < 2; ++ax) {
+    ghost[ax] = S.per[ax] && (S.n[ax] & 1);
+    *maps[ax] = !S.per[ax] ? 1 : (ghost[ax] ? 0 : 2);
   }
+  int its = 0;
+  double res = 0.0;
+  for (bool done = false; !done;) {
+    LAUNCH("sor_reset", k_sor_reset, dim3(1), dim3(64), sb);
+    const int batch = pf->max_iterations - its < SOR_BATCH ? pf->max_iterations - its : SOR_BATCH;
+    for (sa.q = 0; sa.q < batch; ++sa.q)
+      for (int z1 = 1; z1 <= 2; ++z1) {
+        LAUNCH("sor", k_sor_pass, gs, dim3(64), S.g, phi, flux0, z1, sa, sb);
+        sa.first = 0;
+        for (int ax = 0; ax < 2; ++ax) {
+          int rc = ghost[ax] ? line(ax, BC_PER_CELL) : 0;
+          if (rc) return rc;
+        }
+      }
+    HIPCHK(hipMemcpyAsync(&hb, sb, sizeof(hb), hipMemcpyDeviceToHost, S.stream));
+    HIPCHK(hipStreamSynchronize(S.stream));
+    for (int q = 0; q < batch && !done; ++q) {
+      memcpy(&res, &hb.err[q], sizeof(res));
+      ++its;
+      done = res < pf->fractional_error || its >= pf->max_iterations;
+    }
+  }
+  int rc = phi_bcs();
+  if (rc) return rc;
   // B = -grad phi, bfield_bcs, scale by the largest bz below, bfield_bcs
   LAUNCH_BOX("phi_to_b", k_phi_to_b, full_box(), phi, S.bx, S.by, S.bz);
-  int rc = bfield_bcs(S.bx, S.by, S.bz);
+  rc = bfield_bcs(S.bx, S.by, S.bz);
   if (rc) return rc;
   const Box lb = mkbox(1, N0, 1, N2, 0, 0);
   const dim3 gb = box_grid(lb);
@@ -2135,8 +2151,8 @@ int api_potential_field(const lare_potential *pf, int32_t *iterations, double *r
   double bm;
   rc = read_scalars(15, 1, &bm);
   if (rc) return rc;
-  if (iterations) *iterations = (int32_t)h[3];
-  if (residual) *residual = h[4];
+  if (iterations) *iterations = its;
+  if (residual) *residual = res;
   if (bz_max) *bz_max = -bm;
   return 0;
 }

@@ -41,8 +41,8 @@ __device__ __forceinline__ A vl_di(double dfi, double dfu, double sign_v, A dci,
 }
 
 // Inputs of the predictor energy and pressure (lagran.F90:234-249), which
-// the predictor remap's last geometry pass (CV = 1) forms on cells 0..n+1
-// from the cv1 it has just formed (p0 is the start-of-step pressure).
+// k_geom_pred forms on cells 0..n+1 from the predictor volume (p0 is the
+// start-of-step pressure).
 struct PredP {
   const real *energy, *rho, *visc_heat, *p0;
   real *pp;
@@ -50,79 +50,126 @@ struct PredP {
   EosArgs eq;  // partially ionised pressure when eq.xi is set
 };
 
-// Lagrangian geometry of a sweep (xremap.f90:57-105 and analogues).
-// Velocities are the time-centred ones (v in predictor mode).  The node
-// velocities of planes k and k-1 are kept in registers while marching in z.
-// CV selects the outputs: 0 = d?b1 only (which needs only the sweep
-// component of the velocity), 1 = cv1 and d?b1 (and the predictor pressure
-// from pr), 2 = cv1, cv2 and d?b1.
-template <int AX, int CV>
-__global__ __launch_bounds__(BX * BY) void k_geom(Geo g, Box b, const real *__restrict__ ux, const real *__restrict__ uy,
-                       const real *__restrict__ uz, real *__restrict__ cv1, real *__restrict__ cv2,
-                       real *__restrict__ db1, double dt, double xpass, double ypass, double zpass, PredP pr) {
+// Face-averaged velocities at the two faces of a cell along each axis, from
+// the node velocities of planes k (h) and k-1 (l) at the four in-plane nodes;
+// sums in the order of u(c) + u(c-Y) + u(c-Z) + u(c-Y-Z) etc.
+template <int A>
+__device__ __forceinline__ acc face_diff(const Quad &h, const Quad &l) {
+  const acc q4 = 0.25;
+  if (A == 0) {
+    const acc b = (h.p0 + h.py + l.p0 + l.py) * q4, m = (h.px + h.pxy + l.px + l.pxy) * q4;
+    return b - m;
+  }
+  if (A == 1) {
+    const acc b = (h.p0 + h.px + l.p0 + l.px) * q4, m = (h.py + h.pxy + l.py + l.pxy) * q4;
+    return b - m;
+  }
+  const acc b = (h.p0 + h.px + h.py + h.pxy) * q4, m = (l.p0 + l.px + l.py + l.pxy) * q4;
+  return b - m;
+}
+
+// Geometry of a predictor remap (xremap.f90:57-105 with every pass flag 1, and
+// analogues), all three sweeps at once, and the predictor pressure.  Nothing
+// that the three sweeps' geometry depends on changes between them (the node
+// velocities are the step's v), so one pass over the velocities forms the
+// widths d?b1 of all three, and the volume cv1 that the pressure needs stays
+// in a register.  LAST is the axis of the last sweep, whose geometry the
+// reference's predictor pressure uses: it sets the order of the volume's
+// three terms.  Three passes, which stored cv1 as well, took 457 us at 256^3,
+// this one 378 us.
+template <int LAST>
+__global__ __launch_bounds__(BX * BY) void k_geom_pred(Geo g, Box b, const real *__restrict__ ux,
+                                                       const real *__restrict__ uy, const real *__restrict__ uz,
+                                                       real *__restrict__ dx1, real *__restrict__ dy1,
+                                                       real *__restrict__ dz1, double dt, PredP pr) {
   ZCOLUMN(b, i, j, k0, k1);
-  constexpr bool NX = CV > 0 || AX == 0, NY = CV > 0 || AX == 1, NZ = CV > 0 || AX == 2;
   const int Y = g.sy;
   const int cb = g.idx(i, j, k0 - 1);
-  Quad ax = {}, ay = {}, az = {};  // plane k-1
-  if (NX) ax = quad_back(ux, cb, Y);
-  if (NY) ay = quad_back(uy, cb, Y);
-  if (NZ) az = quad_back(uz, cb, Y);
+  Quad lx = quad_back(ux, cb, Y), ly = quad_back(uy, cb, Y), lz = quad_back(uz, cb, Y);  // plane k-1
+  const acc dxb = (acc)g.dxb[i], dyb = (acc)g.dyb[j], tdt = (acc)dt;
+  const bool pin = i >= 0 && i <= g.nx + 1 && j >= 0 && j <= g.ny + 1;
   for (int k = k0; k <= k1; ++k) {
     const int c = g.idx(i, j, k);
-    Quad bx_ = {}, by_ = {}, bz_ = {};  // plane k
-    if (NX) bx_ = quad_back(ux, c, Y);
-    if (NY) by_ = quad_back(uy, c, Y);
-    if (NZ) bz_ = quad_back(uz, c, Y);
-    // sums in the order of u(c) + u(c-Y) + u(c-Z) + u(c-Y-Z) etc.
-    const acc q4 = 0.25, tdt = (acc)dt;
-    const acc vxb = (bx_.p0 + bx_.py + ax.p0 + ax.py) * q4;
-    const acc vxbm = (bx_.px + bx_.pxy + ax.px + ax.pxy) * q4;
-    const acc vyb = (by_.p0 + by_.px + ay.p0 + ay.px) * q4;
-    const acc vybm = (by_.py + by_.pxy + ay.py + ay.pxy) * q4;
-    const acc vzb = (bz_.p0 + bz_.px + bz_.py + bz_.pxy) * q4;
-    const acc vzbm = (az.p0 + az.px + az.py + az.pxy) * q4;
-    const acc dxb = (acc)g.dxb[i], dyb = (acc)g.dyb[j], dzb = (acc)g.dzb[k];
-    acc d1;
-    if (AX == 0) d1 = dxb + (vxb - vxbm) * tdt;
-    else if (AX == 1) d1 = dyb + (vyb - vybm) * tdt;
-    else d1 = dzb + (vzb - vzbm) * tdt;
-    if (CV > 0) {
+    const Quad hx = quad_back(ux, c, Y), hy = quad_back(uy, c, Y), hz = quad_back(uz, c, Y);
+    const acc dvx = face_diff<0>(hx, lx), dvy = face_diff<1>(hy, ly), dvz = face_diff<2>(hz, lz);
+    const acc dzb = (acc)g.dzb[k];
+    if (pin && k >= 0 && k <= g.nz + 1) {
+      const acc tx = dvx / dxb, ty = dvy / dyb, tz = dvz / dzb;
+      const acc dv1 = (LAST == 0 ? ty + tz + tx : (LAST == 1 ? tx + tz + ty : tx + ty + tz)) * tdt;
       const acc cv = (acc)g.cv(i, j, k);
-      acc dv1, dv2;
-      if (AX == 0) {
-        const acc tA = (acc)ypass * (vyb - vybm) / dyb;
-        const acc tB = (acc)zpass * (vzb - vzbm) / dzb;
-        dv1 = (tA + tB + (vxb - vxbm) / dxb) * tdt;
-        dv2 = (tA + tB) * tdt;
-      } else if (AX == 1) {
-        const acc tA = (acc)xpass * (vxb - vxbm) / dxb;
-        const acc tB = (acc)zpass * (vzb - vzbm) / dzb;
-        dv1 = (tA + tB + (vyb - vybm) / dyb) * tdt;
-        dv2 = (tA + tB) * tdt;
-      } else {
-        const acc tA = (acc)xpass * (vxb - vxbm) / dxb;
-        const acc tB = (acc)ypass * (vyb - vybm) / dyb;
-        dv1 = (tA + tB + (vzb - vzbm) / dzb) * tdt;
-        dv2 = (tA + tB) * tdt;
-      }
       const real c1 = cv * ((acc)1.0 + dv1);
-      cv1[c] = c1;
-      if (CV > 1) cv2[c] = cv * ((acc)1.0 + dv2);
-      if (CV == 1 && i >= 0 && i <= g.nx + 1 && j >= 0 && j <= g.ny + 1 && k >= 0 && k <= g.nz + 1) {
-        // predictor energy and pressure (lagran.F90:234-249)
-        const acc r = pr.rho[c];
-        const acc dv = c1 / cv - (acc)1.0;
-        acc e1 = pr.energy[c] - pr.p0[c] * dv / r;
-        e1 = e1 + pr.visc_heat[c] * (acc)pr.dt2 / r;
-        const acc ei = pr.eq.xi ? eos_e<true>(e1, pr.eq, c) : eos_e<false>(e1, pr.eq, c);
-        pr.pp[c] = ei * ((acc)pr.gamma - (acc)1.0) * r * cv / c1;
-      }
+      // predictor energy and pressure (lagran.F90:234-249)
+      const acc r = pr.rho[c];
+      const acc dv = c1 / cv - (acc)1.0;
+      acc e1 = pr.energy[c] - pr.p0[c] * dv / r;
+      e1 = e1 + pr.visc_heat[c] * (acc)pr.dt2 / r;
+      const acc ei = pr.eq.xi ? eos_e<true>(e1, pr.eq, c) : eos_e<false>(e1, pr.eq, c);
+      pr.pp[c] = ei * ((acc)pr.gamma - (acc)1.0) * r * cv / c1;
     }
-    db1[c] = d1;
-    ax = bx_;
-    ay = by_;
-    az = bz_;
+    dx1[c] = dxb + dvx * tdt;
+    dy1[c] = dyb + dvy * tdt;
+    dz1[c] = dzb + dvz * tdt;
+    lx = hx;
+    ly = hy;
+    lz = hz;
+  }
+}
+
+// Geometry of a full sweep along AX (xremap.f90:57-105 and analogues, from
+// the time-centred velocities).  The node velocities of planes k and k-1 are
+// kept in registers while marching in z.  The pass flags take the axes
+// already swept out of the volumes:
+//   cv1 = cv (1 + dt (sum over the axes not swept before)),
+//   cv2 = cv (1 + dt (sum over the axes left after this sweep)),
+// and v1 does not change during the remap, so cv1 of a sweep is cv2 of the
+// one before, bit for bit (a flag of 0 adds a zero to the sum, and the sum of
+// two terms does not depend on their order), and cv2 of the last is cv.
+// Only what is new is formed and stored:
+//   REST = 3, first sweep: d?b1, cv1 and cv2;
+//   REST = the axis left, second sweep: d?b1 and cv2;
+//   REST = -1, last sweep: d?b1.
+// The three passes of a remap at 256^3 took 677 us when each formed all
+// three, and 458 us now; the last sweep's readers form cv2 from the widths.
+template <int AX, int REST>
+__global__ __launch_bounds__(BX * BY) void k_geom(Geo g, Box b, const real *__restrict__ ux,
+                                                  const real *__restrict__ uy, const real *__restrict__ uz,
+                                                  real *__restrict__ cv1, real *__restrict__ cv2,
+                                                  real *__restrict__ db1, double dt) {
+  ZCOLUMN(b, i, j, k0, k1);
+  constexpr bool NX = REST == 3 || AX == 0 || REST == 0, NY = REST == 3 || AX == 1 || REST == 1,
+                 NZ = REST == 3 || AX == 2 || REST == 2;
+  const int Y = g.sy;
+  const int cb = g.idx(i, j, k0 - 1);
+  Quad lx = {}, ly = {}, lz = {};  // plane k-1
+  if (NX) lx = quad_back(ux, cb, Y);
+  if (NY) ly = quad_back(uy, cb, Y);
+  if (NZ) lz = quad_back(uz, cb, Y);
+  const acc dxb = (acc)g.dxb[i], dyb = (acc)g.dyb[j], tdt = (acc)dt;
+  for (int k = k0; k <= k1; ++k) {
+    const int c = g.idx(i, j, k);
+    Quad hx = {}, hy = {}, hz = {};  // plane k
+    if (NX) hx = quad_back(ux, c, Y);
+    if (NY) hy = quad_back(uy, c, Y);
+    if (NZ) hz = quad_back(uz, c, Y);
+    const acc dvx = face_diff<0>(hx, lx), dvy = face_diff<1>(hy, ly), dvz = face_diff<2>(hz, lz);
+    const acc dzb = (acc)g.dzb[k];
+    if constexpr (REST >= 0) {
+      const acc cv = (acc)g.cv(i, j, k);
+      acc dv2;
+      if constexpr (REST == 3) {
+        const acc tx = dvx / dxb, ty = dvy / dyb, tz = dvz / dzb;
+        const acc two = AX == 0 ? ty + tz : (AX == 1 ? tx + tz : tx + ty);
+        cv1[c] = cv * ((acc)1.0 + (two + (AX == 0 ? tx : (AX == 1 ? ty : tz))) * tdt);
+        dv2 = two * tdt;
+      } else {
+        dv2 = (REST == 0 ? dvx / dxb : (REST == 1 ? dvy / dyb : dvz / dzb)) * tdt;
+      }
+      cv2[c] = cv * ((acc)1.0 + dv2);
+    }
+    db1[c] = AX == 0 ? dxb + dvx * tdt : (AX == 1 ? dyb + dvy * tdt : dzb + dvz * tdt);
+    lx = hx;
+    ly = hy;
+    lz = hz;
   }
 }
 
@@ -605,7 +652,9 @@ __device__ __forceinline__ void store_dm(real *__restrict__ dm, int c, int MS, i
 // from its own window at n and uses it at 0.  The new density goes to rho_new and the new energy to
 // e_new, since neighbouring chunks still read the old energy; only cells
 // 1..n are written (the halo refresh after the sweep fills the rest).
-template <int M>
+//
+// LASTSW: the remap's last sweep, whose cv2 is cv (k_geom).
+template <int M, bool LASTSW>
 __global__ __launch_bounds__(BX * BY) void k_mass_rho_energy_m(Geo g, Box b, const real *__restrict__ energy,
                                                                const real *__restrict__ rho1,
                                                                const real *__restrict__ vel,
@@ -678,9 +727,10 @@ __global__ __launch_bounds__(BX * BY) void k_mass_rho_energy_m(Geo g, Box b, con
     const real F = (fu + Di * ((acc)1.0 - dmu)) * dd;
     if (m >= m0 && m >= 1) {
       const acc rr = r[1];
-      const acc rn = (rr * cv1[c] + dp - dmc) / cv2[c];
+      const acc c2 = LASTSW ? (acc)(real)(acc)g.cv(i, j, k) : (acc)cv2[c];
+      const acc rn = (rr * cv1[c] + dp - dmc) / c2;
       rho_new[c] = rn;
-      e_new[c] = (e[1] * cv1[c] * rr + Fp - F) / (cv2[c] * rn);
+      e_new[c] = (e[1] * cv1[c] * rr + Fp - F) / (c2 * rn);
     }
     Fp = F;
     dp = dmc;
@@ -705,6 +755,7 @@ __device__ __forceinline__ acc mass_flux_x(const Geo &g, const real *__restrict_
           dc1<0>(g, db1, c + 1, i + 1), db1[c], db1[c + 1], dt, vad_p, vad_m, dbu, fu, Di, phi);
   return (fu + Di * ((acc)1.0 - phi)) * v_advect * dt * area;
 }
+template <bool LASTSW>
 __global__ __launch_bounds__(BX * BY) void k_mass_rho_energy_x(Geo g, Box b, const real *__restrict__ energy,
                                                                const real *__restrict__ rho1,
                                                                const real *__restrict__ vel,
@@ -751,9 +802,10 @@ __global__ __launch_bounds__(BX * BY) void k_mass_rho_energy_x(Geo g, Box b, con
   const real dmm = __shfl_up(dmc, 1, 64);
   if (!valid || lane < 1 || !inner || i < 1) return;
   const acc r1 = rho1[c];
-  const acc rn = (r1 * cv1[c] + dmm - dmc) / cv2[c];
+  const acc c2 = LASTSW ? (acc)(real)(acc)g.cv(i, j, k) : (acc)cv2[c];
+  const acc rn = (r1 * cv1[c] + dmm - dmc) / c2;
   rho_new[c] = rn;
-  e_new[c] = (energy[c] * cv1[c] * r1 + Fm - F) / (cv2[c] * rn);
+  e_new[c] = (energy[c] * cv1[c] * r1 + Fm - F) / (c2 * rn);
 }
 
 
@@ -784,18 +836,37 @@ template <int N>
 struct VCellN {
   real r[N], a[N], b[N], d[N];
 };
-template <int N>
-__device__ __forceinline__ VCellN<N> vcells_at(const real *__restrict__ rho1, const real *__restrict__ cv1,
-                                               const real *__restrict__ cv2, const real *__restrict__ dm, int c,
-                                               int D) {
+// The cell arrays, and the widths around a column of nodes marching along M
+// for the last sweep, whose cv2 is cv = dxb dyb dzb: dxb at i, i+1, the other
+// transverse width at p, p+1, and the widths along the march.
+struct VSrc {
+  const real *rho1, *cv1, *cv2, *dm;
+  double wx[2], wp[2];
+  const double *wm;
+};
+template <int M>
+__device__ __forceinline__ VSrc vsrc(const Geo &g, const real *rho1, const real *cv1, const real *cv2, const real *dm,
+                                     int i, int p) {
+  const double *dp = M == 2 ? g.dyb : g.dzb;
+  return VSrc{rho1, cv1, cv2, dm, {g.dxb[i], g.dxb[i + 1]}, {dp[p], dp[p + 1]}, M == 2 ? g.dzb : g.dyb};
+}
+// cells with march coordinate m; the pair (N = 2) is at transverse p + P0
+template <int M, bool LASTSW, int N, int P0 = 0>
+__device__ __forceinline__ VCellN<N> vcells_at(const VSrc &s, int c, int D, int m) {
   VCellN<N> v;
+  const double w = LASTSW ? s.wm[m] : 0.0;
 #pragma unroll
   for (int t = 0; t < N; ++t) {
     const int o = c + (t & 1) + (t >> 1) * D;
-    v.r[t] = rho1[o];
-    v.a[t] = cv1[o];
-    v.b[t] = cv2[o];
-    v.d[t] = dm[o];
+    v.r[t] = s.rho1[o];
+    v.a[t] = s.cv1[o];
+    if (LASTSW) {
+      const double x = s.wx[t & 1], p = s.wp[P0 + (t >> 1)];
+      v.b[t] = (real)(acc)(M == 2 ? x * p * w : x * w * p);
+    } else {
+      v.b[t] = s.cv2[o];
+    }
+    v.d[t] = s.dm[o];
   }
   return v;
 }
@@ -846,17 +917,15 @@ struct VMarch {
   VSum head;
   VCellN<M == 1 ? 2 : 1> tail;  // unused for M = 2
 };
-// Vertex quantities of the node at c.  With have set, m holds what the node
-// one step below c along M passed on; on return it holds what this node
-// passes on.
-template <int M>
-__device__ __forceinline__ VertexV vertex_march(const Geo &g, const real *__restrict__ rho1,
-                                                const real *__restrict__ cv1, const real *__restrict__ cv2,
-                                                const real *__restrict__ dm, int c, VMarch<M> &m, bool have) {
+// Vertex quantities of the node at c, march coordinate mm.  With have set, m
+// holds what the node one step below c along M passed on; on return it holds
+// what this node passes on.
+template <int M, bool LASTSW>
+__device__ __forceinline__ VertexV vertex_march(const Geo &g, const VSrc &s, int c, int mm, VMarch<M> &m, bool have) {
   const int Y = g.sy, Z = g.sz;
   if constexpr (M == 2) {
-    const VSum lo = have ? m.head : vsum_first(vcells_at<4>(rho1, cv1, cv2, dm, c, Y));
-    const VCellN<4> hi = vcells_at<4>(rho1, cv1, cv2, dm, c + Z, Y);
+    const VSum lo = have ? m.head : vsum_first(vcells_at<M, LASTSW, 4>(s, c, Y, mm));
+    const VCellN<4> hi = vcells_at<M, LASTSW, 4>(s, c + Z, Y, mm + 1);
     m.head = vsum_first(hi);
     return vertex_of(vsum_add(lo, hi));
   } else {
@@ -866,11 +935,11 @@ __device__ __forceinline__ VertexV vertex_march(const Geo &g, const real *__rest
       p = m.head;
       c45 = m.tail;
     } else {
-      p = vsum_first(vcells_at<2>(rho1, cv1, cv2, dm, c, Y));
-      c45 = vcells_at<2>(rho1, cv1, cv2, dm, c + Z, Y);
+      p = vsum_first(vcells_at<M, LASTSW, 2>(s, c, Y, mm));
+      c45 = vcells_at<M, LASTSW, 2, 1>(s, c + Z, Y, mm);
     }
-    const VCellN<2> c23 = vcells_at<2>(rho1, cv1, cv2, dm, c + Y, Y);
-    const VCellN<2> c67 = vcells_at<2>(rho1, cv1, cv2, dm, c + Y + Z, Y);
+    const VCellN<2> c23 = vcells_at<M, LASTSW, 2>(s, c + Y, Y, mm + 1);
+    const VCellN<2> c67 = vcells_at<M, LASTSW, 2, 1>(s, c + Y + Z, Y, mm + 1);
     p = vsum_add(p, c23);
     p = vsum_add(p, c45);
     p = vsum_add(p, c67);
@@ -915,7 +984,7 @@ __device__ __forceinline__ acc rke_edge(acc vs, acc vp, acc flm, acc fl, acc flp
 }
 #define MOMX_OUT 62
 #define MOMX_OUT_RKE 61
-template <bool RKE>
+template <bool RKE, bool LASTSW>
 __global__ __launch_bounds__(BX * BY) void k_mom_remap_x(Geo g, Box b, const real *__restrict__ vx,
                                                          const real *__restrict__ vy, const real *__restrict__ vz,
                                                          const real *__restrict__ vel1,
@@ -943,6 +1012,7 @@ __global__ __launch_bounds__(BX * BY) void k_mom_remap_x(Geo g, Box b, const rea
   const bool writer = valid && lane >= 1 && lane <= OUT;
   // vertex box: x -1..n+1, transverse 0..n
   const bool vin = j >= 0 && j <= g.ny && i >= -1 && i <= n + 1;
+  const VSrc vs = vsrc<2>(g, rho1, cv1, cv2, dm, i <= n + 1 ? i : n + 1, j <= g.ny + 1 ? j : g.ny + 1);
   VMarch<2> w;
   bool have = false;  // w holds what node k-1 passed on
   for (int k = k0; k <= k1; ++k) {
@@ -950,7 +1020,7 @@ __global__ __launch_bounds__(BX * BY) void k_mom_remap_x(Geo g, Box b, const rea
     const bool iny = j >= 0 && j <= g.ny && k >= 0 && k <= g.nz;
     VertexV vq = {0, 0, 0, 0};
     if (vin && k >= 0 && k <= g.nz) {
-      vq = vertex_march<2>(g, rho1, cv1, cv2, dm, c, w, have);
+      vq = vertex_march<2, LASTSW>(g, vs, c, k, w, have);
       have = true;
     }
     const real rvp = __shfl_down(vq.rv, 1, 64);  // rho_v of node i+1 (lanes 0..62)
@@ -1037,7 +1107,7 @@ __global__ __launch_bounds__(BX * BY) void k_mom_remap_x(Geo g, Box b, const rea
 // 0..n-1 along the sweep, transverse 0..n), formed one point behind the
 // march: the term of the edge at m-1 needs the flux velocity at m, so a
 // chunk runs one point past its last node when that node's edge exists.
-template <int M, bool RKE>
+template <int M, bool RKE, bool LASTSW>
 __global__ __launch_bounds__(BX * BY) void k_mom_remap_m(Geo g, Box b, const real *__restrict__ vx,
                                                          const real *__restrict__ vy, const real *__restrict__ vz,
                                                          const real *__restrict__ vel1,
@@ -1076,9 +1146,10 @@ __global__ __launch_bounds__(BX * BY) void k_mom_remap_m(Geo g, Box b, const rea
   for (int t = 0; t < 3; ++t) d[t] = db1[c + t * MS];
   v0 = vel1[c];
   v1 = vel1[c + MS];
+  const VSrc vs = vsrc<M>(g, rho1, cv1, cv2, dm, i, p);
   VMarch<M> w;
-  VertexV vc = vertex_march<M>(g, rho1, cv1, cv2, dm, c, w, false);
-  VertexV vn = vertex_march<M>(g, rho1, cv1, cv2, dm, c + MS, w, true);
+  VertexV vc = vertex_march<M, LASTSW>(g, vs, c, ms - 1, w, false);
+  VertexV vn = vertex_march<M, LASTSW>(g, vs, c + MS, ms, w, true);
   real Fp[3], dp = 0;
   // rke: flux velocities, dm and node mass carried from m-1 and m-2
   real FLp[3] = {0, 0, 0}, FLpp[3] = {0, 0, 0}, dpp = 0;
@@ -1100,7 +1171,7 @@ __global__ __launch_bounds__(BX * BY) void k_mom_remap_m(Geo g, Box b, const rea
       v0 = v1;
       v1 = vel1[c + 2 * MS];
       vc = vn;
-      vn = vertex_march<M>(g, rho1, cv1, cv2, dm, c + 2 * MS, w, true);
+      vn = vertex_march<M, LASTSW>(g, vs, c + 2 * MS, m + 1, w, true);
       c += MS;
     }
     const int j = MJ(M, m, p), k = MK(M, m, p);

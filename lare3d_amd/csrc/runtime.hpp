@@ -441,7 +441,7 @@ int strides(int ax) { return ax == 0 ? 1 : (ax == 1 ? S.sy : S.sz); }
 // remap.f90:44-67 folded in).  sc = -1 (last predictor sweep): out gets B
 // back (remap.f90:102-125 folded in).
 template <int AX>
-int ct_sweep(const double *const in[3], double *const out[3], const real *vel, double dt, int sc) {
+int ct_sweep(const double *const in[3], double *const out[3], const real *vel, const real *db1, double dt, int sc) {
   const int N[3] = {nx(), ny(), nz()};
   const Box ub = mkbox(0, N[0] + 1, 0, N[1] + 1, 0, N[2] + 1);
   // (transverse field t, velocity-average axis, geometry-average axis, box_t, box_a) x 2
@@ -469,13 +469,13 @@ int ct_sweep(const double *const in[3], double *const out[3], const real *vel, d
     const dim3 grid((unsigned)(ntx * nty), 1, (unsigned)((N[2] + 4 + mc) / mc));
     if (sc > 0)
       LAUNCH("ct_sweep", k_ct_sweep_x<1>, grid, blk, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX], vel,
-             S.db1, strides(ga1), strides(va2), dt, ntx, mc, bt1, ba1, bt2, ba2);
+             db1, strides(ga1), strides(va2), dt, ntx, mc, bt1, ba1, bt2, ba2);
     else if (sc < 0)
       LAUNCH("ct_sweep", k_ct_sweep_x<-1>, grid, blk, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX], vel,
-             S.db1, strides(ga1), strides(va2), dt, ntx, mc, bt1, ba1, bt2, ba2);
+             db1, strides(ga1), strides(va2), dt, ntx, mc, bt1, ba1, bt2, ba2);
     else
       LAUNCH("ct_sweep", k_ct_sweep_x<0>, grid, blk, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX], vel,
-             S.db1, strides(ga1), strides(va2), dt, ntx, mc, bt1, ba1, bt2, ba2);
+             db1, strides(ga1), strides(va2), dt, ntx, mc, bt1, ba1, bt2, ba2);
   } else {
     // y and z sweeps march along the sweep axis; tiles of CTM_XW - 1 points
     // in x by CTM_ROWS - 1 rows along the other transverse axis
@@ -486,13 +486,13 @@ int ct_sweep(const double *const in[3], double *const out[3], const real *vel, d
     const dim3 blkm(CTM_THREADS, 1, 1);
     if (sc > 0)
       LAUNCH("ct_sweep", (k_ct_sweep_m<AX, 1>), grid, blkm, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX],
-             vel, S.db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, mc, bt1, ba1, bt2, ba2);
+             vel, db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, mc, bt1, ba1, bt2, ba2);
     else if (sc < 0)
       LAUNCH("ct_sweep", (k_ct_sweep_m<AX, -1>), grid, blkm, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX],
-             vel, S.db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, mc, bt1, ba1, bt2, ba2);
+             vel, db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, mc, bt1, ba1, bt2, ba2);
     else
       LAUNCH("ct_sweep", (k_ct_sweep_m<AX, 0>), grid, blkm, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX],
-             vel, S.db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, mc, bt1, ba1, bt2, ba2);
+             vel, db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, mc, bt1, ba1, bt2, ba2);
   }
   return 0;
 }
@@ -506,49 +506,80 @@ void swap_spare(double *&ax, double *&ay, double *&az) {
   t = az; az = S.fzr; S.fzr = t;
 }
 
+// the widths d?b1 of the predictor sweeps live in db1 and, since a predictor
+// remap stores no volumes, in cv1 and cv2
+real *pred_db1(int ax) { return ax == 0 ? S.db1 : (ax == 1 ? S.cv1 : S.cv2); }
+
+// the geometry of a predictor remap whose last sweep is along `last`, and the
+// predictor pressure
+int geom_predictor(int last, double dt) {
+  const PredP pr = {S.energy, S.rho, S.visc_heat, S.p0, S.pp, S.p.gamma, S.dt2, eos_args()};
+  const Box cb = marched(cell_box());
+#define GEOM_PRED(L)                                                                                                 \
+  LAUNCH("geom", k_geom_pred<L>, zchunk_grid(cb), box_block(), S.g, cb, S.vx, S.vy, S.vz, pred_db1(0), pred_db1(1), \
+         pred_db1(2), dt, pr)
+  if (last == 0) GEOM_PRED(0);
+  else if (last == 1) GEOM_PRED(1);
+  else GEOM_PRED(2);
+#undef GEOM_PRED
+  return 0;
+}
+
 // one predictor-mode sweep (B only, no flag reset, no halo refresh) of the
 // copy bp of B; the first sweep reads B itself, the last converts back
 template <int AX>
 int sweep_predictor(double dt, bool first, bool last) {
-  // the last pass also forms the predictor energy and pressure
-  const PredP pr = {S.energy, S.rho, S.visc_heat, S.p0, S.pp, S.p.gamma, S.dt2, eos_args()};
-  const Box cb = marched(cell_box());
-  if (last)
-    LAUNCH("geom", (k_geom<AX, 1>), zchunk_grid(cb), box_block(), S.g, cb, S.vx, S.vy, S.vz, S.cv1,
-           S.cv2, S.db1, dt, 1.0, 1.0, 1.0, pr);
-  else
-    LAUNCH("geom", (k_geom<AX, 0>), zchunk_grid(cb), box_block(), S.g, cb, S.vx, S.vy, S.vz, S.cv1,
-           S.cv2, S.db1, dt, 1.0, 1.0, 1.0, pr);
   const real *vel = AX == 0 ? S.vx : (AX == 1 ? S.vy : S.vz);
   if (first) {
     // B itself stays untouched: the first sweep writes the copy
     const double *const Bin[3] = {S.bx, S.by, S.bz};
     double *const Bp[3] = {S.bpx, S.bpy, S.bpz};
-    return ct_sweep<AX>(Bin, Bp, vel, dt, 1);
+    return ct_sweep<AX>(Bin, Bp, vel, pred_db1(AX), dt, 1);
   }
   const double *const Bp[3] = {S.bpx, S.bpy, S.bpz};
   double *const spare[3] = {S.fxr, S.fyr, S.fzr};
-  int rc = ct_sweep<AX>(Bp, spare, vel, dt, last ? -1 : 0);
+  int rc = ct_sweep<AX>(Bp, spare, vel, pred_db1(AX), dt, last ? -1 : 0);
   if (rc) return rc;
   swap_spare(S.bpx, S.bpy, S.bpz);
   return 0;
 }
 
+// the geometry of a full sweep along AX; rest is the axis still to be swept
+// after it, 3 for the first sweep (two are) and -1 for the last.  From the
+// second sweep on, cv1 is the cv2 of the sweep before.
 template <int AX>
-int sweep_full(double dt, double pass[3], bool first, bool last) {
+int geom_full(int rest, double dt) {
+  const Box cb = marched(cell_box());
+#define GEOM(R)                                                                                                      \
+  LAUNCH("geom", (k_geom<AX, R>), zchunk_grid(cb), box_block(), S.g, cb, S.vx1, S.vy1, S.vz1, S.cv1, S.cv2, S.db1, dt)
+  if (rest == 3) {
+    GEOM(3);
+    return 0;
+  }
+  real *t = S.cv1;
+  S.cv1 = S.cv2;
+  S.cv2 = t;
+  if (rest < 0) GEOM(-1);
+  else if (rest == (AX + 1) % 3) GEOM((AX + 1) % 3);
+  else GEOM((AX + 2) % 3);
+#undef GEOM
+  return 0;
+}
+
+// one full sweep; first, last: its place in the remap, rest: see geom_full
+template <int AX>
+int sweep_full(double dt, bool first, bool last, int rest) {
   const int N[3] = {nx(), ny(), nz()};
   const real *vel = AX == 0 ? S.vx1 : (AX == 1 ? S.vy1 : S.vz1);
-  const Box cb = marched(cell_box());
-  LAUNCH("geom", (k_geom<AX, 2>), zchunk_grid(cb), box_block(), S.g, cb, S.vx1, S.vy1, S.vz1, S.cv1,
-         S.cv2, S.db1, dt, pass[0], pass[1], pass[2], PredP{});
+  int rc = geom_full<AX>(rest, dt);
+  if (rc) return rc;
   {
     const double *const B[3] = {S.bx, S.by, S.bz};
     double *const spare[3] = {S.fxr, S.fyr, S.fzr};
-    int rc = ct_sweep<AX>(B, spare, vel, dt, first ? 1 : (last ? -1 : 0));
+    rc = ct_sweep<AX>(B, spare, vel, S.db1, dt, first ? 1 : (last ? -1 : 0));
     if (rc) return rc;
     swap_spare(S.bx, S.by, S.bz);
   }
-  int rc = 0;
   int hi[3] = {N[0] + 1, N[1] + 1, N[2] + 1};
   hi[AX] = N[AX];
   Box mb = mkbox(0, hi[0], 0, hi[1], 0, hi[2]);
@@ -560,11 +591,19 @@ int sweep_full(double dt, double pass[3], bool first, bool last) {
   if constexpr (AX == 0) {
     const dim3 gx(wave_blocks((long)(mb.x1 - mb.x0 + 1) * (mb.y1 - mb.y0 + 1), REX_OUT), 1,
                   (unsigned)(mb.z1 - mb.z0 + 1));
-    LAUNCH("rho_energy", k_mass_rho_energy_x, gx, box_block(), S.g, mb, S.energy, S.rho, vel, S.db1, S.dm, S.cv1,
-           S.cv2, S.rho_alt, S.Fe, dt, S.per[AX] ? 1 : 0);
+#define RHO_ENERGY(L)                                                                                               \
+  LAUNCH("rho_energy", k_mass_rho_energy_x<L>, gx, box_block(), S.g, mb, S.energy, S.rho, vel, S.db1, S.dm, S.cv1, \
+         S.cv2, S.rho_alt, S.Fe, dt, S.per[AX] ? 1 : 0)
+    if (last) RHO_ENERGY(true);
+    else RHO_ENERGY(false);
+#undef RHO_ENERGY
   } else {
-    LAUNCH("rho_energy", k_mass_rho_energy_m<AX>, zchunk_grid(march_box(mb, AX)), box_block(), S.g, mb, S.energy,
-           S.rho, vel, S.db1, S.dm, S.cv1, S.cv2, S.rho_alt, S.Fe, dt, S.per[AX] ? 1 : 0);
+#define RHO_ENERGY(L)                                                                                               \
+  LAUNCH("rho_energy", (k_mass_rho_energy_m<AX, L>), zchunk_grid(march_box(mb, AX)), box_block(), S.g, mb, S.energy, \
+         S.rho, vel, S.db1, S.dm, S.cv1, S.cv2, S.rho_alt, S.Fe, dt, S.per[AX] ? 1 : 0)
+    if (last) RHO_ENERGY(true);
+    else RHO_ENERGY(false);
+#undef RHO_ENERGY
   }
   if (S.any_open) {
     // the new energy and density cover cells 1..n; the ghosts of a BC_OPEN
@@ -588,20 +627,24 @@ int sweep_full(double dt, double pass[3], bool first, bool last) {
                                       S.delta_ke ? MOMX_OUT_RKE : MOMX_OUT);
       xb.zc = march_chunk(pb, xb.z1 - xb.z0 + 1);
       const dim3 gx(pb, 1, (unsigned)((xb.z1 - xb.z0 + xb.zc) / xb.zc));
-      if (S.delta_ke)
-        LAUNCH("mom_remap", k_mom_remap_x<true>, gx, box_block(), S.g, xb, S.vx, S.vy, S.vz, vel, S.db1, S.rho,
-               S.cv1, S.cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk);
-      else
-        LAUNCH("mom_remap", k_mom_remap_x<false>, gx, box_block(), S.g, xb, S.vx, S.vy, S.vz, vel, S.db1, S.rho,
-               S.cv1, S.cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk);
+#define MOM_REMAP(R, L)                                                                                          \
+  LAUNCH("mom_remap", (k_mom_remap_x<R, L>), gx, box_block(), S.g, xb, S.vx, S.vy, S.vz, vel, S.db1, S.rho, S.cv1, \
+         S.cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk)
+      if (S.delta_ke && last) MOM_REMAP(true, true);
+      else if (S.delta_ke) MOM_REMAP(true, false);
+      else if (last) MOM_REMAP(false, true);
+      else MOM_REMAP(false, false);
+#undef MOM_REMAP
     } else {
       xb = marched(xb, AX);
-      if (S.delta_ke)
-        LAUNCH("mom_remap", (k_mom_remap_m<AX, true>), zchunk_grid(march_box(xb, AX)), box_block(), S.g, xb, S.vx,
-               S.vy, S.vz, vel, S.db1, S.rho, S.cv1, S.cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk);
-      else
-        LAUNCH("mom_remap", (k_mom_remap_m<AX, false>), zchunk_grid(march_box(xb, AX)), box_block(), S.g, xb, S.vx,
-               S.vy, S.vz, vel, S.db1, S.rho, S.cv1, S.cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk);
+#define MOM_REMAP(R, L)                                                                                               \
+  LAUNCH("mom_remap", (k_mom_remap_m<AX, R, L>), zchunk_grid(march_box(xb, AX)), box_block(), S.g, xb, S.vx, S.vy,  \
+         S.vz, vel, S.db1, S.rho, S.cv1, S.cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk)
+      if (S.delta_ke && last) MOM_REMAP(true, true);
+      else if (S.delta_ke) MOM_REMAP(true, false);
+      else if (last) MOM_REMAP(false, true);
+      else MOM_REMAP(false, false);
+#undef MOM_REMAP
     }
     // rke: this sweep's edge terms into delta_ke
     if (S.delta_ke) LAUNCH_BOX("rke_gather", k_rke_gather<AX>, interior(), S.rk, S.delta_ke);
@@ -613,10 +656,7 @@ int sweep_full(double dt, double pass[3], bool first, bool last) {
   real *t = S.rho;
   S.rho = S.rho_alt;
   S.rho_alt = t;
-  rc = boundary_conditions();
-  if (rc) return rc;
-  pass[AX] = 0.0;
-  return 0;
+  return boundary_conditions();
 }
 
 const int kStrang[6][3] = {{0, 1, 2}, {1, 2, 0}, {2, 0, 1}, {0, 2, 1}, {2, 1, 0}, {1, 0, 2}};
@@ -631,10 +671,12 @@ int eulerian_remap(int step, bool predictor) {
   // bfield_bcs after the scaling back in the reference writes from the same
   // interior.
   if (predictor) {
+    int rc = geom_predictor(kStrang[c][2], dt);
+    if (rc) return rc;
     for (int q = 0; q < 3; ++q) {
       const int ax = kStrang[c][q];
       const bool first = q == 0, last = q == 2;
-      int rc = ax == 0 ? sweep_predictor<0>(dt, first, last)
+      rc = ax == 0 ? sweep_predictor<0>(dt, first, last)
                        : (ax == 1 ? sweep_predictor<1>(dt, first, last) : sweep_predictor<2>(dt, first, last));
       if (rc) return rc;
     }
@@ -642,12 +684,12 @@ int eulerian_remap(int step, bool predictor) {
   }
   // rke: delta_ke = 0 (remap.f90:38); only the interior is ever read
   if (S.delta_ke) LAUNCH_BOX("fill", k_fill, interior(), S.delta_ke, 0.0);
-  double pass[3] = {1.0, 1.0, 1.0};
   for (int q = 0; q < 3; ++q) {
     const int ax = kStrang[c][q];
     const bool first = q == 0, last = q == 2;
-    int rc = ax == 0 ? sweep_full<0>(dt, pass, first, last)
-                     : (ax == 1 ? sweep_full<1>(dt, pass, first, last) : sweep_full<2>(dt, pass, first, last));
+    const int rest = first ? 3 : (last ? -1 : kStrang[c][2]);
+    int rc = ax == 0 ? sweep_full<0>(dt, first, last, rest)
+                     : (ax == 1 ? sweep_full<1>(dt, first, last, rest) : sweep_full<2>(dt, first, last, rest));
     if (rc) return rc;
   }
   return 0;

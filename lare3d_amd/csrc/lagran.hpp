@@ -1079,7 +1079,10 @@ __global__ __launch_bounds__(BX * BY) void k_force(Geo g, Box b, const real *__r
 }
 
 // shock_heating (lagran.F90:861-937) + corrector (:415-462) over cells
-// 1..n; total_visc_heating partial sums.  COOL: cooling_term on.
+// 1..n and v = 2 v1 - v (:399-407) at the nodes 0..n, which is the launch box
+// (a cell goes with its upper corner's node); total_visc_heating partial
+// sums.  COOL: cooling_term on.  The nodes with an index 0 had a launch of
+// their own, 27 us at 256^3 and 4 us on small grids.
 template <bool COOL>
 __global__ __launch_bounds__(BX * BY) void k_shock_corr(Geo g, Box b, const real *__restrict__ vx, const real *__restrict__ vy,
                              const real *__restrict__ vz, const real *__restrict__ vx1,
@@ -1091,15 +1094,15 @@ __global__ __launch_bounds__(BX * BY) void k_shock_corr(Geo g, Box b, const real
                              real *__restrict__ cool_v, double alpha_av, double *__restrict__ partial, double dt) {
   // cool_v: cool_term_v of the cooling_term (lagran.F90:464-476), unused
   // without COOL
-  // cells 1..n, marching in z: the node values (v, v1) and al1/al2 of plane
-  // k are reused as plane k-1 / k values of the next cell.  The new
-  // velocity v = 2 v1 - v of node (i, j, k), the cell's upper corner, goes
-  // to vxo..vzo, since neighbouring cells still read the old v.
+  // marching in z: the node values (v, v1) and al1/al2 of plane k are reused
+  // as plane k-1 / k values of the next cell.  The new velocity goes to
+  // vxo..vzo, since neighbouring cells still read the old v.
   PLANE_POS(b, i, j)
   ZRANGE(b, k0, k1)
   double v[1] = {0.0};
   if (j <= b.y1) {
     const int Y = g.sy, Z = g.sz;
+    const bool column = i >= 1 && j >= 1;
     const int cb = g.idx(i, j, k0) - Z;
     Node4 lx = node4(vx, cb, Y), ly = node4(vy, cb, Y), lz = node4(vz, cb, Y);
     Node4 lx1 = node4(vx1, cb, Y), ly1 = node4(vy1, cb, Y), lz1 = node4(vz1, cb, Y);
@@ -1109,46 +1112,47 @@ __global__ __launch_bounds__(BX * BY) void k_shock_corr(Geo g, Box b, const real
       const Node4 hx = node4(vx, c, Y), hy = node4(vy, c, Y), hz = node4(vz, c, Y);
       const Node4 hx1 = node4(vx1, c, Y), hy1 = node4(vy1, c, Y), hz1 = node4(vz1, c, Y);
       const Al12 ahi = al12(al1, al2, c + Z, Y);
-      acc aa[12];
-      // (v(first) - v(second)) . (v1(first) - v1(second)) per edge
+      if (column && k >= 1) {
+        acc aa[12];
+        // (v(first) - v(second)) . (v1(first) - v1(second)) per edge
 #define AAS(q, P1, N1, P2, N2)                                                            \
-  aa[q] = (P1##x.N1 - P2##x.N2) * (P1##x1.N1 - P2##x1.N2) + (P1##y.N1 - P2##y.N2) * (P1##y1.N1 - P2##y1.N2) + \
-          (P1##z.N1 - P2##z.N2) * (P1##z1.N1 - P2##z1.N2);
-      EDGES(AAS)
+    aa[q] = (P1##x.N1 - P2##x.N2) * (P1##x1.N1 - P2##x1.N2) + (P1##y.N1 - P2##y.N2) * (P1##y1.N1 - P2##y1.N2) + \
+            (P1##z.N1 - P2##z.N2) * (P1##z1.N1 - P2##z1.N2);
+        EDGES(AAS)
 #undef AAS
-      const acc a30 = al3[c], a3x = al3[c - 1], a3xy = al3[c - 1 - Y], a3y = al3[c - Y];
-      const acc vh = max0(edge_heat_v((acc)g.dxb[i], (acc)g.dyb[j], (acc)g.dzb[k], (acc)g.cv(i, j, k), alo, ahi, a30,
-                                      a3x, a3xy, a3y, aa));
-      // face-averaged v1 (quad sums in the order c, c-Y, c-Z, c-Y-Z etc.;
-      // node C = c, B = c-Y, D = c-X, A = c-X-Y)
-      const acc q4 = 0.25;
-      const acc vxb = (hx1.c + hx1.b + lx1.c + lx1.b) * q4;
-      const acc vxbm = (hx1.d + hx1.a + lx1.d + lx1.a) * q4;
-      const acc vyb = (hy1.c + hy1.d + ly1.c + ly1.d) * q4;
-      const acc vybm = (hy1.b + hy1.a + ly1.b + ly1.a) * q4;
-      const acc vzb = (hz1.c + hz1.d + hz1.b + hz1.a) * q4;
-      const acc vzbm = (lz1.c + lz1.d + lz1.b + lz1.a) * q4;
-      const acc dta = (acc)dt;
-      const acc dv =
-          ((vxb - vxbm) / (acc)g.dxb[i] + (vyb - vybm) / (acc)g.dyb[j] + (vzb - vzbm) / (acc)g.dzb[k]) * dta;
-      const acc r = rho[c];
-      const real e1 = energy[c] + (dta * vh - dv * pp[c]) / r;
-      visc_dep[c] = visc_dep[c] + dta * vh;
-      const real rn = r / ((acc)1.0 + dv);
-      rho[c] = rn;
-      if (COOL) {
-        // a running average of the viscous heating is removed again, and
-        // energy = MAX(energy, 0)
-        const acc aav = (acc)alpha_av;
-        const real ct = aav * dta * vh / rn + ((acc)1.0 - aav) * cool_v[c];
-        cool_v[c] = ct;
-        energy[c] = max0((acc)(e1 - ct));
-      } else {
-        energy[c] = e1;
+        const acc a30 = al3[c], a3x = al3[c - 1], a3xy = al3[c - 1 - Y], a3y = al3[c - Y];
+        const acc vh = max0(edge_heat_v((acc)g.dxb[i], (acc)g.dyb[j], (acc)g.dzb[k], (acc)g.cv(i, j, k), alo, ahi, a30,
+                                        a3x, a3xy, a3y, aa));
+        // face-averaged v1 (quad sums in the order c, c-Y, c-Z, c-Y-Z etc.;
+        // node C = c, B = c-Y, D = c-X, A = c-X-Y)
+        const acc q4 = 0.25;
+        const acc vxb = (hx1.c + hx1.b + lx1.c + lx1.b) * q4;
+        const acc vxbm = (hx1.d + hx1.a + lx1.d + lx1.a) * q4;
+        const acc vyb = (hy1.c + hy1.d + ly1.c + ly1.d) * q4;
+        const acc vybm = (hy1.b + hy1.a + ly1.b + ly1.a) * q4;
+        const acc vzb = (hz1.c + hz1.d + hz1.b + hz1.a) * q4;
+        const acc vzbm = (lz1.c + lz1.d + lz1.b + lz1.a) * q4;
+        const acc dta = (acc)dt;
+        const acc dv =
+            ((vxb - vxbm) / (acc)g.dxb[i] + (vyb - vybm) / (acc)g.dyb[j] + (vzb - vzbm) / (acc)g.dzb[k]) * dta;
+        const acc r = rho[c];
+        const real e1 = energy[c] + (dta * vh - dv * pp[c]) / r;
+        visc_dep[c] = visc_dep[c] + dta * vh;
+        const real rn = r / ((acc)1.0 + dv);
+        rho[c] = rn;
+        if (COOL) {
+          // a running average of the viscous heating is removed again, and
+          // energy = MAX(energy, 0)
+          const acc aav = (acc)alpha_av;
+          const real ct = aav * dta * vh / rn + ((acc)1.0 - aav) * cool_v[c];
+          cool_v[c] = ct;
+          energy[c] = max0((acc)(e1 - ct));
+        } else {
+          energy[c] = e1;
+        }
+        v[0] += dt * (double)vh * g.cv(i, j, k);
       }
-      v[0] += dt * (double)vh * g.cv(i, j, k);
-      // v = 2 v1 - v (:399-407) at node (i, j, k); k_vupdate_low does the
-      // nodes with an index 0
+      // v = 2 v1 - v (:399-407) at node (i, j, k)
       vxo[c] = (real)((acc)2.0 * hx1.c - hx.c);
       vyo[c] = (real)((acc)2.0 * hy1.c - hy.c);
       vzo[c] = (real)((acc)2.0 * hz1.c - hz.c);
@@ -1163,45 +1167,6 @@ __global__ __launch_bounds__(BX * BY) void k_shock_corr(Geo g, Box b, const real
   }
   const int ops[1] = {1};
   block_reduce_store<1>(v, ops, partial);
-}
-
-
-// v = 2 v1 - v (:399-407) into vxo..vzo at the nodes 0..n that have an
-// index 0 (k_shock_corr does the rest): the plane k = 0 and, above it, the
-// faces i = 0 and j = 0.  One thread per node of the (n+1)^2 plane, then
-// one per node of the two faces, flattened.
-__global__ __launch_bounds__(256) void k_vupdate_low(Geo g, const real *__restrict__ vx, const real *__restrict__ vy,
-                                                     const real *__restrict__ vz, const real *__restrict__ vx1,
-                                                     const real *__restrict__ vy1, const real *__restrict__ vz1,
-                                                     real *__restrict__ vxo, real *__restrict__ vyo,
-                                                     real *__restrict__ vzo) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long px = g.nx + 1, py = g.ny + 1;
-  const long plane = px * py;                 // k = 0
-  const long face = (long)g.nz * (px + py - 1);  // k = 1..n: i = 0 or j = 0
-  if (t >= plane + face) return;
-  int i, j, k;
-  if (t < plane) {
-    k = 0;
-    j = (int)(t / px);
-    i = (int)(t - (long)j * px);
-  } else {
-    const long u = t - plane;
-    const long row = px + py - 1;  // (0, j) for j = 0..ny, then (i, 0) for i = 1..nx
-    k = 1 + (int)(u / row);
-    const int r = (int)(u - (long)(k - 1) * row);
-    if (r < py) {
-      i = 0;
-      j = r;
-    } else {
-      i = r - (int)py + 1;
-      j = 0;
-    }
-  }
-  const int c = g.idx(i, j, k);
-  vxo[c] = (real)(2.0 * vx1[c] - vx[c]);
-  vyo[c] = (real)(2.0 * vy1[c] - vy[c]);
-  vzo[c] = (real)(2.0 * vz1[c] - vz[c]);
 }
 
 // Element offsets of the fields energy_account reads, per staggering.

@@ -93,11 +93,14 @@ int api_energy_account_noalloc(const lare_grid *grid, const lare_fields *f, doub
   HIPCHK(hipGetLastError());
   // the fold of fp64::final_reduce, on the scratch array
   const int nbi = (int)nb, nv = 4, minmask = 8;
-  const int chunk = (nbi + RED_ROWS - 1) / RED_ROWS;
-  const int rows = (nbi + chunk - 1) / chunk;
-  hipLaunchKernelGGL(fp64::k_reduce_rows, dim3(rows), dim3(256), 0, 0, partial, nbi, nv, minmask, chunk, level1);
-  HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL(fp64::k_final_reduce, dim3(1), dim3(256), 0, 0, level1, rows, nv, minmask, 0, out);
+  int rows;
+  const int chunk = fp64::fold_chunk(nbi, &rows);
+  if (chunk) {
+    hipLaunchKernelGGL(fp64::k_reduce_rows, dim3(rows), dim3(256), 0, 0, partial, nbi, nv, minmask, chunk, level1);
+    HIPCHK(hipGetLastError());
+  }
+  hipLaunchKernelGGL(fp64::k_final_reduce, dim3(1), dim3(256), 0, 0, chunk ? level1 : partial, rows, nv, minmask, 0, out,
+                     (double *)nullptr);
   HIPCHK(hipGetLastError());
   double v[4];
   HIPCHK(hipMemcpy(v, out, sizeof(v), hipMemcpyDeviceToHost));

@@ -198,15 +198,20 @@ dim3 zchunk_grid(const Box &b) { return dim3(plane_blocks(b), 1, (unsigned)((b.z
 // reduction over partials of a grid launched from index 0 on every axis
 dim3 grid_from0(int x1, int y1, int z1) { return box_grid(mkbox(0, x1, 0, y1, 0, z1)); }
 
-// Two-level reduction of the per-block partials (rows of nv values; bit q of
-// minmask selects min, else sum).  Level 1: RED_ROWS blocks each fold one
-// contiguous chunk of rows; level 2: one block folds the RED_ROWS results and
-// stores (or adds) the nv scalars.
+// Reduction of the per-block partials (rows of nv values; bit q of minmask
+// selects min, else sum).  Up to RED_DIRECT rows one block folds them all (at
+// most four per thread); beyond, RED_ROWS blocks each fold one contiguous
+// chunk of rows and one block folds the RED_ROWS results.  The last block
+// stores (or adds) the nv scalars, in device memory and in the pinned host
+// mirror, so that reading them takes a synchronisation and no copy: a
+// reduction read by the host was three launches (the copy is one), 12 to 14
+// us at any size, and is one or two.
 #define RED_ROWS 512
+#define RED_DIRECT 1024
 #define RED_MAXV 4
 
 __device__ __forceinline__ void fold_rows(const double *__restrict__ rows, int r0, int r1, int nv, int minmask,
-                                          double *__restrict__ out, int accumulate) {
+                                          double *__restrict__ out, int accumulate, double *__restrict__ host = nullptr) {
   __shared__ double red[4][RED_MAXV];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int q = 0; q < nv; ++q) {
@@ -227,6 +232,7 @@ __device__ __forceinline__ void fold_rows(const double *__restrict__ rows, int r
     for (int w = 1; w < 4; ++w) r = isMin ? dmin(r, red[w][q]) : r + red[w][q];
     if (accumulate) r = out[q] + r;
     out[q] = r;
+    if (host) host[q] = r;
   }
 }
 
@@ -238,26 +244,40 @@ __global__ __launch_bounds__(256) void k_reduce_rows(const double *__restrict__ 
 }
 
 __global__ __launch_bounds__(256) void k_final_reduce(const double *__restrict__ level1, int nrows, int nv, int minmask,
-                                                      int accumulate, double *__restrict__ out) {
-  fold_rows(level1, 0, nrows, nv, minmask, out, accumulate);
+                                                      int accumulate, double *__restrict__ out,
+                                                      double *__restrict__ host) {
+  fold_rows(level1, 0, nrows, nv, minmask, out, accumulate, host);
+}
+
+// Rows per level-1 block of a fold of nb rows and the number of level-1
+// results; 0 (and nb rows) when one block folds the rows directly.
+int fold_chunk(int nb, int *rows) {
+  *rows = nb;
+  if (nb <= RED_DIRECT) return 0;
+  const int chunk = (nb + RED_ROWS - 1) / RED_ROWS;
+  *rows = (nb + chunk - 1) / chunk;  // every level-1 block has >= 1 row
+  return chunk;
 }
 
 int final_reduce(dim3 grid, int nv, int minmask, int slot, int accumulate) {
   const int nb = (int)(grid.x * grid.y * grid.z);
   if (nv > RED_MAXV || (size_t)nb * nv > S.partial_cap)
     return fail(LARE_E_ARG, "reduction of %d x %d values exceeds the partial buffer", nb, nv);
-  const int chunk = (nb + RED_ROWS - 1) / RED_ROWS;
-  const int rows = (nb + chunk - 1) / chunk;  // every level-1 block has >= 1 row
-  double *level1 = S.partial + S.partial_cap;
-  LAUNCH("reduce_rows", k_reduce_rows, dim3(rows), dim3(256), S.partial, nb, nv, minmask, chunk, level1);
-  LAUNCH("final_reduce", k_final_reduce, dim3(1), dim3(256), level1, rows, nv, minmask, accumulate, S.dscal + slot);
+  const double *rows = S.partial;
+  int nrows = nb;
+  if (const int chunk = fold_chunk(nb, &nrows)) {
+    double *level1 = S.partial + S.partial_cap;
+    LAUNCH("reduce_rows", k_reduce_rows, dim3(nrows), dim3(256), S.partial, nb, nv, minmask, chunk, level1);
+    rows = level1;
+  }
+  LAUNCH("final_reduce", k_final_reduce, dim3(1), dim3(256), rows, nrows, nv, minmask, accumulate, S.dscal + slot,
+         S.hscal + slot);
   return 0;
 }
 
 int read_scalars(int slot, int count, double *out) {
-  HIPCHK(hipMemcpyAsync(S.hscal, S.dscal + slot, sizeof(double) * count, hipMemcpyDeviceToHost, S.stream));
   HIPCHK(hipStreamSynchronize(S.stream));
-  for (int q = 0; q < count; ++q) out[q] = S.hscal[q];
+  for (int q = 0; q < count; ++q) out[q] = ((volatile double *)S.hscal)[slot + q];
   return 0;
 }
 
@@ -1016,7 +1036,7 @@ int lagrangian_step() {
   }
 
   // predictor-corrector (lagran.F90:208-478)
-  const Box nb = marched(nodes0n()), ib = marched(interior());
+  const Box nb = marched(nodes0n());
   if (S.p.cauchy) {
     // the Cauchy solution for the cell-centred B1 (B1 cv1 in the spare
     // predictor-B arrays), cv1 and the predictor pressure; no predictor remap
@@ -1052,22 +1072,17 @@ int lagrangian_step() {
     rc = open_save();
     if (rc) return rc;
   }
-  dim3 g3 = zchunk_grid(ib);
+  dim3 g3 = zchunk_grid(nb);
   if (S.cool_v)
-    LAUNCH("shock_corr", k_shock_corr<true>, g3, box_block(), S.g, ib, S.vx, S.vy, S.vz, S.vx1, S.vy1, S.vz1,
+    LAUNCH("shock_corr", k_shock_corr<true>, g3, box_block(), S.g, nb, S.vx, S.vy, S.vz, S.vx1, S.vy1, S.vz1,
            S.al1, S.al2, S.al3, S.pp, S.energy, S.rho, S.visc_dep, S.Fx, S.Fy, S.Fz, S.cool_v, S.p.alpha_av,
            S.partial, S.dt);
   else
-    LAUNCH("shock_corr", k_shock_corr<false>, g3, box_block(), S.g, ib, S.vx, S.vy, S.vz, S.vx1, S.vy1, S.vz1,
+    LAUNCH("shock_corr", k_shock_corr<false>, g3, box_block(), S.g, nb, S.vx, S.vy, S.vz, S.vx1, S.vy1, S.vz1,
            S.al1, S.al2, S.al3, S.pp, S.energy, S.rho, S.visc_dep, S.Fx, S.Fy, S.Fz, S.cool_v, S.p.alpha_av,
            S.partial, S.dt);
   rc = final_reduce(g3, 1, 0, 8, 1);
   if (rc) return rc;
-  {
-    const long nlow = (long)(nx() + 1) * (ny() + 1) + (long)nz() * (nx() + ny() + 1);
-    LAUNCH("vupdate_low", k_vupdate_low, dim3((unsigned)((nlow + 255) / 256)), dim3(256), S.g, S.vx, S.vy, S.vz,
-           S.vx1, S.vy1, S.vz1, S.Fx, S.Fy, S.Fz);
-  }
   // the new velocities went to the momentum-flux arrays, which swap roles
   // with the velocity arrays; the boundary fill below sets their ghosts
   if (S.any_open) {
@@ -1337,6 +1352,7 @@ int api_init(const lare_grid *grid, const lare_params *params) {
   HIPCHK(hipMalloc((void **)&S.dscal, sizeof(double) * 16));
   HIPCHK(hipMemset(S.dscal, 0, sizeof(double) * 16));
   HIPCHK(hipHostMalloc((void **)&S.hscal, sizeof(double) * 16));
+  memset(S.hscal, 0, sizeof(double) * 16);
   HIPCHK(hipStreamSynchronize(S.stream));
   S.dt = S.dt2 = S.dtr = S.time = 0.0;
   S.n_s_stages = S.peak_substeps = S.last_substeps = 0;
@@ -1397,6 +1413,8 @@ int api_set_scalars(const lare_scalars *in) {
   S.step = in->step;
   double acc[2] = {in->total_visc_heating, in->total_ohmic_heating};
   HIPCHK(hipMemcpy(S.dscal + 8, acc, sizeof(acc), hipMemcpyHostToDevice));
+  S.hscal[8] = acc[0];
+  S.hscal[9] = acc[1];
   return 0;
 }
 

@@ -1624,8 +1624,9 @@ struct Sur {
   bool standardised = false;
   // mini-batch work arrays (capacity bcap columns)
   int bcap = 0;
-  float *Xb = nullptr, *yb = nullptr, *Z1 = nullptr, *H1 = nullptr, *Z2 = nullptr, *H2 = nullptr, *yo = nullptr,
-        *dy = nullptr, *dZ2 = nullptr, *dH1 = nullptr, *dZ1 = nullptr, *lossacc = nullptr, *losshist = nullptr;
+  float *Xb = nullptr, *yb = nullptr, *H1 = nullptr, *H2 = nullptr, *yo = nullptr, *dy = nullptr, *dZ2 = nullptr,
+        *dZ1 = nullptr, *lossacc = nullptr, *losshist = nullptr;
+  int *row = nullptr;
   int losscap = 0;
   // use inside lagrangian_step
   int enabled = 0;
@@ -1642,8 +1643,8 @@ void sfree(T *&p) {
 }
 
 void sur_free_batch() {
-  sfree(SU.Xb); sfree(SU.yb); sfree(SU.Z1); sfree(SU.H1); sfree(SU.Z2); sfree(SU.H2); sfree(SU.yo);
-  sfree(SU.dy); sfree(SU.dZ2); sfree(SU.dH1); sfree(SU.dZ1); sfree(SU.lossacc);
+  sfree(SU.Xb); sfree(SU.yb); sfree(SU.row); sfree(SU.H1); sfree(SU.H2); sfree(SU.yo);
+  sfree(SU.dy); sfree(SU.dZ2); sfree(SU.dZ1); sfree(SU.lossacc);
   SU.bcap = 0;
 }
 
@@ -1700,14 +1701,12 @@ int sur_ensure_batch(int cols) {
   const size_t c = (size_t)cols;
   int rc = salloc(&SU.Xb, c * SUR_K);
   if (!rc) rc = salloc(&SU.yb, c);
-  if (!rc) rc = salloc(&SU.Z1, c * SUR_H);
+  if (!rc) rc = salloc(&SU.row, c);
   if (!rc) rc = salloc(&SU.H1, c * SUR_H);
-  if (!rc) rc = salloc(&SU.Z2, c * SUR_H);
   if (!rc) rc = salloc(&SU.H2, c * SUR_H);
   if (!rc) rc = salloc(&SU.yo, c);
   if (!rc) rc = salloc(&SU.dy, c);
   if (!rc) rc = salloc(&SU.dZ2, c * SUR_H);
-  if (!rc) rc = salloc(&SU.dH1, c * SUR_H);
   if (!rc) rc = salloc(&SU.dZ1, c * SUR_H);
   if (!rc) rc = salloc(&SU.lossacc, (c + 255) / 256);
   if (rc) return rc;
@@ -1717,47 +1716,15 @@ int sur_ensure_batch(int cols) {
 
 unsigned blocks_for(size_t n, unsigned bs = 256) { return (unsigned)((n + bs - 1) / bs); }
 
-int gemm(int M, int N, int K, const float *A, int sam, int sak, const float *B, int sbk, int sbn, float *C, int scm,
-         int scn) {
-  LAUNCH("sur_gemm", k_gemm_bf16, dim3((unsigned)(N / 16), (unsigned)(M / 16)), dim3(64), M, N, K, A, sam, sak, B, sbk,
-         sbn, C, scm, scn);
-  return 0;
+// Forward pass (and, with targets y, backward) over nb columns, a multiple of
+// 16, of which the first nreal are rows of X: rows drawn by hash of seed from
+// the first `draw`, or (draw = 0) rows 0 .. nreal-1.
+SurBatch sur_batch(const float *X, const float *y, int nb, int nreal) {
+  return SurBatch{X, y, SU.row, SU.H1, SU.H2, SU.dZ1, SU.dZ2, SU.yo, SU.dy, nb, nreal};
 }
-
-// Forward pass on SU.Xb (nb columns, a multiple of 16; the first nreal are
-// real rows).  With tgt: loss partials and dy as well.
-int sur_forward(int nb, int nreal, const float *tgt) {
-  int rc = gemm(SUR_H, nb, SUR_K, SU.w + SUR_OFF_W1, 1, SUR_H, SU.Xb, 1, SUR_K, SU.Z1, nb, 1);
-  if (rc) return rc;
-  LAUNCH("sur_bias_gelu", k_bias_gelu, dim3(blocks_for((size_t)SUR_H * nb)), dim3(256), SU.Z1, SU.H1,
-         SU.w + SUR_OFF_B1, SUR_H, nb);
-  rc = gemm(SUR_H, nb, SUR_H, SU.w + SUR_OFF_W2, 1, SUR_H, SU.H1, nb, 1, SU.Z2, nb, 1);
-  if (rc) return rc;
-  LAUNCH("sur_bias_gelu", k_bias_gelu, dim3(blocks_for((size_t)SUR_H * nb)), dim3(256), SU.Z2, SU.H2,
-         SU.w + SUR_OFF_B2, SUR_H, nb);
-  LAUNCH("sur_out", k_out_layer, dim3(blocks_for(nb)), dim3(256), SU.H2, SU.w, tgt, nb, nreal, SU.yo, SU.dy,
-         SU.lossacc);
+int sur_fb(const SurBatch &b, int draw, unsigned long long seed) {
+  LAUNCH("sur_fb", k_sur_fb, dim3((unsigned)(b.nb / 16)), dim3(256), b, SU.w, draw, seed);
   return 0;
-}
-
-// Backward pass after sur_forward with a target: gradient into SU.gr.
-int sur_backward(int nb) {
-  LAUNCH("sur_rowdot", k_rowdot, dim3(SUR_H), dim3(256), SU.H2, SU.dy, nb, SU.gr + SUR_OFF_W3);
-  LAUNCH("sur_rowdot", k_rowdot, dim3(1), dim3(256), SU.dy, (const float *)nullptr, nb, SU.gr + SUR_OFF_B3);
-  LAUNCH("sur_back_out", k_back_out, dim3(blocks_for((size_t)SUR_H * nb)), dim3(256), SU.Z2, SU.w, SU.dy, nb,
-         SU.dZ2);
-  LAUNCH("sur_rowdot", k_rowdot, dim3(SUR_H), dim3(256), SU.dZ2, (const float *)nullptr, nb, SU.gr + SUR_OFF_B2);
-  // dW2[k][f] = sum_b H1[k][b] dZ2[f][b]
-  int rc = gemm(SUR_H, SUR_H, nb, SU.H1, nb, 1, SU.dZ2, 1, nb, SU.gr + SUR_OFF_W2, SUR_H, 1);
-  if (rc) return rc;
-  // dH1[k][b] = sum_f W2[k][f] dZ2[f][b]
-  rc = gemm(SUR_H, nb, SUR_H, SU.w + SUR_OFF_W2, SUR_H, 1, SU.dZ2, nb, 1, SU.dH1, nb, 1);
-  if (rc) return rc;
-  LAUNCH("sur_gelu_back", k_gelu_back, dim3(blocks_for((size_t)SUR_H * nb)), dim3(256), SU.Z1, SU.dH1,
-         SUR_H * nb, SU.dZ1);
-  LAUNCH("sur_rowdot", k_rowdot, dim3(SUR_H), dim3(256), SU.dZ1, (const float *)nullptr, nb, SU.gr + SUR_OFF_B1);
-  // dW1[k][f] = sum_b X[b][k] dZ1[f][b]
-  return gemm(SUR_K, SUR_H, nb, SU.Xb, 1, SUR_K, SU.dZ1, 1, nb, SU.gr + SUR_OFF_W1, SUR_H, 1);
 }
 
 int sur_enabled() { return SU.enabled; }
@@ -1987,18 +1954,14 @@ int api_sur_train(int32_t steps, int32_t batch, float lr, uint64_t seed, float *
   const float b1 = 0.9f, b2 = 0.999f;
   for (int s = 0; s < steps; ++s) {
     const unsigned long long bseed = mix64(seed * 0x9E3779B97F4A7C15ull + (unsigned long long)s);
-    LAUNCH("sur_batch", k_sur_batch, dim3(blocks_for((size_t)batch * SUR_K)), dim3(256), SU.X, SU.y, SU.rows, bseed,
-           batch, SU.Xb, SU.yb);
-    rc = sur_forward(batch, batch, SU.yb);
-    if (rc) return rc;
-    LAUNCH("sur_loss", k_sum_into, dim3(1), dim3(64), SU.lossacc, (int)blocks_for(batch), 1.0f / (float)batch,
-           SU.losshist + s);
-    rc = sur_backward(batch);
+    const SurBatch bt = sur_batch(SU.X, SU.y, batch, batch);
+    rc = sur_fb(bt, SU.rows, bseed);
     if (rc) return rc;
     SU.adam_t += 1;
     const float c1 = 1.0f - powf(b1, (float)SU.adam_t), c2 = 1.0f - powf(b2, (float)SU.adam_t);
-    LAUNCH("sur_adam", k_adam, dim3(blocks_for(SUR_NPARAM)), dim3(256), SU.w, SU.gr, SU.m, SU.v, SUR_NPARAM, lr, b1,
-           b2, 1.0e-8f, c1, c2);
+    const AdamArgs aa = {SU.w, SU.m, SU.v, lr, b1, b2, 1.0e-8f, c1, c2};
+    LAUNCH("sur_grads", k_sur_grads<true>, dim3(SUR_GB_ALL), dim3(256), bt, aa, SU.gr, SU.lossacc,
+           1.0f / (float)batch, SU.losshist + s, 1);
   }
   rc = sur_pack();
   if (rc) return rc;
@@ -2014,7 +1977,7 @@ int api_sur_forward(const float *X, int32_t rows, float *y) {
   int nb;
   int rc = sur_stage_rows(X, nullptr, rows, &nb);
   if (rc) return rc;
-  rc = sur_forward(nb, rows, nullptr);
+  rc = sur_fb(sur_batch(SU.Xb, nullptr, nb, rows), 0, 0);
   if (rc) return rc;
   HIPCHK(hipStreamSynchronize(S.stream));
   HIPCHK(hipMemcpy(y, SU.yo, sizeof(float) * rows, hipMemcpyDeviceToHost));
@@ -2028,10 +1991,11 @@ int api_sur_grad(const float *X, const float *t, int32_t rows, float *grad, floa
   int nb;
   int rc = sur_stage_rows(X, t, rows, &nb);
   if (rc) return rc;
-  rc = sur_forward(nb, rows, SU.yb);
+  const SurBatch bt = sur_batch(SU.Xb, SU.yb, nb, rows);
+  rc = sur_fb(bt, 0, 0);
   if (rc) return rc;
-  rc = sur_backward(nb);
-  if (rc) return rc;
+  LAUNCH("sur_grads", k_sur_grads<false>, dim3(SUR_GB_ALL), dim3(256), bt, AdamArgs{}, SU.gr, SU.lossacc, 1.0f,
+         (float *)nullptr, 0);
   HIPCHK(hipStreamSynchronize(S.stream));
   HIPCHK(hipMemcpy(grad, SU.gr, sizeof(float) * SUR_NPARAM, hipMemcpyDeviceToHost));
   if (loss) {

@@ -173,130 +173,281 @@ __global__ void k_sur_standardise(float *__restrict__ X, float *__restrict__ y, 
 // ----------------------------------------------------------------------------
 // training
 // ----------------------------------------------------------------------------
-// C(m, n) = sum_k A(m, k) B(k, n) with BF16 operands (rounded from FP32) and
-// FP32 accumulation; element (m, k) of A at A[m * sam + k * sak], and so on.
-// M, N, K multiples of 16; one wave per 16 x 16 tile of C.
-__global__ __launch_bounds__(64) void k_gemm_bf16(int M, int N, int K, const float *__restrict__ A, int sam, int sak,
-                                                  const float *__restrict__ B, int sbk, int sbn,
-                                                  float *__restrict__ C, int scm, int scn) {
-  const int l = threadIdx.x;
-  const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16;
-  if (m0 >= M || n0 >= N) return;
-  const int am = m0 + (l & 15), bn = n0 + (l & 15), kq = 4 * (l >> 4);
-  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    const int kb = k0 + kq;
-    const float *pa = A + (size_t)am * sam + (size_t)kb * sak;
-    const float *pb = B + (size_t)kb * sbk + (size_t)bn * sbn;
-    const bf16x4 a = pack4(pa[0], pa[sak], pa[2 * sak], pa[3 * sak]);
-    const bf16x4 b = pack4(pb[0], pb[sbk], pb[2 * sbk], pb[3 * sbk]);
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+// A mini-batch takes two launches: k_sur_fb runs forward and backward through
+// the network, 16 columns per block, and k_sur_grads forms every parameter
+// gradient (and applies Adam).  On batches of some hundred rows it is all
+// latency; the sixteen launches of separate products, activations, row sums
+// and the update took 78 us per step of 512 rows, these two take 22.
+//
+// Products have BF16 operands (rounded from FP32) and FP32 accumulation, K in
+// steps of 16 in order; everything else is FP32.
+
+// Columns of one mini-batch and what k_sur_fb leaves for k_sur_grads,
+// feature-major rows of length nb (a multiple of 16).
+struct SurBatch {
+  const float *X, *y;        // rows of SUR_K inputs; targets, or NULL
+  int *row;                  // row of X (and y) of each column
+  float *H1, *H2, *dZ1, *dZ2;
+  float *yo, *dy;
+  int nb, nreal;             // columns; those that are rows (the rest is padding)
+};
+
+// Forward and, with a target, backward over 16 columns.  Wave w holds features
+// 16 w .. 16 w + 15: the fragment that the MFMA leaves in its registers is the
+// K step w of the next product's B operand, so layers pass BF16 fragments
+// through LDS.  With draw >= 0 rows are given, column b takes row
+// hash(seed, b) % draw and keeps it in row[]; otherwise row b, and the
+// padding columns zeros.
+// All weights but layer 1's are loaded ahead of the products that need them.
+#define SUR_FB_K 21  // K steps of layer 1 whose loads are issued together
+static_assert((SUR_K / 16) % SUR_FB_K == 0, "layer 1 in whole batches of K steps");
+__global__ __launch_bounds__(256) void k_sur_fb(SurBatch s, const float *__restrict__ w, int draw,
+                                                unsigned long long seed) {
+  __shared__ bf16x4 frag[2][4][64];
+  __shared__ float sh2[SUR_H][17], sdy[16], sw3[SUR_H];
+  const int l = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+  const int col = l & 15, kq = 4 * (l >> 4);
+  const int b = (int)blockIdx.x * 16 + col;
+  const bool real_row = b < s.nreal;
+  int r = b;
+  if (draw > 0) {
+    r = (int)(mix64(seed + (unsigned long long)b) % (unsigned long long)draw);
+    if (threadIdx.x < 16) s.row[b] = r;
   }
-  const int cn = n0 + (l & 15);
+  const int f0 = wave * 16;
+  bf16x4 w2f[4], w2b[4];  // W2 for the forward and the backward product
+  float b1[4], b2[4], w3[4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) C[(size_t)(m0 + kq + r) * scm + (size_t)cn * scn] = acc[r];
-}
-
-// Z[f][b] += bias[f]; H = GELU(Z)   (feature-major, rows of length nb)
-__global__ void k_bias_gelu(float *__restrict__ Z, float *__restrict__ H, const float *__restrict__ bias, int nf,
-                            int nb) {
-  const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (t >= nf * nb) return;
-  const float z = Z[t] + bias[t / nb];
-  Z[t] = z;
-  H[t] = gelu(z);
-}
-
-// output layer, loss and its gradient over columns b < nb (row length nb):
-// y[b] = sum_f W3[f] H2[f][b] + b3; for the first nreal columns with a
-// target, dy[b] = 2 (y - t) / nreal and lossacc[block] = sum (y - t)^2;
-// dy = 0 on padding columns.
-__global__ __launch_bounds__(256) void k_out_layer(const float *__restrict__ H2, const float *__restrict__ w,
-                                                   const float *__restrict__ tgt, int nb, int nreal,
-                                                   float *__restrict__ yout, float *__restrict__ dy,
-                                                   float *__restrict__ lossacc) {
-  __shared__ float red[4];
-  const int b = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  float e2 = 0.0f;
-  if (b < nb) {
-    float y = w[SUR_OFF_B3];
-    for (int f = 0; f < SUR_H; ++f) y += w[SUR_OFF_W3 + f] * H2[(size_t)f * nb + b];
-    yout[b] = y;
-    if (tgt) {
+  for (int kk = 0; kk < 4; ++kk) {
+    const float *pf = w + SUR_OFF_W2 + (kk * 16 + kq) * SUR_H + f0 + col;
+    w2f[kk] = pack4(pf[0], pf[SUR_H], pf[2 * SUR_H], pf[3 * SUR_H]);
+    const float *pb = w + SUR_OFF_W2 + (f0 + col) * SUR_H + kk * 16 + kq;
+    w2b[kk] = pack4(pb[0], pb[1], pb[2], pb[3]);
+    b1[kk] = w[SUR_OFF_B1 + f0 + kq + kk];
+    b2[kk] = w[SUR_OFF_B2 + f0 + kq + kk];
+    w3[kk] = w[SUR_OFF_W3 + f0 + kq + kk];
+  }
+  const float b3 = w[SUR_OFF_B3];
+  if (threadIdx.x < SUR_H) sw3[threadIdx.x] = w[SUR_OFF_W3 + threadIdx.x];
+  const float tgt = s.y && real_row ? s.y[r] : 0.0f;
+  // layer 1
+  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int st = 0; st < SUR_K / 16; st += SUR_FB_K) {
+    float wa[SUR_FB_K][4];
+    float4 xb[SUR_FB_K];
+#pragma unroll
+    for (int q = 0; q < SUR_FB_K; ++q) {
+      const int kb = (st + q) * 16 + kq;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) wa[q][t] = w[SUR_OFF_W1 + (kb + t) * SUR_H + f0 + col];
+      xb[q] = real_row ? *(const float4 *)(s.X + (size_t)r * SUR_K + kb) : float4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+#pragma unroll
+    for (int q = 0; q < SUR_FB_K; ++q)
+      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pack4(wa[q][0], wa[q][1], wa[q][2], wa[q][3]),
+                                                      pack4(xb[q].x, xb[q].y, xb[q].z, xb[q].w), acc, 0, 0, 0);
+  }
+  float z1[4], h[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    z1[t] = acc[t] + b1[t];
+    h[t] = gelu(z1[t]);
+    if (s.y) s.H1[(size_t)(f0 + kq + t) * s.nb + b] = h[t];
+  }
+  frag[0][wave][l] = pack4(h[0], h[1], h[2], h[3]);
+  __syncthreads();
+  // layer 2
+  acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk)
+    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w2f[kk], frag[0][kk][l], acc, 0, 0, 0);
+  float z2[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    z2[t] = acc[t] + b2[t];
+    h[t] = gelu(z2[t]);
+    sh2[f0 + kq + t][col] = h[t];
+    if (s.y) s.H2[(size_t)(f0 + kq + t) * s.nb + b] = h[t];
+  }
+  __syncthreads();
+  // output layer: y = W3 . H2 + b3 in feature order; dy = 2 (y - t) / nreal on
+  // the real columns, 0 on the padding
+  if (threadIdx.x < 16) {
+    float y = b3;
+#pragma unroll 16
+    for (int f = 0; f < SUR_H; ++f) y += sw3[f] * sh2[f][col];
+    s.yo[b] = y;
+    if (s.y) {
       float d = 0.0f;
-      if (b < nreal) {
-        const float e = y - tgt[b];
-        e2 = e * e;
-        d = 2.0f * e / (float)nreal;
+      if (real_row) {
+        const float e = y - tgt;
+        d = 2.0f * e / (float)s.nreal;
       }
-      dy[b] = d;
+      s.dy[b] = d;
+      sdy[col] = d;
     }
   }
-  for (int off = 32; off > 0; off >>= 1) e2 += __shfl_down(e2, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e2;
+  if (!s.y) return;
   __syncthreads();
-  if (threadIdx.x == 0) lossacc[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
-}
-
-// dZ2[f][b] = W3[f] dy[b] * gelu'(Z2[f][b])
-__global__ void k_back_out(const float *__restrict__ Z2, const float *__restrict__ w, const float *__restrict__ dy,
-                           int nb, float *__restrict__ dZ2) {
-  const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (t >= SUR_H * nb) return;
-  const int f = t / nb, b = t % nb;
-  dZ2[t] = w[SUR_OFF_W3 + f] * dy[b] * gelu_grad(Z2[t]);
-}
-
-// dZ[t] = dH[t] * gelu'(Z[t])
-__global__ void k_gelu_back(const float *__restrict__ Z, const float *__restrict__ dH, int n, float *__restrict__ dZ) {
-  const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (t >= n) return;
-  dZ[t] = dH[t] * gelu_grad(Z[t]);
-}
-
-// out[r] = sum_b M[r][b] * (v ? v[b] : 1)  (one block per row)
-__global__ __launch_bounds__(256) void k_rowdot(const float *__restrict__ Mx, const float *__restrict__ v, int nb,
-                                                float *__restrict__ out) {
-  __shared__ float red[4];
-  const int r = blockIdx.x;
-  float s = 0.0f;
-  for (int b = threadIdx.x; b < nb; b += 256) s += Mx[(size_t)r * nb + b] * (v ? v[b] : 1.0f);
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  // backward: dZ2 = W3 dy gelu'(Z2), dH1 = W2 dZ2, dZ1 = dH1 gelu'(Z1)
+  float dz[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    dz[t] = w3[t] * sdy[col] * gelu_grad(z2[t]);
+    s.dZ2[(size_t)(f0 + kq + t) * s.nb + b] = dz[t];
+  }
+  frag[1][wave][l] = pack4(dz[0], dz[1], dz[2], dz[3]);
   __syncthreads();
-  if (threadIdx.x == 0) out[r] = red[0] + red[1] + red[2] + red[3];
-}
-
-// mini-batch of a training step: rows picked by hash (with replacement)
-__global__ void k_sur_batch(const float *__restrict__ X, const float *__restrict__ y, int rows,
-                            unsigned long long seed, int nb, float *__restrict__ Xb, float *__restrict__ yb) {
-  const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (t >= nb * SUR_K) return;
-  const int b = t / SUR_K, kk = t % SUR_K;
-  const int r = (int)(mix64(seed + (unsigned long long)b) % (unsigned long long)rows);
-  Xb[t] = X[(size_t)r * SUR_K + kk];
-  if (kk == 0) yb[b] = y[r];
-}
-
-// *out = scale * sum of n partials (one thread)
-__global__ void k_sum_into(const float *__restrict__ part, int n, float scale, float *__restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  float s = 0.0f;
-  for (int q = 0; q < n; ++q) s += part[q];
-  *out = s * scale;
+  acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk)
+    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w2b[kk], frag[1][kk][l], acc, 0, 0, 0);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) s.dZ1[(size_t)(f0 + kq + t) * s.nb + b] = acc[t] * gelu_grad(z1[t]);
 }
 
 // Adam (Kingma & Ba 2015) on the FP32 master parameters.
-__global__ void k_adam(float *__restrict__ w, const float *__restrict__ gr, float *__restrict__ m,
-                       float *__restrict__ v, int n, float lr, float b1, float b2, float eps, float c1, float c2) {
-  const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (t >= n) return;
-  const float gg = gr[t];
-  const float mm = b1 * m[t] + (1.0f - b1) * gg;
-  const float vv = b2 * v[t] + (1.0f - b2) * gg * gg;
-  m[t] = mm;
-  v[t] = vv;
-  w[t] = w[t] - lr * (mm / c1) / (sqrtf(vv / c2) + eps);
+struct AdamArgs {
+  float *w, *m, *v;
+  float lr, b1, b2, eps, c1, c2;
+};
+__device__ __forceinline__ void adam(const AdamArgs &a, int t, float gg) {
+  const float mm = a.b1 * a.m[t] + (1.0f - a.b1) * gg;
+  const float vv = a.b2 * a.v[t] + (1.0f - a.b2) * gg * gg;
+  a.m[t] = mm;
+  a.v[t] = vv;
+  a.w[t] = a.w[t] - a.lr * (mm / a.c1) / (sqrtf(vv / a.c2) + a.eps);
+}
+
+// Parameter gradients of a batch, one role per block:
+//   blocks 0 .. SUR_GB_W1-1   dW1[k][f] = sum_b X[b][k] dZ1[f][b], four 16 x 16
+//                             tiles each (one per wave)
+//   the next SUR_GB_W2        dW2[k][f] = sum_b H1[k][b] dZ2[f][b]
+//   then one row sum each     dW3[f] = sum_b H2[f][b] dy[b], db3 = sum dy,
+//                             db2[f] = sum dZ2[f], db1[f] = sum dZ1[f]
+//   the last                  the loss: lossacc[q] = sum (y - t)^2 over columns
+//                             256 q .. 256 q + 255, loss = scale sum lossacc
+// ADAM: the update runs on the gradient where it is formed (nothing here
+// reads the parameters); otherwise the gradients go to gr.
+#define SUR_GB_W1 (SUR_K / 16)
+#define SUR_GB_W2 4
+#define SUR_GB_ROWS (3 * SUR_H + 1)
+#define SUR_GB_ALL (SUR_GB_W1 + SUR_GB_W2 + SUR_GB_ROWS + 1)
+// The products take SUR_GB_C columns at a time: the block gathers its 16
+// inputs of those rows (64 bytes each) into LDS as BF16, all loads in flight
+// together, and the waves issue SUR_GB_U loads of their other operand at once.
+#define SUR_GB_C 512
+#define SUR_GB_P (SUR_GB_C + 8)  // padded LDS row
+#define SUR_GB_U 16
+template <bool ADAM>
+__global__ __launch_bounds__(256) void k_sur_grads(SurBatch s, AdamArgs a, float *__restrict__ gr,
+                                                   float *__restrict__ lossacc, float scale, float *__restrict__ loss,
+                                                   int drawn) {
+  __shared__ float red[4];
+  __shared__ __attribute__((aligned(16))) unsigned short sA[16 * SUR_GB_P];
+  const int l = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+  const int col = l & 15, kq = 4 * (l >> 4), nb = s.nb;
+  const int blk = (int)blockIdx.x;
+  auto put = [&](int t, float v) {
+    if (ADAM) adam(a, t, v);
+    else gr[t] = v;
+  };
+  if (blk < SUR_GB_W1 + SUR_GB_W2) {
+    const bool first = blk < SUR_GB_W1;
+    const int m0 = (first ? blk : blk - SUR_GB_W1) * 16, n0 = wave * 16;
+    const float *pb = (first ? s.dZ1 : s.dZ2) + (size_t)(n0 + col) * nb;
+    const int t = (int)threadIdx.x, rq = t >> 2, cq = 4 * (t & 3);
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int c0 = 0; c0 < nb; c0 += SUR_GB_C) {
+      const int cn = nb - c0 < SUR_GB_C ? nb - c0 : SUR_GB_C;
+      // A(m, b): inputs m0 .. m0+15 (or rows of H1) of the columns, to sA[m][b]
+      float4 v[SUR_GB_C / 64];
+      if (first) {
+        int row[SUR_GB_C / 64];
+#pragma unroll
+        for (int q = 0; q < SUR_GB_C / 64; ++q) {
+          const int c = c0 + 64 * q + rq;
+          row[q] = c < s.nreal ? (drawn ? s.row[c] : c) : -1;
+        }
+#pragma unroll
+        for (int q = 0; q < SUR_GB_C / 64; ++q)
+          v[q] = row[q] >= 0 ? *(const float4 *)(s.X + (size_t)row[q] * SUR_K + m0 + cq)
+                             : float4{0.0f, 0.0f, 0.0f, 0.0f};
+      } else {
+        // thread (t & 15, t >> 4): row m0 + (t & 15), four columns at a time
+#pragma unroll
+        for (int q = 0; q < SUR_GB_C / 64; ++q) {
+          const int c = 64 * q + 4 * (t >> 4);
+          v[q] = c < cn ? *(const float4 *)(s.H1 + (size_t)(m0 + (t & 15)) * nb + c0 + c)
+                        : float4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < SUR_GB_C / 64; ++q) {
+        const bf16x4 p = pack4(v[q].x, v[q].y, v[q].z, v[q].w);
+        if (first) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) sA[(cq + j) * SUR_GB_P + 64 * q + rq] = (unsigned short)p[j];
+        } else {
+          *(bf16x4 *)(sA + (t & 15) * SUR_GB_P + 64 * q + 4 * (t >> 4)) = p;
+        }
+      }
+      __syncthreads();
+      for (int k0 = 0; k0 < cn; k0 += 16 * SUR_GB_U) {
+        float4 bv[SUR_GB_U];
+#pragma unroll
+        for (int q = 0; q < SUR_GB_U; ++q) {
+          const int k = k0 + 16 * q < cn ? k0 + 16 * q : 0;  // past the end: any column, unused
+          bv[q] = *(const float4 *)(pb + c0 + k + kq);
+        }
+#pragma unroll
+        for (int q = 0; q < SUR_GB_U; ++q)
+          if (k0 + 16 * q < cn)
+            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                *(const bf16x4 *)(sA + col * SUR_GB_P + k0 + 16 * q + kq),
+                pack4(bv[q].x, bv[q].y, bv[q].z, bv[q].w), acc, 0, 0, 0);
+      }
+    }
+    const int off = first ? SUR_OFF_W1 : SUR_OFF_W2;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) put(off + (m0 + kq + j) * SUR_H + n0 + col, acc[j]);
+    return;
+  }
+  const int rs = blk - SUR_GB_W1 - SUR_GB_W2;
+  if (rs < SUR_GB_ROWS) {
+    const int f = rs < SUR_H ? rs : (rs - 1) % SUR_H;
+    const float *m = rs < SUR_H ? s.H2 : (rs == SUR_H ? s.dy : (rs <= 2 * SUR_H ? s.dZ2 : s.dZ1));
+    const int t = rs < SUR_H ? SUR_OFF_W3 + f
+                             : (rs == SUR_H ? SUR_OFF_B3 : (rs <= 2 * SUR_H ? SUR_OFF_B2 + f : SUR_OFF_B1 + f));
+    if (rs != SUR_H) m += (size_t)f * nb;
+    float v = 0.0f;
+    for (int b = (int)threadIdx.x; b < nb; b += 256) v += m[b] * (rs < SUR_H ? s.dy[b] : 1.0f);
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    if (l == 0) red[wave] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) put(t, red[0] + red[1] + red[2] + red[3]);
+    return;
+  }
+  float sum = 0.0f;
+  for (int q = 0; q * 256 < nb; ++q) {
+    const int b = q * 256 + (int)threadIdx.x;
+    float e2 = 0.0f;
+    if (b < s.nreal) {
+      const float e = s.yo[b] - s.y[drawn ? s.row[b] : b];
+      e2 = e * e;
+    }
+    for (int off = 32; off > 0; off >>= 1) e2 += __shfl_down(e2, off, 64);
+    if (l == 0) red[wave] = e2;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const float part = red[0] + red[1] + red[2] + red[3];
+      lossacc[q] = part;
+      sum += part;
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0 && loss) *loss = sum * scale;
 }
 
 // ----------------------------------------------------------------------------

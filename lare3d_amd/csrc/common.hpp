@@ -143,6 +143,18 @@ __device__ __forceinline__ float operator/(float a, const Recip<float> &b) {
   q = fmaf(fmaf(-b.d, q, a), b.y, q);
   return fmaf(fmaf(-b.d, q, a), b.y, q);
 }
+// Square root of a positive normal number: the steps of the compiler's
+// correctly rounded root (Goldschmidt's iteration with fused remainders) less
+// its scaling and its cases for zero and infinity.
+__device__ __forceinline__ double sqrt_pos(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  h = fma(h, r, h);
+  g = fma(g, r, g);
+  g = fma(fma(-g, g, x), h, g);
+  return fma(fma(-g, g, x), h, g);
+}
 // the same divisor for FP64 numerators
 __device__ __forceinline__ const Recip<double> &wide(const Recip<double> &r) { return r; }
 __device__ __forceinline__ Recip<double> wide(const Recip<float> &r) { return recip((double)r.d); }

@@ -54,11 +54,16 @@ __device__ __forceinline__ double ghost_read(const Geo &g, const real *__restric
 // and t*sqrt(t) carried in double-double (FMA-exact products, sqrt(t) =
 // r + (t - r^2) / (2r)), rounded once.  The oracle computes the same
 // operations (a libm pow is not correctly rounded for every argument).
+// The root's low part is a division whose quotient matters to its leading
+// bits only; arguments outside 1e+-100 take the library root.
+__device__ __forceinline__ double root(double t) {
+  return __builtin_expect(t > 1.0e-100 && t < 1.0e100, 1) ? sqrt_pos(t) : sqrt(t);
+}
 __device__ __forceinline__ double pow25(double t) {
   if (!(t > 0.0) || t == INFINITY) return t == 0.0 ? 0.0 : (t > 0.0 ? t : __builtin_nan(""));
-  const double r = sqrt(t);
+  const double r = root(t);
   const double e = fma(-r, r, t);
-  const double rl = e / (2.0 * r);
+  const double rl = e / recip(2.0 * r);
   const double h2 = t * t;
   const double l2 = fma(t, t, -h2);
   const double p = h2 * r;
@@ -68,9 +73,9 @@ __device__ __forceinline__ double pow25(double t) {
 }
 __device__ __forceinline__ double pow15(double t) {
   if (!(t > 0.0) || t == INFINITY) return t == 0.0 ? 0.0 : (t > 0.0 ? t : __builtin_nan(""));
-  const double r = sqrt(t);
+  const double r = root(t);
   const double e = fma(-r, r, t);
-  const double rl = e / (2.0 * r);
+  const double rl = e / recip(2.0 * r);
   const double p = t * r;
   if (!(p < INFINITY)) return p;
   const double pl = fma(t, r, -p);
@@ -148,76 +153,65 @@ __global__ __launch_bounds__(BX * BY) void k_larsen(Geo g, const real *__restric
   block_reduce_store<1>(v, ops, partial);
 }
 
-// Face flux fc_sp of conduct.f90:176-207 (x face between cells ix, ix+1),
-// given the temperature neighbourhood T[a][b][c] with a,b,c in {0,1,2}
-// meaning offsets -1,0,+1 around the *lower* cell... see callers.
-// The three face kinds are written out separately, in the reference's
-// operation order.
+// Face flux fc_sp of conduct.f90:176-207 (x face between cells ix, ix+1, and
+// the y and z analogues) from the field at the face, the larger of the face
+// temperature tb and 0, and the temperature gradients along the normal (tg)
+// and along the two transverse axes (a1, a2).  b: the field along x, y, z at
+// the face; n, t1, t2: its normal and transverse components.
+struct FaceB {
+  acc x, y, z;
+};
+__device__ __forceinline__ acc face_flux(const FaceB &b, acc n, acc t1, acc t2, acc tb, acc tg, acc a1, acc a2,
+                                         acc L, acc kappa_0) {
+  const acc modb = b.x * b.x + b.y * b.y + b.z * b.z + (acc)MIN_B;
+  tb = dmax(tb, (acc)0.0);
+  return -L * kappa_0 * pow25(tb) * (n * (tg * n + a1 * t1 + a2 * t2) + tg * (acc)MIN_B) / recip(modb);
+}
+// average of four values of the FP64 face field, in the reference's order
+__device__ __forceinline__ acc mean4(double a, double b, double c, double d) { return (acc)(0.25 * (a + b + c + d)); }
 
 struct Tn {  // 3x3x3 temperature neighbourhood of a cell (corners unused)
   acc t[3][3][3];
 };
-
-// x face between (ox,oy,oz)+(0,0,0) and +(1,0,0) relative to centre index
-// (1,1,1) of the neighbourhood, lower cell at neighbourhood x index lx.
-__device__ __forceinline__ acc flux_x_face(const Geo &g, const Tn &T, int lx, int ix, int iy, int iz,
-                                              const double *__restrict__ bx, const double *__restrict__ by,
-                                              const double *__restrict__ bz, acc L, acc kappa_0) {
-  const int c = g.idx(ix, iy, iz);
-  const acc byf = (acc)(0.25 * (by[c] + by[c + 1] + by[c - g.sy] + by[c + 1 - g.sy]));
-  const acc bzf = (acc)(0.25 * (bz[c] + bz[c + 1] + bz[c - g.sz] + bz[c + 1 - g.sz]));
-  const acc bxc = (acc)bx[c];
-  const acc modb = bxc * bxc + byf * byf + bzf * bzf + (acc)MIN_B;
-  acc tb = (T.t[lx + 1][1][1] + T.t[lx][1][1]) / (acc)2.0;
-  acc tb_p = (T.t[lx + 1][2][1] + T.t[lx][2][1]) / (acc)2.0;
-  acc tb_m = (T.t[lx + 1][0][1] + T.t[lx][0][1]) / (acc)2.0;
-  const acc tg_a1 = (tb_p - tb_m) / (acc)(g.dyc[iy] + g.dyc[iy - 1]);
-  tb_p = (T.t[lx + 1][1][2] + T.t[lx][1][2]) / (acc)2.0;
-  tb_m = (T.t[lx + 1][1][0] + T.t[lx][1][0]) / (acc)2.0;
-  const acc tg_a2 = (tb_p - tb_m) / (acc)(g.dzc[iz] + g.dzc[iz - 1]);
-  const acc tg = (T.t[lx + 1][1][1] - T.t[lx][1][1]) / (acc)g.dxc[ix];
-  tb = dmax(tb, (acc)0.0);
-  return -L * kappa_0 * pow25(tb) * (bxc * (tg * bxc + tg_a1 * byf + tg_a2 * bzf) + tg * (acc)MIN_B) / modb;
+// Temperatures of the three face kinds, the lower cell at neighbourhood index
+// l along the normal.  Divisors as reciprocals: dn the centre distance along
+// the normal, s1 and s2 the double distances (dyc(iy) + dyc(iy-1) etc.) of
+// the transverse gradients.
+__device__ __forceinline__ acc flux_x_face(const Tn &T, int l, const FaceB &b, acc L, acc kappa_0,
+                                           const Recip<acc> &dn, const Recip<acc> &s1, const Recip<acc> &s2) {
+  const acc tb = (T.t[l + 1][1][1] + T.t[l][1][1]) / (acc)2.0;
+  acc tb_p = (T.t[l + 1][2][1] + T.t[l][2][1]) / (acc)2.0;
+  acc tb_m = (T.t[l + 1][0][1] + T.t[l][0][1]) / (acc)2.0;
+  const acc a1 = (tb_p - tb_m) / s1;
+  tb_p = (T.t[l + 1][1][2] + T.t[l][1][2]) / (acc)2.0;
+  tb_m = (T.t[l + 1][1][0] + T.t[l][1][0]) / (acc)2.0;
+  const acc a2 = (tb_p - tb_m) / s2;
+  const acc tg = (T.t[l + 1][1][1] - T.t[l][1][1]) / dn;
+  return face_flux(b, b.x, b.y, b.z, tb, tg, a1, a2, L, kappa_0);
 }
-
-__device__ __forceinline__ acc flux_y_face(const Geo &g, const Tn &T, int ly, int ix, int iy, int iz,
-                                              const double *__restrict__ bx, const double *__restrict__ by,
-                                              const double *__restrict__ bz, acc L, acc kappa_0) {
-  const int c = g.idx(ix, iy, iz);
-  const acc bxf = (acc)(0.25 * (bx[c] + bx[c + g.sy] + bx[c - 1] + bx[c - 1 + g.sy]));
-  const acc bzf = (acc)(0.25 * (bz[c] + bz[c + g.sy] + bz[c - g.sz] + bz[c + g.sy - g.sz]));
-  const acc byc = (acc)by[c];
-  const acc modb = bxf * bxf + byc * byc + bzf * bzf + (acc)MIN_B;
-  acc tb = (T.t[1][ly + 1][1] + T.t[1][ly][1]) / (acc)2.0;
-  acc tb_p = (T.t[2][ly][1] + T.t[2][ly + 1][1]) / (acc)2.0;
-  acc tb_m = (T.t[0][ly + 1][1] + T.t[0][ly][1]) / (acc)2.0;
-  const acc tg_a1 = (tb_p - tb_m) / (acc)(g.dxc[ix] + g.dxc[ix - 1]);
-  tb_p = (T.t[1][ly + 1][2] + T.t[1][ly][2]) / (acc)2.0;
-  tb_m = (T.t[1][ly + 1][0] + T.t[1][ly][0]) / (acc)2.0;
-  const acc tg_a2 = (tb_p - tb_m) / (acc)(g.dzc[iz] + g.dzc[iz - 1]);
-  const acc tg = (T.t[1][ly + 1][1] - T.t[1][ly][1]) / (acc)g.dyc[iy];
-  tb = dmax(tb, (acc)0.0);
-  return -L * kappa_0 * pow25(tb) * (byc * (tg * byc + tg_a1 * bxf + tg_a2 * bzf) + tg * (acc)MIN_B) / modb;
+__device__ __forceinline__ acc flux_y_face(const Tn &T, int l, const FaceB &b, acc L, acc kappa_0,
+                                           const Recip<acc> &dn, const Recip<acc> &s1, const Recip<acc> &s2) {
+  const acc tb = (T.t[1][l + 1][1] + T.t[1][l][1]) / (acc)2.0;
+  acc tb_p = (T.t[2][l][1] + T.t[2][l + 1][1]) / (acc)2.0;
+  acc tb_m = (T.t[0][l + 1][1] + T.t[0][l][1]) / (acc)2.0;
+  const acc a1 = (tb_p - tb_m) / s1;
+  tb_p = (T.t[1][l + 1][2] + T.t[1][l][2]) / (acc)2.0;
+  tb_m = (T.t[1][l + 1][0] + T.t[1][l][0]) / (acc)2.0;
+  const acc a2 = (tb_p - tb_m) / s2;
+  const acc tg = (T.t[1][l + 1][1] - T.t[1][l][1]) / dn;
+  return face_flux(b, b.y, b.x, b.z, tb, tg, a1, a2, L, kappa_0);
 }
-
-__device__ __forceinline__ acc flux_z_face(const Geo &g, const Tn &T, int lz, int ix, int iy, int iz,
-                                              const double *__restrict__ bx, const double *__restrict__ by,
-                                              const double *__restrict__ bz, acc L, acc kappa_0) {
-  const int c = g.idx(ix, iy, iz);
-  const acc bxf = (acc)(0.25 * (bx[c] + bx[c + g.sz] + bx[c - 1] + bx[c - 1 + g.sz]));
-  const acc byf = (acc)(0.25 * (by[c] + by[c + g.sz] + by[c - g.sy] + by[c - g.sy + g.sz]));
-  const acc bzc = (acc)bz[c];
-  const acc modb = bxf * bxf + byf * byf + bzc * bzc + (acc)MIN_B;
-  acc tb = (T.t[1][1][lz + 1] + T.t[1][1][lz]) / (acc)2.0;
-  acc tb_p = (T.t[2][1][lz + 1] + T.t[2][1][lz]) / (acc)2.0;
-  acc tb_m = (T.t[0][1][lz + 1] + T.t[0][1][lz]) / (acc)2.0;
-  const acc tg_a1 = (tb_p - tb_m) / (acc)(g.dxc[ix] + g.dxc[ix - 1]);
-  tb_p = (T.t[1][2][lz + 1] + T.t[1][2][lz]) / (acc)2.0;
-  tb_m = (T.t[1][0][lz + 1] + T.t[1][0][lz]) / (acc)2.0;
-  const acc tg_a2 = (tb_p - tb_m) / (acc)(g.dyc[iy] + g.dyc[iy - 1]);
-  const acc tg = (T.t[1][1][lz + 1] - T.t[1][1][lz]) / (acc)g.dzc[iz];
-  tb = dmax(tb, (acc)0.0);
-  return -L * kappa_0 * pow25(tb) * (bzc * (tg * bzc + tg_a1 * bxf + tg_a2 * byf) + tg * (acc)MIN_B) / modb;
+__device__ __forceinline__ acc flux_z_face(const Tn &T, int l, const FaceB &b, acc L, acc kappa_0,
+                                           const Recip<acc> &dn, const Recip<acc> &s1, const Recip<acc> &s2) {
+  const acc tb = (T.t[1][1][l + 1] + T.t[1][1][l]) / (acc)2.0;
+  acc tb_p = (T.t[2][1][l + 1] + T.t[2][1][l]) / (acc)2.0;
+  acc tb_m = (T.t[0][1][l + 1] + T.t[0][1][l]) / (acc)2.0;
+  const acc a1 = (tb_p - tb_m) / s1;
+  tb_p = (T.t[1][2][l + 1] + T.t[1][2][l]) / (acc)2.0;
+  tb_m = (T.t[1][0][l + 1] + T.t[1][0][l]) / (acc)2.0;
+  const acc a2 = (tb_p - tb_m) / s2;
+  const acc tg = (T.t[1][1][l + 1] - T.t[1][1][l]) / dn;
+  return face_flux(b, b.z, b.x, b.y, tb, tg, a1, a2, L, kappa_0);
 }
 
 // Ghost mapping of one coordinate under a read mode (the per-axis part of
@@ -244,9 +238,19 @@ __device__ __forceinline__ void map_coord(int c, int n, int user, int olo, int o
 // provide their out face.  Each shared flux is the same expression on the
 // same values as the neighbour's own, and the six are summed in the order
 // of cell_heat_flux.
+//
+// Bound by load and operation latency at few waves per SIMD, not by bytes (80 B
+// per cell: 2.9 TB/s at 256^3).  The divisors fixed along the march are held
+// as reciprocals, the face field shared by successive planes in registers
+// (14 loads of B per cell instead of 22), and the common FP64 form is held to
+// the registers of three waves per SIMD (44 bytes of spills; the others fit
+// two, and FP32 four, by themselves).  A stage at 256^3 in FP64: 560 us, with
+// the reciprocals 501, with three waves 457; FP32 373, 363, and with the
+// carried field 294; 64 x 64 x 128 FP64 30.2 -> 26.3.
 #define RKL_OUT 63
+#define RKL_WAVES(PI, OPEN) (sizeof(acc) == sizeof(double) && !(PI) && !(OPEN) ? 3 : 1)
 template <int MODE, int FIRST, bool PI, bool OPEN>
-__global__ __launch_bounds__(BX * BY) void k_rkl2_z(Geo g, Box b, const real *__restrict__ Y2, const real *__restrict__ Y1,
+__global__ __launch_bounds__(BX * BY, RKL_WAVES(PI, OPEN)) void k_rkl2_z(Geo g, Box b, const real *__restrict__ Y2, const real *__restrict__ Y1,
                                                     const real *__restrict__ E0, const real *__restrict__ rho,
                                                     const double *__restrict__ bx, const double *__restrict__ by,
                                                     const double *__restrict__ bz, const real *__restrict__ larsen,
@@ -272,6 +276,10 @@ __global__ __launch_bounds__(BX * BY) void k_rkl2_z(Geo g, Box b, const real *__
     map_coord<MODE, OPEN>(j + q - 1, g.ny, g.user[1], g.open_lo[1], g.open_hi[1], ym[q], ys[q]);
   }
   const acc kap = (acc)a.kappa_0, tdt = (acc)a.dt;
+  // divisors fixed along the march
+  const Recip<acc> rdx = recip((acc)g.dxc[i]), rsx = recip((acc)(g.dxc[i] + g.dxc[i - 1]));
+  const Recip<acc> rdy0 = recip((acc)g.dyc[j - 1]), rdy1 = recip((acc)g.dyc[j]),
+                   rsy = recip((acc)(g.dyc[j] + g.dyc[j - 1]));
   // T.t[p][q][r]: x offset p-1, y offset q-1, plane k-1+r
   Tn T;
 #define RKL_LOAD_PLANE(kk, r)                                                    \
@@ -288,31 +296,57 @@ __global__ __launch_bounds__(BX * BY) void k_rkl2_z(Geo g, Box b, const real *__
   RKL_LOAD_PLANE(k0 - 1, 0)
   RKL_LOAD_PLANE(k0, 1)
   acc fz_in = 0.0;
+  // face B carried from plane to plane: bx at i, i-1 and by at j, j-1 of plane
+  // k; bz at (i, j), (i+1, j), (i, j-1), (i, j+1) of plane k-1
+  const int Y = g.sy, Z = g.sz;
+  const int ck = g.idx(i, j, k0);
+  double bx0 = bx[ck], bxm = bx[ck - 1], by0 = by[ck], bym = by[ck - Y];
+  double bzl0 = bz[ck - Z], bzlX = bz[ck + 1 - Z], bzlY = bz[ck - Y - Z], bzlP = bz[ck + Y - Z];
   for (int k = k0; k <= k1; ++k) {
     RKL_LOAD_PLANE(k + 1, 2)
     const int c0 = g.idx(i, j, k);
     const acc L0 = larsen[c0];
-    const acc fx_out = flux_x_face(g, T, 1, i, j, k, bx, by, bz, L0, kap);
+    const double bxY = bx[c0 - Y], bxmY = bx[c0 - 1 - Y], bxP = bx[c0 + Y], bxmP = bx[c0 - 1 + Y], bxZ = bx[c0 + Z],
+                 bxmZ = bx[c0 - 1 + Z];
+    const double byX = by[c0 + 1], byXm = by[c0 + 1 - Y], byZ = by[c0 + Z], bymZ = by[c0 - Y + Z];
+    const double bz0 = bz[c0], bzX = bz[c0 + 1], bzY = bz[c0 - Y], bzP = bz[c0 + Y];
+    const Recip<acc> rsz = recip((acc)(g.dzc[k] + g.dzc[k - 1]));
+    const acc fx_out = flux_x_face(T, 1, FaceB{(acc)bx0, mean4(by0, byX, bym, byXm), mean4(bz0, bzX, bzl0, bzlX)}, L0, kap, rdx,
+                                   rsy, rsz);
     const acc fx_in = __shfl_up(fx_out, 1, 64);
-    if (k == k0) fz_in = flux_z_face(g, T, 0, i, j, k - 1, bx, by, bz, (acc)larsen[c0 - g.sz], kap);
-    const acc fy_in = flux_y_face(g, T, 0, i, j - 1, k, bx, by, bz, (acc)larsen[c0 - g.sy], kap);
-    const acc fy_out = flux_y_face(g, T, 1, i, j, k, bx, by, bz, L0, kap);
-    const acc fz_out = flux_z_face(g, T, 1, i, j, k, bx, by, bz, L0, kap);
+    if (k == k0)
+      fz_in = flux_z_face(T, 0, FaceB{mean4(bx[c0 - Z], bx0, bx[c0 - 1 - Z], bxm),
+                                      mean4(by[c0 - Z], by0, by[c0 - Y - Z], bym), (acc)bzl0},
+                          (acc)larsen[c0 - Z], kap, recip((acc)g.dzc[k - 1]), rsx, rsy);
+    const acc fy_in = flux_y_face(T, 0, FaceB{mean4(bxY, bx0, bxmY, bxm), (acc)bym, mean4(bzY, bz0, bzlY, bzl0)},
+                                  (acc)larsen[c0 - Y], kap, rdy0, rsx, rsz);
+    const acc fy_out = flux_y_face(T, 1, FaceB{mean4(bx0, bxP, bxm, bxmP), (acc)by0, mean4(bz0, bzP, bzl0, bzlP)}, L0, kap, rdy1,
+                                   rsx, rsz);
+    const acc fz_out = flux_z_face(T, 1, FaceB{mean4(bx0, bxZ, bxm, bxmZ), mean4(by0, byZ, bym, bymZ), (acc)bz0}, L0, kap,
+                                   recip((acc)g.dzc[k]), rsx, rsy);
+    bx0 = bxZ;
+    bxm = bxmZ;
+    by0 = byZ;
+    bym = bymZ;
+    bzl0 = bz0;
+    bzlX = bzX;
+    bzlY = bzY;
+    bzlP = bzP;
     if (out) {
-      acc fl = (acc)0.0 + fz_in / (acc)g.dzb[k - 1];
-      fl = fl + fy_in / (acc)g.dyb[j - 1];
-      fl = fl + fx_in / (acc)g.dxb[i - 1];
-      fl = fl - fx_out / (acc)g.dxb[i];
-      fl = fl - fy_out / (acc)g.dyb[j];
-      fl = fl - fz_out / (acc)g.dzb[k];
+      acc fl = (acc)0.0 + fz_in / recip((acc)g.dzb[k - 1]);
+      fl = fl + fy_in / recip((acc)g.dyb[j - 1]);
+      fl = fl + fx_in / recip((acc)g.dxb[i - 1]);
+      fl = fl - fx_out / recip((acc)g.dxb[i]);
+      fl = fl - fy_out / recip((acc)g.dyb[j]);
+      fl = fl - fz_out / recip((acc)g.dzb[k]);
       if (FIRST) {
-        const acc lc = ((acc)1.0 / rho[c0]) * fl;
+        const acc lc = ((acc)1.0 / recip((acc)rho[c0])) * fl;
         Lc[c0] = lc;
         const acc cc = (acc)mu_t * tdt * lc;
         Yout[c0] = E0[c0] + cc;
       } else {
         const acc cc0 = (acc)gam_t * tdt * Lc[c0];
-        const acc lj = ((acc)1.0 / rho[c0]) * fl;
+        const acc lj = ((acc)1.0 / recip((acc)rho[c0])) * fl;
         const acc cc1 = (acc)mu_t * tdt * lj;
         acc y3;
         if constexpr (sizeof(acc) == sizeof(double)) {

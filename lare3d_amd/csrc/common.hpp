@@ -155,6 +155,11 @@ __device__ __forceinline__ double sqrt_pos(double x) {
   g = fma(fma(-g, g, x), h, g);
   return fma(fma(-g, g, x), h, g);
 }
+// sqrt(x): the short form in its range, the library's elsewhere (zero too)
+__device__ __forceinline__ double root(double x) {
+  return __builtin_expect(x > 1.0e-280 && x < 1.0e280, 1) ? sqrt_pos(x) : sqrt(x);
+}
+__device__ __forceinline__ float root(float x) { return sqrtf(x); }
 // the same divisor for FP64 numerators
 __device__ __forceinline__ const Recip<double> &wide(const Recip<double> &r) { return r; }
 __device__ __forceinline__ Recip<double> wide(const Recip<float> &r) { return recip((double)r.d); }

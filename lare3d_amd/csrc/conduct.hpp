@@ -54,11 +54,6 @@ __device__ __forceinline__ double ghost_read(const Geo &g, const real *__restric
 // and t*sqrt(t) carried in double-double (FMA-exact products, sqrt(t) =
 // r + (t - r^2) / (2r)), rounded once.  The oracle computes the same
 // operations (a libm pow is not correctly rounded for every argument).
-// The root's low part is a division whose quotient matters to its leading
-// bits only; arguments outside 1e+-100 take the library root.
-__device__ __forceinline__ double root(double t) {
-  return __builtin_expect(t > 1.0e-100 && t < 1.0e100, 1) ? sqrt_pos(t) : sqrt(t);
-}
 __device__ __forceinline__ double pow25(double t) {
   if (!(t > 0.0) || t == INFINITY) return t == 0.0 ? 0.0 : (t > 0.0 ? t : __builtin_nan(""));
   const double r = root(t);

@@ -132,12 +132,13 @@ __global__ __launch_bounds__(BX * BY) void k_vertex_prep(Geo g, Box b, const rea
     acc sc = cvs[0];
 #pragma unroll
     for (int q = 1; q < 8; ++q) sc = sc + cvs[q];
-    rho_v[c] = s / sc;
-    const acc cvv = (acc)0.125 * sc;
+    const Recip<acc> rsc = recip(sc);
+    rho_v[c] = s / rsc;
     acc scs = lo.cs[0] * cvs[0];
 #pragma unroll
     for (int q = 1; q < 8; ++q) scs = scs + (q < 4 ? lo.cs[q] : hi.cs[q - 4]) * cvs[q];
-    cs_v[c] = (acc)0.125 * scs / cvv;
+    // (scs / 8) / (sc / 8): the eighths are exact and cancel
+    cs_v[c] = scs / rsc;
     lo = hi;
   }
 }
@@ -332,7 +333,7 @@ __device__ __forceinline__ acc edge_heat_v(acc dxb, acc dyb, acc dzb, acc cv, co
   h = h - (acc)0.25 * dxb * dyb * a3x * aa[9];
   h = h - (acc)0.25 * dxb * dyb * a3xy * aa[10];
   h = h - (acc)0.25 * dxb * dyb * a3y * aa[11];
-  return h / cv;
+  return h / recip(cv);
 }
 
 // p_visc + visc_heat over cells 0..n+1; pressure p0 of lagran.F90:93 stored
@@ -375,9 +376,9 @@ __global__ __launch_bounds__(BX * BY) void k_visc_dt(Geo g, Box bx0, const real 
 #undef AAV
       const acc a30 = al3[c], a3x = al3[c - 1], a3xy = al3[c - 1 - Y], a3y = al3[c - Y];
       acc pv = 0.0;
-      pv = dmax(pv, -(acc)alo.a1 * sqrt(aa[0]));
-      pv = dmax(pv, -(acc)alo.a2 * sqrt(aa[1]));
-      pv = dmax(pv, -a30 * sqrt(aa[8]));
+      pv = dmax(pv, -(acc)alo.a1 * root(aa[0]));
+      pv = dmax(pv, -(acc)alo.a2 * root(aa[1]));
+      pv = dmax(pv, -a30 * root(aa[8]));
       visc_heat[c] = edge_heat_v((acc)g.dxb[i], (acc)g.dyb[j], (acc)g.dzb[k], (acc)g.cv(i, j, k), alo, ahi, a30, a3x,
                                  a3xy, a3y, aa);
       const acc r = rho[c];
@@ -393,11 +394,12 @@ __global__ __launch_bounds__(BX * BY) void k_visc_dt(Geo g, Box bx0, const real 
           if (a.write_gb) gbo[c] = (real)g_b;
           g_b = (real)g_b;
         }
-        const double cs2 = (a.gamma * (double)p + g_b * w1) / rho0;
-        const double c_visc2 = pv / rho0;
+        const Recip<double> rr = recip(rho0);
+        const double cs2 = (a.gamma * (double)p + g_b * w1) / rr;
+        const double c_visc2 = (double)pv / rr;
         const double dxb = g.dxb[i], dyb = g.dyb[j], dzb = g.dzb[k];
         const double length = dmin(dmin(dxb, dyb), dzb);
-        const double dt1 = length / (sqrt(c_visc2) + sqrt(cs2 + c_visc2));
+        const double dt1 = length / (root(c_visc2) + root(cs2 + c_visc2));
         const double dt2 = dmin(dmin(dxb / dmax(fabs((double)hx.c), NONE_ZERO), dyb / dmax(fabs((double)hy.c), NONE_ZERO)),
                                 dzb / dmax(fabs((double)hz.c), NONE_ZERO));
         v[0] = dmin(v[0], dmin(dt1, dt2));
@@ -485,23 +487,21 @@ __device__ __forceinline__ void vertex_current_vals(double dxc, double dyc, doub
   jz = (jz1 + jz2) * 0.5;
 }
 
-// The same vertex current in the arithmetic type A: the differences of
-// the FP64 face field are taken in FP64 and divided by the widths in A (for
-// A = double, the operations of vertex_current_vals).
-template <class A>
-__device__ __forceinline__ void vertex_current_acc(double dxc, double dyc, double dzc, const BPlane &lo,
-                                                   const BPlane &hi, double bz0, double bzx, double bzy, double bzxy,
-                                                   A &jx, A &jy, A &jz) {
-  const A ax = (A)dxc, ay = (A)dyc, az = (A)dzc;
-  const A jx1 = (A)(bzy - bz0) / ay - (A)(hi.by0 - lo.by0) / az;
-  const A jx2 = (A)(bzxy - bzx) / ay - (A)(hi.byx - lo.byx) / az;
-  const A jy1 = (A)(hi.bx0 - lo.bx0) / az - (A)(bzx - bz0) / ax;
-  const A jy2 = (A)(hi.bxy - lo.bxy) / az - (A)(bzxy - bzy) / ax;
-  const A jz1 = (A)(lo.byx - lo.by0) / ax - (A)(lo.bxy - lo.bx0) / ay;
-  const A jz2 = (A)(hi.byx - hi.by0) / ax - (A)(hi.bxy - hi.bx0) / ay;
-  jx = (jx1 + jx2) * (A)0.5;
-  jy = (jy1 + jy2) * (A)0.5;
-  jz = (jz1 + jz2) * (A)0.5;
+// The same vertex current in the arithmetic type: the differences of the
+// FP64 face field are taken in FP64 and divided by the widths (as reciprocals
+// of dxc, dyc, dzc) in it; for FP64, the quotients of vertex_current_vals.
+__device__ __forceinline__ void vertex_current_acc(const Recip<acc> &ax, const Recip<acc> &ay, const Recip<acc> &az,
+                                                   const BPlane &lo, const BPlane &hi, double bz0, double bzx,
+                                                   double bzy, double bzxy, acc &jx, acc &jy, acc &jz) {
+  const acc jx1 = (acc)(bzy - bz0) / ay - (acc)(hi.by0 - lo.by0) / az;
+  const acc jx2 = (acc)(bzxy - bzx) / ay - (acc)(hi.byx - lo.byx) / az;
+  const acc jy1 = (acc)(hi.bx0 - lo.bx0) / az - (acc)(bzx - bz0) / ax;
+  const acc jy2 = (acc)(hi.bxy - lo.bxy) / az - (acc)(bzxy - bzy) / ax;
+  const acc jz1 = (acc)(lo.byx - lo.by0) / ax - (acc)(lo.bxy - lo.bx0) / ay;
+  const acc jz2 = (acc)(hi.byx - hi.by0) / ax - (acc)(hi.bxy - hi.bx0) / ay;
+  jx = (jx1 + jx2) * (acc)0.5;
+  jy = (jy1 + jy2) * (acc)0.5;
+  jz = (jz1 + jz2) * (acc)0.5;
 }
 
 // the same vertex current, read from memory at node (i, j, k)
@@ -521,13 +521,13 @@ __global__ __launch_bounds__(BX * BY) void k_eta(Geo g, Box b, const double *__r
                       double j_max) {
   ZCOLUMN(b, i, j, k0, k1);
   const int Y = g.sy, Z = g.sz;
+  const Recip<acc> rx = recip((acc)g.dxc[i]), ry = recip((acc)g.dyc[j]);
   BPlane lo = bplane(bx, by, g.idx(i, j, k0), Y);
   for (int k = k0; k <= k1; ++k) {
     const int c = g.idx(i, j, k);
     const BPlane hi = bplane(bx, by, c + Z, Y);
     acc jx, jy, jz;
-    vertex_current_acc<acc>(g.dxc[i], g.dyc[j], g.dzc[k], lo, hi, bz[c], bz[c + 1], bz[c + Y], bz[c + 1 + Y], jx, jy,
-                            jz);
+    vertex_current_acc(rx, ry, recip((acc)g.dzc[k]), lo, hi, bz[c], bz[c + 1], bz[c + Y], bz[c + 1 + Y], jx, jy, jz);
     eta[c] = sqrt(jx * jx + jy * jy + jz * jz) > (acc)j_max ? eta_bg + eta0 : eta_bg;
     lo = hi;
   }
@@ -615,6 +615,7 @@ __global__ __launch_bounds__(64 * RS_ROWS) void k_resist(Geo g, Box b, int tiles
   // cell box of the energy clamp, in the plane
   const bool cij = i >= -1 && i <= g.nx + 2 && j >= -1 && j <= g.ny + 2;
   const bool hij = i >= 1 && i <= g.nx && j >= 1 && j <= g.ny;  // heated cells, in the plane
+  const Recip<acc> rx = recip(eij ? (acc)g.dxc[i] : (acc)1.0), ry = recip(eij ? (acc)g.dyc[j] : (acc)1.0);
   double v = 0.0;
   EPlane m = {0, 0, 0, 0, 0, 0, 0};  // plane k-1
   acc mq[4] = {0, 0, 0, 0};          // curlb of plane k-1 at (i,j), (i-1,j), (i,j-1), (i-1,j-1)
@@ -627,8 +628,8 @@ __global__ __launch_bounds__(64 * RS_ROWS) void k_resist(Geo g, Box b, int tiles
       if (!have_lo) lo = bplane(bx, by, c, Y);
       const BPlane hi = bplane(bx, by, c + Z, Y);
       acc jx, jy, jz;
-      vertex_current_acc<acc>(g.dxc[i], g.dyc[j], g.dzc[k], lo, hi, bz[c], bz[c + 1], bz[c + Y], bz[c + 1 + Y], jx,
-                              jy, jz);
+      vertex_current_acc(rx, ry, recip((acc)g.dzc[k]), lo, hi, bz[c], bz[c + 1], bz[c + Y], bz[c + 1 + Y], jx, jy,
+                         jz);
       const BPlane plo = lo;
       lo = hi;
       have_lo = true;
@@ -671,17 +672,17 @@ __global__ __launch_bounds__(64 * RS_ROWS) void k_resist(Geo g, Box b, int tiles
         double nbx = bx[c], nby = by[c], nbz = bz[c];
         if (upd && j >= 1 && k >= 1) {
           const double area = g.dyb[j] * g.dzb[k];
-          nbx = nbx + ((double)p.kz0 - p.kzm + m.kz0 - m.kzm - p.ky0 + m.ky0 - p.kym + m.kym) * dt / area;
+          nbx = nbx + ((double)p.kz0 - p.kzm + m.kz0 - m.kzm - p.ky0 + m.ky0 - p.kym + m.kym) * dt / recip(area);
         }
         if (upd && i >= 1 && k >= 1) {
           const double area = g.dxb[i] * g.dzb[k];
-          nby = nby + ((double)p.kx0 - m.kx0 + p.kxm - m.kxm - p.kz0 + p.kzx - m.kz0 + m.kzx) * dt / area;
+          nby = nby + ((double)p.kx0 - m.kx0 + p.kxm - m.kxm - p.kz0 + p.kzx - m.kz0 + m.kzx) * dt / recip(area);
         }
         if (upd && i >= 1 && j >= 1) {
           const double area = g.dxb[i] * g.dyb[j];
           nbz = nbz + ((double)p.ky0 - s[1][w][l - 1] + p.kym - s[1][w - 1][l - 1] - p.kx0 + s[0][w - 1][l] - p.kxm +
                        s[0][w - 1][l - 1]) *
-                          dt / area;
+                          dt / recip(area);
         }
         bxo[c] = nbx;
         byo[c] = nby;
@@ -693,7 +694,7 @@ __global__ __launch_bounds__(64 * RS_ROWS) void k_resist(Geo g, Box b, int tiles
         if (hij && k >= 1 && k <= g.nz) {
           // curlb(c) + (c-X) + (c-Y) + (c-X-Y) + (c-Z) + (c-X-Z) + (c-Y-Z) + (c-X-Y-Z)
           const acc sq = pq[0] + pq[1] + pq[2] + pq[3] + mq[0] + mq[1] + mq[2] + mq[3];
-          const acc lh = sq * (acc)dt / ((acc)8.0 * rho[c]);
+          const acc lh = sq * (acc)dt / recip((acc)8.0 * rho[c]);
           ohmic_dep[c] = ohmic_dep[c] + lh;
           e = e + lh;
         }
@@ -741,8 +742,8 @@ __global__ __launch_bounds__(BX * BY) void k_rk4_emf(Geo g, Box b, const double 
   const int c = g.idx(i, j, kk);
   const BPlane lo = bplane(bx, by, c, Y), hi = bplane(bx, by, c + Z, Y);
   acc jx, jy, jz;
-  vertex_current_acc<acc>(g.dxc[i], g.dyc[j], g.dzc[kk], lo, hi, bz[c], bz[c + 1], bz[c + Y], bz[c + 1 + Y], jx, jy,
-                          jz);
+  vertex_current_acc(recip((acc)g.dxc[i]), recip((acc)g.dyc[j]), recip((acc)g.dzc[kk]), lo, hi, bz[c], bz[c + 1],
+                     bz[c + Y], bz[c + 1 + Y], jx, jy, jz);
   const acc e = eta[c];
   real v[4];
   if constexpr (COWL) {
@@ -1003,9 +1004,12 @@ __global__ __launch_bounds__(BX * BY) void k_force(Geo g, Box b, const real *__r
   if (CAUCHY) clo = cplane(cv1, b1x, b1y, b1z, cb, Y);
   else blo = bplane(bx, by, cb, Y);
   real a3lo = al3[cb];
+  const acc dxc = (acc)g.dxc[i], dyc = (acc)g.dyc[j];
+  const Recip<acc> rx = recip(dxc), ry = recip(dyc);
   for (int k = k0; k <= k1; ++k) {
     const int c = g.idx(i, j, k);
-    const acc dxc = (acc)g.dxc[i], dyc = (acc)g.dyc[j], dzc = (acc)g.dzc[k];
+    const acc dzc = (acc)g.dzc[k];
+    const Recip<acc> rz = recip(dzc);
     real up[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) up[q] = V[q][c + Z];
@@ -1022,7 +1026,7 @@ __global__ __launch_bounds__(BX * BY) void k_force(Geo g, Box b, const real *__r
     const acc a4 = al2[c + Y + Z] * dxc * dzc;
     const acc a5 = a3lo * dxc * dyc;
     const acc a6 = a3hi * dxc * dyc;
-    const acc cvv = (acc)0.125 * (acc)cv_sum8(g, i, j, k);
+    const Recip<acc> cvv = recip((acc)0.125 * (acc)cv_sum8(g, i, j, k));
     acc fv[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
@@ -1037,13 +1041,13 @@ __global__ __launch_bounds__(BX * BY) void k_force(Geo g, Box b, const real *__r
     const acc ppxy = plo.pxy, ppxz = phi.px, ppyz = phi.py, ppxyz = phi.pxy;
     acc w1 = (p + ppy + ppz + ppyz) * q4;
     acc w2 = (ppx + ppxy + ppxz + ppxyz) * q4;
-    acc fx = -(w2 - w1) / dxc;
+    acc fx = -(w2 - w1) / rx;
     w1 = (p + ppx + ppz + ppxz) * q4;
     w2 = (ppy + ppxy + ppyz + ppxyz) * q4;
-    acc fy = -(w2 - w1) / dyc;
+    acc fy = -(w2 - w1) / ry;
     w1 = (p + ppx + ppy + ppxy) * q4;
     w2 = (ppz + ppxz + ppyz + ppxyz) * q4;
-    acc fz = -(w2 - w1) / dzc;
+    acc fz = -(w2 - w1) / rz;
     acc bxv, byv, bzv, jx, jy, jz;
     if (CAUCHY) {
       cauchy_jb(dxc, dyc, dzc, clo, chi, jx, jy, jz, bxv, byv, bzv);
@@ -1054,7 +1058,7 @@ __global__ __launch_bounds__(BX * BY) void k_force(Geo g, Box b, const real *__r
       bxv = 0.25 * (blo.bx0 + blo.bxy + bhi.bx0 + bhi.bxy);
       byv = 0.25 * (blo.by0 + blo.byx + bhi.by0 + bhi.byx);
       bzv = 0.25 * (bz0 + bzy + bzx + bzxy);
-      vertex_current_acc<acc>(g.dxc[i], g.dyc[j], g.dzc[k], blo, bhi, bz0, bzx, bzy, bzxy, jx, jy, jz);
+      vertex_current_acc(rx, ry, rz, blo, bhi, bz0, bzx, bzy, bzxy, jx, jy, jz);
     }
     const acc g_b = gb ? (acc)gb[c] : (acc)1.0;
     fx = fx + g_b * (jy * bzv - jz * byv);
@@ -1063,9 +1067,10 @@ __global__ __launch_bounds__(BX * BY) void k_force(Geo g, Box b, const real *__r
     const acc rv = rho_v[c];
     fz = fz - rv * (acc)g.grav[k];
     const acc h = (acc)dt2;
-    vx1[c] = u0[0] + h * (fv[0] + fx) / rv;
-    vy1[c] = u0[1] + h * (fv[1] + fy) / rv;
-    vz1[c] = u0[2] + h * (fv[2] + fz) / rv;
+    const Recip<acc> rrv = recip(rv);
+    vx1[c] = u0[0] + h * (fv[0] + fx) / rrv;
+    vy1[c] = u0[1] + h * (fv[1] + fy) / rrv;
+    vz1[c] = u0[2] + h * (fv[2] + fz) / rrv;
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
       um[q] = u0[q];
@@ -1103,6 +1108,7 @@ __global__ __launch_bounds__(BX * BY) void k_shock_corr(Geo g, Box b, const real
   if (j <= b.y1) {
     const int Y = g.sy, Z = g.sz;
     const bool column = i >= 1 && j >= 1;
+    const Recip<acc> rx = recip((acc)g.dxb[i]), ry = recip((acc)g.dyb[j]);
     const int cb = g.idx(i, j, k0) - Z;
     Node4 lx = node4(vx, cb, Y), ly = node4(vy, cb, Y), lz = node4(vz, cb, Y);
     Node4 lx1 = node4(vx1, cb, Y), ly1 = node4(vy1, cb, Y), lz1 = node4(vz1, cb, Y);
@@ -1134,11 +1140,11 @@ __global__ __launch_bounds__(BX * BY) void k_shock_corr(Geo g, Box b, const real
         const acc vzbm = (lz1.c + lz1.d + lz1.b + lz1.a) * q4;
         const acc dta = (acc)dt;
         const acc dv =
-            ((vxb - vxbm) / (acc)g.dxb[i] + (vyb - vybm) / (acc)g.dyb[j] + (vzb - vzbm) / (acc)g.dzb[k]) * dta;
+            ((vxb - vxbm) / rx + (vyb - vybm) / ry + (vzb - vzbm) / recip((acc)g.dzb[k])) * dta;
         const acc r = rho[c];
-        const real e1 = energy[c] + (dta * vh - dv * pp[c]) / r;
+        const real e1 = energy[c] + (dta * vh - dv * pp[c]) / recip(r);
         visc_dep[c] = visc_dep[c] + dta * vh;
-        const real rn = r / ((acc)1.0 + dv);
+        const real rn = r / recip((acc)1.0 + dv);
         rho[c] = rn;
         if (COOL) {
           // a running average of the viscous heating is removed again, and

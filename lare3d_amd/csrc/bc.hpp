@@ -68,18 +68,23 @@ __device__ __forceinline__ HaloMap halo_map(int c, int n, int periodic, int open
 }
 
 // Fields of one fill: the face field (NB = 1: b[0..2]), NC cell fields and
-// NN node fields (0 or 3).
+// NN node fields (0, 3 or 6).
 struct HaloSet {
   double *b[3];
   real *cell[2];
-  real *node[3];
+  real *node[6];
 };
 
 // One thread per point of the shell: the z layers over the whole (x, y)
 // extent, the y layers over k = 1..n-1, the x layers over j, k = 1..n-1.  All
-// loads of a point are issued before its stores.
+// loads of a point are issued before its stores.  One block more folds the
+// heating total of the kernel before the fill, if there is one to fold.
 template <int NB, int NC, int NN>
-__global__ __launch_bounds__(256) void k_halo(Geo g, HaloSet s) {
+__global__ __launch_bounds__(256) void k_halo(Geo g, HaloSet s, FoldJob job) {
+  if (job.rows && blockIdx.x + 1 == gridDim.x) {
+    fold_rows(job.rows, 0, job.nrows, 1, 0, job.out, 1, job.host);
+    return;
+  }
   const unsigned t = blockIdx.x * 256u + threadIdx.x;
   const unsigned wx = (unsigned)g.nx + 5u, wy = (unsigned)g.ny + 5u;
   const unsigned my = (unsigned)g.ny - 1u, mz = (unsigned)g.nz - 1u;
@@ -112,7 +117,7 @@ __global__ __launch_bounds__(256) void k_halo(Geo g, HaloSet s) {
             sz = g.idx(mx.cell, my_.cell, mz_.face), sc = g.idx(mx.cell, my_.cell, mz_.cell),
             sn = g.idx(mx.node, my_.node, mz_.node);
   double vb[3] = {0.0, 0.0, 0.0};
-  real vc[2] = {0, 0}, vn[3] = {0, 0, 0};
+  real vc[2] = {0, 0}, vn[6] = {0, 0, 0, 0, 0, 0};
   if constexpr (NB) {
     vb[0] = s.b[0][sx];
     vb[1] = s.b[1][sy];

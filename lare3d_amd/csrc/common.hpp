@@ -207,6 +207,44 @@ __device__ __forceinline__ void block_reduce_store(double (&v)[NV], const int *o
   }
 }
 
+// One block of 256 threads folds rows r0 .. r1-1 of nv values (bit q of
+// minmask selects min, else sum) and stores (or adds) the nv results, in out
+// and, if given, in the pinned host mirror.
+#define RED_MAXV 4
+__device__ __forceinline__ void fold_rows(const double *__restrict__ rows, int r0, int r1, int nv, int minmask,
+                                          double *__restrict__ out, int accumulate, double *__restrict__ host = nullptr) {
+  __shared__ double red[4][RED_MAXV];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int q = 0; q < nv; ++q) {
+    const bool isMin = (minmask >> q) & 1;
+    double v = isMin ? 1.7976931348623157e+308 : 0.0;
+    for (int r = r0 + (int)threadIdx.x; r < r1; r += 256) {
+      const double x = rows[(size_t)r * nv + q];
+      v = isMin ? dmin(v, x) : v + x;
+    }
+    v = isMin ? wave_min(v) : wave_sum(v);
+    if (lane == 0) red[wave][q] = v;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < nv) {
+    const int q = threadIdx.x;
+    const bool isMin = (minmask >> q) & 1;
+    double r = red[0][q];
+    for (int w = 1; w < 4; ++w) r = isMin ? dmin(r, red[w][q]) : r + red[w][q];
+    if (accumulate) r = out[q] + r;
+    out[q] = r;
+    if (host) host[q] = r;
+  }
+}
+
+// A sum of one value per row that a launch folds beside its own work, in a
+// block of its own (rows NULL: none).
+struct FoldJob {
+  const double *rows;
+  int nrows;
+  double *out, *host;
+};
+
 // Columns of a z-marching launch: thread (i, j) of the flattened plane tile
 // blockIdx.x walks planes k0 .. k1 of its chunk (b.zc planes per block).
 #define ZRANGE(b, k0, k1)                                             \

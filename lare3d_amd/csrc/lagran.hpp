@@ -637,7 +637,7 @@ __global__ __launch_bounds__(64 * RS_ROWS, RS_WAVES) void k_resist(Geo g, Box b,
       lo = hi;
       have_lo = true;
       const real es = sqrt(jx * jx + jy * jy + jz * jz) > (acc)j_max ? eta_bg + eta0 : eta_bg;
-      if (out && k >= k0) eta[c] = es;
+      if (out && k >= k0 && eta) eta[c] = es;
       if (kij && k >= 0 && k <= g.nz) {
         const acc e = es;
         acc cb;
@@ -862,7 +862,7 @@ __global__ __launch_bounds__(BX * BY) void k_cauchy_b(Geo g, Box b, const real *
                                                       const real *__restrict__ rho,
                                                       const real *__restrict__ visc_heat,
                                                       const real *__restrict__ p0, real *__restrict__ pp,
-                                                      double gamma, double dt2, EosArgs eq) {
+                                                      double gamma, double dt2, EosArgs eq, bool clamp) {
   BOX_INDEX(b, i, j, k);
   const int X = 1, Y = g.sy, Z = g.sz;
   const int c = g.idx(i, j, k);
@@ -917,7 +917,7 @@ __global__ __launch_bounds__(BX * BY) void k_cauchy_b(Geo g, Box b, const real *
     // predictor energy and pressure (lagran.F90:234-249)
     const acc r = rho[c];
     const acc dvv = c1 / cv - (acc)1.0;
-    acc e1 = energy[c] - p0[c] * dvv / r;
+    acc e1 = (clamp ? max0((acc)energy[c]) : (acc)energy[c]) - p0[c] * dvv / r;
     e1 = e1 + visc_heat[c] * h / r;
     const acc ei = eq.xi ? eos_e<true>(e1, eq, c) : eos_e<false>(e1, eq, c);
     pp[c] = ei * ((acc)gamma - (acc)1.0) * r * cv / c1;
@@ -975,6 +975,31 @@ __device__ __forceinline__ void cauchy_jb(acc dxc, acc dyc, acc dzc, const CPlan
   bzv = (lo.z[0] + lo.z[1] + lo.z[2] + lo.z[3] + hi.z[0] + hi.z[1] + hi.z[2] + hi.z[3]) / (cvx + cvxp);
 }
 
+// Stores a node's three values at (i, j, k) of 0..n as remap_v_bcs leaves the
+// nodes 0..n (no BC_OPEN side): zero on the nodes of a wall; on a periodic
+// axis node n takes node 0's values, stored by that node's thread.
+__device__ __forceinline__ void store_node3(const Geo &g, int c, int i, int j, int k, real x, real y, real z,
+                                            real *__restrict__ ox, real *__restrict__ oy, real *__restrict__ oz) {
+  const bool ei = i == 0 || i == g.nx, ej = j == 0 || j == g.ny, ek = k == 0 || k == g.nz;
+  if (!(ei || ej || ek)) {
+    ox[c] = x;
+    oy[c] = y;
+    oz[c] = z;
+    return;
+  }
+  if ((g.per[0] && i == g.nx) || (g.per[1] && j == g.ny) || (g.per[2] && k == g.nz)) return;
+  if ((g.user[0] && ei) || (g.user[1] && ej) || (g.user[2] && ek)) x = y = z = 0;
+  const int di = g.per[0] && ei ? g.nx : 0, dj = g.per[1] && ej ? g.ny * g.sy : 0,
+            dk = g.per[2] && ek ? g.nz * g.sz : 0;
+  for (int q = 0; q < 8; ++q) {
+    if (((q & 1) && !di) || ((q & 2) && !dj) || ((q & 4) && !dk)) continue;
+    const int o = c + ((q & 1) ? di : 0) + ((q & 2) ? dj : 0) + ((q & 4) ? dk : 0);
+    ox[o] = x;
+    oy[o] = y;
+    oz[o] = z;
+  }
+}
+
 // predictor momentum (lagran.F90:251-387) with fx/fy/fz_visc (:745-789)
 // recomputed here from alpha and v.  Without CAUCHY, B is the half-step
 // (predictor-remapped) face field; with CAUCHY, J and B come from the
@@ -987,7 +1012,7 @@ __global__ __launch_bounds__(BX * BY) void k_force(Geo g, Box b, const real *__r
                         const real *__restrict__ al2, const real *__restrict__ al3, const real *__restrict__ gb,
                         real *__restrict__ vx1, real *__restrict__ vy1, real *__restrict__ vz1, double dt2,
                         const real *__restrict__ cv1, const real *__restrict__ b1x, const real *__restrict__ b1y,
-                        const real *__restrict__ b1z) {
+                        const real *__restrict__ b1z, int wall) {
   // gb: gamma_boris of this step's set_dt (lagran.F90:375-377), NULL for 1
   ZCOLUMN(b, i, j, k0, k1);
   const int X = 1, Y = g.sy, Z = g.sz;
@@ -1071,9 +1096,15 @@ __global__ __launch_bounds__(BX * BY) void k_force(Geo g, Box b, const real *__r
     fz = fz - rv * (acc)g.grav[k];
     const acc h = (acc)dt2;
     const Recip<acc> rrv = recip(rv);
-    vx1[c] = u0[0] + h * (fv[0] + fx) / rrv;
-    vy1[c] = u0[1] + h * (fv[1] + fy) / rrv;
-    vz1[c] = u0[2] + h * (fv[2] + fz) / rrv;
+    const real w1x = u0[0] + h * (fv[0] + fx) / rrv, w1y = u0[1] + h * (fv[1] + fy) / rrv,
+               w1z = u0[2] + h * (fv[2] + fz) / rrv;
+    if (wall) {
+      store_node3(g, c, i, j, k, w1x, w1y, w1z, vx1, vy1, vz1);
+    } else {
+      vx1[c] = w1x;
+      vy1[c] = w1y;
+      vz1[c] = w1z;
+    }
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
       um[q] = u0[q];
@@ -1099,7 +1130,7 @@ __global__ __launch_bounds__(BX * BY) void k_shock_corr(Geo g, Box b, const real
                              const real *__restrict__ al3, const real *__restrict__ pp,
                              real *__restrict__ energy, real *__restrict__ rho, real *__restrict__ visc_dep,
                              real *__restrict__ vxo, real *__restrict__ vyo, real *__restrict__ vzo,
-                             real *__restrict__ cool_v, double alpha_av, double *__restrict__ partial, double dt) {
+                             real *__restrict__ cool_v, double alpha_av, double *__restrict__ partial, double dt, bool clamp) {
   // cool_v: cool_term_v of the cooling_term (lagran.F90:464-476), unused
   // without COOL
   // marching in z: the node values (v, v1) and al1/al2 of plane k are reused
@@ -1145,7 +1176,8 @@ __global__ __launch_bounds__(BX * BY) void k_shock_corr(Geo g, Box b, const real
         const acc dv =
             ((vxb - vxbm) / rx + (vyb - vybm) / ry + (vzb - vzbm) / recip((acc)g.dzb[k])) * dta;
         const acc r = rho[c];
-        const real e1 = energy[c] + (dta * vh - dv * pp[c]) / recip(r);
+        const acc e0 = clamp ? max0((acc)energy[c]) : (acc)energy[c];
+        const real e1 = e0 + (dta * vh - dv * pp[c]) / recip(r);
         visc_dep[c] = visc_dep[c] + dta * vh;
         const real rn = r / recip((acc)1.0 + dv);
         rho[c] = rn;

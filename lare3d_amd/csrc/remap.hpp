@@ -65,6 +65,7 @@ struct PredP {
   real *pp;
   double gamma, dt2;
   EosArgs eq;  // partially ionised pressure when eq.xi is set
+  bool clamp;  // take MAX(energy, 0) (lagran.F90:180-181)
 };
 
 // Face-averaged velocities at the two faces of a cell along each axis, from
@@ -118,7 +119,7 @@ __global__ __launch_bounds__(BX * BY) void k_geom_pred(Geo g, Box b, const real 
       // predictor energy and pressure (lagran.F90:234-249)
       const acc r = pr.rho[c];
       const acc dv = c1 / cv - (acc)1.0;
-      acc e1 = pr.energy[c] - pr.p0[c] * dv / r;
+      acc e1 = (pr.clamp ? max0((acc)pr.energy[c]) : (acc)pr.energy[c]) - pr.p0[c] * dv / r;
       e1 = e1 + pr.visc_heat[c] * (acc)pr.dt2 / r;
       const acc ei = pr.eq.xi ? eos_e<true>(e1, pr.eq, c) : eos_e<false>(e1, pr.eq, c);
       pr.pp[c] = ei * ((acc)pr.gamma - (acc)1.0) * r * cv / c1;

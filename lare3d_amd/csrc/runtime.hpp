@@ -44,6 +44,7 @@ struct Dev {
   int bc[6];
   int per[3], user[3];
   bool any_open = false;  // some side is BC_OPEN
+  bool clamp = false;     // predictor and corrector of this step clamp the energy they read
   lare_params p;
   double tfac, visc2_norm;
   hipStream_t stream = nullptr;
@@ -208,33 +209,6 @@ dim3 grid_from0(int x1, int y1, int z1) { return box_grid(mkbox(0, x1, 0, y1, 0,
 // us at any size, and is one or two.
 #define RED_ROWS 512
 #define RED_DIRECT 1024
-#define RED_MAXV 4
-
-__device__ __forceinline__ void fold_rows(const double *__restrict__ rows, int r0, int r1, int nv, int minmask,
-                                          double *__restrict__ out, int accumulate, double *__restrict__ host = nullptr) {
-  __shared__ double red[4][RED_MAXV];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int q = 0; q < nv; ++q) {
-    const bool isMin = (minmask >> q) & 1;
-    double v = isMin ? 1.7976931348623157e+308 : 0.0;
-    for (int r = r0 + (int)threadIdx.x; r < r1; r += 256) {
-      const double x = rows[(size_t)r * nv + q];
-      v = isMin ? dmin(v, x) : v + x;
-    }
-    v = isMin ? wave_min(v) : wave_sum(v);
-    if (lane == 0) red[wave][q] = v;
-  }
-  __syncthreads();
-  if ((int)threadIdx.x < nv) {
-    const int q = threadIdx.x;
-    const bool isMin = (minmask >> q) & 1;
-    double r = red[0][q];
-    for (int w = 1; w < 4; ++w) r = isMin ? dmin(r, red[w][q]) : r + red[w][q];
-    if (accumulate) r = out[q] + r;
-    out[q] = r;
-    if (host) host[q] = r;
-  }
-}
 
 __global__ __launch_bounds__(256) void k_reduce_rows(const double *__restrict__ partial, int nrows, int nv, int minmask,
                                                      int chunk, double *__restrict__ level1) {
@@ -275,6 +249,22 @@ int final_reduce(dim3 grid, int nv, int minmask, int slot, int accumulate) {
   return 0;
 }
 
+// the fold of one accumulated sum as a job for the launch that follows: the
+// level-1 rows are formed here if there are many
+int fold_job(dim3 grid, int slot, FoldJob *job) {
+  const int nb = (int)(grid.x * grid.y * grid.z);
+  if ((size_t)nb > S.partial_cap) return fail(LARE_E_ARG, "reduction of %d values exceeds the partial buffer", nb);
+  job->rows = S.partial;
+  if (const int chunk = fold_chunk(nb, &job->nrows)) {
+    double *level1 = S.partial + S.partial_cap;
+    LAUNCH("reduce_rows", k_reduce_rows, dim3(job->nrows), dim3(256), S.partial, nb, 1, 0, chunk, level1);
+    job->rows = level1;
+  }
+  job->out = S.dscal + slot;
+  job->host = S.hscal + slot;
+  return 0;
+}
+
 int read_scalars(int slot, int count, double *out) {
   HIPCHK(hipStreamSynchronize(S.stream));
   for (int q = 0; q < count; ++q) out[q] = ((volatile double *)S.hscal)[slot + q];
@@ -288,23 +278,29 @@ enum FieldKind { FK_CELL, FK_NODE, FK_BX, FK_BY, FK_BZ };
 
 // the fields of h that NB, NC and NN say, every axis at once
 template <int NB, int NC, int NN>
-int fill_halo(const HaloSet &h, const char *name) {
-  LAUNCH(name, (k_halo<NB, NC, NN>), dim3(halo_blocks(S.g)), dim3(256), S.g, h);
+int fill_halo(const HaloSet &h, const char *name, const FoldJob &job = FoldJob{}) {
+  LAUNCH(name, (k_halo<NB, NC, NN>), dim3(halo_blocks(S.g) + (job.rows ? 1 : 0)), dim3(256), S.g, h, job);
   return 0;
 }
 
-int bfield_bcs(double *bx, double *by, double *bz) {
-  return fill_halo<1, 0, 0>({{bx, by, bz}, {nullptr, nullptr}, {nullptr, nullptr, nullptr}}, "bc_bfield");
-}
-int energy_bcs() {
-  return fill_halo<0, 1, 0>({{nullptr, nullptr, nullptr}, {S.energy, nullptr}, {nullptr, nullptr, nullptr}},
-                            "bc_energy");
-}
-int node_bcs(real *ux, real *uy, real *uz, const char *name) {
-  return fill_halo<0, 0, 3>({{nullptr, nullptr, nullptr}, {nullptr, nullptr}, {ux, uy, uz}}, name);
-}
+// the state's fields, with v1 after v
 HaloSet state_halo() {
-  return {{S.bx, S.by, S.bz}, {S.energy, S.rho}, {S.vx, S.vy, S.vz}};
+  return {{S.bx, S.by, S.bz}, {S.energy, S.rho}, {S.vx, S.vy, S.vz, S.vx1, S.vy1, S.vz1}};
+}
+int bfield_bcs(double *bx, double *by, double *bz) {
+  HaloSet h = state_halo();
+  h.b[0] = bx;
+  h.b[1] = by;
+  h.b[2] = bz;
+  return fill_halo<1, 0, 0>(h, "bc_bfield");
+}
+int energy_bcs() { return fill_halo<0, 1, 0>(state_halo(), "bc_energy"); }
+int node_bcs(real *ux, real *uy, real *uz, const char *name) {
+  HaloSet h = state_halo();
+  h.node[0] = ux;
+  h.node[1] = uy;
+  h.node[2] = uz;
+  return fill_halo<0, 0, 3>(h, name);
 }
 int boundary_conditions() { return fill_halo<1, 2, 3>(state_halo(), "bc_all"); }
 
@@ -533,7 +529,7 @@ real *pred_db1(int ax) { return ax == 0 ? S.db1 : (ax == 1 ? S.cv1 : S.cv2); }
 // the geometry of a predictor remap whose last sweep is along `last`, and the
 // predictor pressure
 int geom_predictor(int last, double dt) {
-  const PredP pr = {S.energy, S.rho, S.visc_heat, S.p0, S.pp, S.p.gamma, S.dt2, eos_args()};
+  const PredP pr = {S.energy, S.rho, S.visc_heat, S.p0, S.pp, S.p.gamma, S.dt2, eos_args(), S.clamp};
   const Box cb = marched(cell_box());
 #define GEOM_PRED(L)                                                                                                 \
   LAUNCH("geom", k_geom_pred<L>, zchunk_grid(cb), box_block(), S.g, cb, S.vx, S.vy, S.vz, pred_db1(0), pred_db1(1), \
@@ -995,15 +991,18 @@ int lagrangian_step() {
         if (rc) return rc;
         continue;
       }
+      // the eta of a substep is read within it; the last one's is kept
+      real *const eta_out = sc == substeps ? S.eta : nullptr;
       if (S.eta_perp)
         LAUNCH("resist", k_resist<true>, g2, dim3(64, RS_ROWS, 1), S.g, fb, tiles_x, S.bx, S.by, S.bz, S.fxr, S.fyr,
-               S.fzr, S.eta, S.energy, S.ohmic_dep, S.rho, S.curlb, S.partial, S.dt, S.p.eta_background, S.p.eta0,
+               S.fzr, eta_out, S.energy, S.ohmic_dep, S.rho, S.curlb, S.partial, S.dt, S.p.eta_background, S.p.eta0,
                S.p.j_max, S.eta_perp);
       else
         LAUNCH("resist", k_resist<false>, g2, dim3(64, RS_ROWS, 1), S.g, fb, tiles_x, S.bx, S.by, S.bz, S.fxr, S.fyr,
-               S.fzr, S.eta, S.energy, S.ohmic_dep, S.rho, S.curlb, S.partial, S.dt, S.p.eta_background, S.p.eta0,
+               S.fzr, eta_out, S.energy, S.ohmic_dep, S.rho, S.curlb, S.partial, S.dt, S.p.eta_background, S.p.eta0,
                S.p.j_max, S.eta_perp);
-      rc = final_reduce(g2, 1, 0, 9, 1);
+      FoldJob job = {};
+      rc = fold_job(g2, 9, &job);
       if (rc) return rc;
       if (S.curlb)
         LAUNCH_BOX("cool_b", k_cool_b, interior(), S.curlb, S.rho, S.cool_b, S.energy, S.p.alpha_av, S.dt);
@@ -1011,7 +1010,7 @@ int lagrangian_step() {
       tb = S.bx; S.bx = S.fxr; S.fxr = tb;
       tb = S.by; S.by = S.fyr; S.fyr = tb;
       tb = S.bz; S.bz = S.fzr; S.fzr = tb;
-      rc = fill_halo<1, 1, 0>(state_halo(), "bc_resistive");
+      rc = fill_halo<1, 1, 0>(state_halo(), "bc_resistive", job);
       if (rc) return rc;
     }
     S.dt = actual_dt;
@@ -1027,25 +1026,33 @@ int lagrangian_step() {
       rc = heat_conduct_sts2(1);
       if (rc) return rc;
     }
-  } else if (!S.p.resistive_mhd || S.p.fourth_order) {
-    // energy = MAX(energy0 + 0, 0) (lagran.F90:180-181).  After a
-    // first-order resistive step it changes nothing: the last substep's ohmic
-    // heating already clamped the whole cell box (:1305) and energy_bcs only
-    // copies clamped values, so the launch is left out then.
-    LAUNCH_BOX("energy_max", k_energy_max, cell_box(), S.energy);
   }
+  // Without conduction, energy = MAX(energy0 + 0, 0) (lagran.F90:180-181).
+  // After a first-order resistive step it changes nothing: the last substep's
+  // ohmic heating already clamped the whole cell box (:1305) and energy_bcs
+  // only copies clamped values.  Otherwise its two readers, the predictor and
+  // the corrector, clamp what they read, and the fill after the corrector
+  // writes the ghosts anew; a BC_OPEN side's ghosts are not written again, so
+  // then the array itself is clamped.
+  const bool clamp = !S.p.conduction && (!S.p.resistive_mhd || S.p.fourth_order);
+  if (clamp && S.any_open) LAUNCH_BOX("energy_max", k_energy_max, cell_box(), S.energy);
+  S.clamp = clamp && !S.any_open;
 
   // predictor-corrector (lagran.F90:208-478)
   const Box nb = marched(nodes0n());
+  // k_force gives the nodes 0..n of v1 what remap_v_bcs gives them, the only
+  // ones that the corrector reads; the ghosts follow in its fill.  With a
+  // BC_OPEN side remap_v_bcs comes at once, before v's ghosts are copied.
+  const int wall = S.any_open ? 0 : 1;
   if (S.p.cauchy) {
     // the Cauchy solution for the cell-centred B1 (B1 cv1 in the spare
     // predictor-B arrays), cv1 and the predictor pressure; no predictor remap
     real *b1[3] = {(real *)S.bpx, (real *)S.bpy, (real *)S.bpz};
     LAUNCH_BOX("cauchy_b", k_cauchy_b, cell_box(), S.vx, S.vy, S.vz, S.bx, S.by, S.bz, S.cv1, b1[0], b1[1], b1[2],
-               S.energy, S.rho, S.visc_heat, S.p0, S.pp, S.p.gamma, S.dt2, eos_args());
+               S.energy, S.rho, S.visc_heat, S.p0, S.pp, S.p.gamma, S.dt2, eos_args(), S.clamp);
     LAUNCH("force", k_force<true>, zchunk_grid(nb), box_block(), S.g, nb, S.vx, S.vy, S.vz, S.pp,
            S.bx, S.by, S.bz, S.rho_v, S.al1, S.al2, S.al3, S.gamma_boris, S.vx1, S.vy1, S.vz1, S.dt2, S.cv1, b1[0],
-           b1[1], b1[2]);
+           b1[1], b1[2], wall);
   } else {
     const double dt_full = S.dt;
     S.dt = 0.5 * dt_full;
@@ -1056,11 +1063,11 @@ int lagrangian_step() {
     // remap's last geometry pass
     LAUNCH("force", k_force<false>, zchunk_grid(nb), box_block(), S.g, nb, S.vx, S.vy, S.vz, S.pp,
            S.bpx, S.bpy, S.bpz, S.rho_v, S.al1, S.al2, S.al3, S.gamma_boris, S.vx1, S.vy1, S.vz1, S.dt2, S.cv1,
-           nullptr, nullptr, nullptr);
+           nullptr, nullptr, nullptr, wall);
   }
-  rc = node_bcs(S.vx1, S.vy1, S.vz1, "bc_v1");
-  if (rc) return rc;
   if (S.any_open) {
+    rc = node_bcs(S.vx1, S.vy1, S.vz1, "bc_v1");
+    if (rc) return rc;
     // v1 = v over the whole array before the predictor remap
     // (lagran.F90:1051-1053); the forces then set nodes 0..n and
     // remap_v_bcs the filled sides, so a BC_OPEN side keeps v's ghosts
@@ -1076,12 +1083,13 @@ int lagrangian_step() {
   if (S.cool_v)
     LAUNCH("shock_corr", k_shock_corr<true>, g3, box_block(), S.g, nb, S.vx, S.vy, S.vz, S.vx1, S.vy1, S.vz1,
            S.al1, S.al2, S.al3, S.pp, S.energy, S.rho, S.visc_dep, S.Fx, S.Fy, S.Fz, S.cool_v, S.p.alpha_av,
-           S.partial, S.dt);
+           S.partial, S.dt, S.clamp);
   else
     LAUNCH("shock_corr", k_shock_corr<false>, g3, box_block(), S.g, nb, S.vx, S.vy, S.vz, S.vx1, S.vy1, S.vz1,
            S.al1, S.al2, S.al3, S.pp, S.energy, S.rho, S.visc_dep, S.Fx, S.Fy, S.Fz, S.cool_v, S.p.alpha_av,
-           S.partial, S.dt);
-  rc = final_reduce(g3, 1, 0, 8, 1);
+           S.partial, S.dt, S.clamp);
+  FoldJob job = {};
+  rc = fold_job(g3, 8, &job);
   if (rc) return rc;
   // the new velocities went to the momentum-flux arrays, which swap roles
   // with the velocity arrays; the boundary fill below sets their ghosts
@@ -1103,9 +1111,9 @@ int lagrangian_step() {
     if (rc) return rc;
     rc = open_bcs();
     if (rc) return rc;
-    return fill_halo<0, 2, 0>(state_halo(), "bc_lagrangian");
+    return fill_halo<0, 2, 0>(state_halo(), "bc_lagrangian", job);
   }
-  return fill_halo<0, 2, 3>(state_halo(), "bc_lagrangian");
+  return fill_halo<0, 2, 6>(state_halo(), "bc_lagrangian", job);
 }
 
 // ----------------------------------------------------------------------------

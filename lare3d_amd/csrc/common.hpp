@@ -209,10 +209,14 @@ __device__ __forceinline__ void block_reduce_store(double (&v)[NV], const int *o
 
 // One block of 256 threads folds rows r0 .. r1-1 of nv values (bit q of
 // minmask selects min, else sum) and stores (or adds) the nv results, in out
-// and, if given, in the pinned host mirror.
+// and, if given, in the pinned host mirror, whose ticket word it then sets.
 #define RED_MAXV 4
+struct HostOut {
+  double *v;
+  unsigned long long *ticket, number;
+};
 __device__ __forceinline__ void fold_rows(const double *__restrict__ rows, int r0, int r1, int nv, int minmask,
-                                          double *__restrict__ out, int accumulate, double *__restrict__ host = nullptr) {
+                                          double *__restrict__ out, int accumulate, const HostOut &host = HostOut{}) {
   __shared__ double red[4][RED_MAXV];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int q = 0; q < nv; ++q) {
@@ -233,7 +237,15 @@ __device__ __forceinline__ void fold_rows(const double *__restrict__ rows, int r
     for (int w = 1; w < 4; ++w) r = isMin ? dmin(r, red[w][q]) : r + red[w][q];
     if (accumulate) r = out[q] + r;
     out[q] = r;
-    if (host) host[q] = r;
+    if (host.v) {
+      ((volatile double *)host.v)[q] = r;
+      __threadfence_system();
+    }
+  }
+  if (host.v) {
+    // the values (one wave's stores) reach the host before the ticket
+    __syncthreads();
+    if (threadIdx.x == 0) *(volatile unsigned long long *)host.ticket = host.number;
   }
 }
 
@@ -242,7 +254,8 @@ __device__ __forceinline__ void fold_rows(const double *__restrict__ rows, int r
 struct FoldJob {
   const double *rows;
   int nrows;
-  double *out, *host;
+  double *out;
+  HostOut host;
 };
 
 // Columns of a z-marching launch: thread (i, j) of the flattened plane tile

@@ -138,7 +138,7 @@ int api_energy_account_noalloc(const lare_grid *grid, const lare_fields *f, doub
     HIPCHK(hipGetLastError());
   }
   hipLaunchKernelGGL(fp64::k_final_reduce, dim3(1), dim3(256), 0, 0, chunk ? level1 : partial, rows, nv, minmask, 0, out,
-                     (double *)nullptr);
+                     fp64::HostOut{});
   HIPCHK(hipGetLastError());
   double v[4];
   HIPCHK(hipMemcpy(v, out, sizeof(v), hipMemcpyDeviceToHost));

@@ -133,58 +133,47 @@ __global__ __launch_bounds__(BX * BY) void k_geom_pred(Geo g, Box b, const real 
   }
 }
 
-// Geometry of a full sweep along AX (xremap.f90:57-105 and analogues, from
-// the time-centred velocities).  The node velocities of planes k and k-1 are
-// kept in registers while marching in z.  The pass flags take the axes
-// already swept out of the volumes:
+// Geometry of a full remap (xremap.f90:57-105 and analogues, from the
+// time-centred velocities), all three sweeps in one pass: sweep along A0 first,
+// A1 second, the axis left last.  Nothing here changes during the remap, and
+// the pass flags take the axes already swept out of the volumes:
 //   cv1 = cv (1 + dt (sum over the axes not swept before)),
 //   cv2 = cv (1 + dt (sum over the axes left after this sweep)),
-// and v1 does not change during the remap, so cv1 of a sweep is cv2 of the
-// one before, bit for bit (a flag of 0 adds a zero to the sum, and the sum of
-// two terms does not depend on their order), and cv2 of the last is cv.
-// Only what is new is formed and stored:
-//   REST = 3, first sweep: d?b1, cv1 and cv2;
-//   REST = the axis left, second sweep: d?b1 and cv2;
-//   REST = -1, last sweep: d?b1.
-// The three passes of a remap at 256^3 took 677 us when each formed all
-// three, and 458 us now; the last sweep's readers form cv2 from the widths.
-template <int AX, int REST>
+// so cv1 of a sweep is cv2 of the one before, bit for bit (a flag of 0 adds a
+// zero to the sum, and the sum of two terms does not depend on their order),
+// and cv2 of the last is cv, which its readers form from the widths.  So v1
+// is read once, and the widths of the three axes and three volumes are
+// written: vol0 (cv1 of the first sweep), vol1 (its cv2, cv1 of the second) and
+// vol2 (cv2 of the second, cv1 of the last).  The node velocities of planes
+// k and k-1 are kept in registers while marching in z.  At 256^3, bound by
+// its nine arrays: one pass per sweep that formed and stored all three took
+// 677 us, one per sweep with only what is new 458, this one 367.
+template <int A0, int A1>
 __global__ __launch_bounds__(BX * BY) void k_geom(Geo g, Box b, const real *__restrict__ ux,
                                                   const real *__restrict__ uy, const real *__restrict__ uz,
-                                                  real *__restrict__ cv1, real *__restrict__ cv2,
-                                                  real *__restrict__ db1, double dt) {
+                                                  real *__restrict__ vol0, real *__restrict__ vol1,
+                                                  real *__restrict__ vol2, real *__restrict__ dx1,
+                                                  real *__restrict__ dy1, real *__restrict__ dz1, double dt) {
   ZCOLUMN(b, i, j, k0, k1);
-  constexpr bool NX = REST == 3 || AX == 0 || REST == 0, NY = REST == 3 || AX == 1 || REST == 1,
-                 NZ = REST == 3 || AX == 2 || REST == 2;
+  constexpr int A2 = 3 - A0 - A1;
   const int Y = g.sy;
   const int cb = g.idx(i, j, k0 - 1);
-  Quad lx = {}, ly = {}, lz = {};  // plane k-1
-  if (NX) lx = quad_back(ux, cb, Y);
-  if (NY) ly = quad_back(uy, cb, Y);
-  if (NZ) lz = quad_back(uz, cb, Y);
+  Quad lx = quad_back(ux, cb, Y), ly = quad_back(uy, cb, Y), lz = quad_back(uz, cb, Y);  // plane k-1
   const acc dxb = (acc)g.dxb[i], dyb = (acc)g.dyb[j], tdt = (acc)dt;
   for (int k = k0; k <= k1; ++k) {
     const int c = g.idx(i, j, k);
-    Quad hx = {}, hy = {}, hz = {};  // plane k
-    if (NX) hx = quad_back(ux, c, Y);
-    if (NY) hy = quad_back(uy, c, Y);
-    if (NZ) hz = quad_back(uz, c, Y);
+    const Quad hx = quad_back(ux, c, Y), hy = quad_back(uy, c, Y), hz = quad_back(uz, c, Y);
     const acc dvx = face_diff<0>(hx, lx), dvy = face_diff<1>(hy, ly), dvz = face_diff<2>(hz, lz);
     const acc dzb = (acc)g.dzb[k];
-    if constexpr (REST >= 0) {
-      const acc cv = (acc)g.cv(i, j, k);
-      acc dv2;
-      if constexpr (REST == 3) {
-        const acc tx = dvx / dxb, ty = dvy / dyb, tz = dvz / dzb;
-        const acc two = AX == 0 ? ty + tz : (AX == 1 ? tx + tz : tx + ty);
-        cv1[c] = cv * ((acc)1.0 + (two + (AX == 0 ? tx : (AX == 1 ? ty : tz))) * tdt);
-        dv2 = two * tdt;
-      } else {
-        dv2 = (REST == 0 ? dvx / dxb : (REST == 1 ? dvy / dyb : dvz / dzb)) * tdt;
-      }
-      cv2[c] = cv * ((acc)1.0 + dv2);
-    }
-    db1[c] = AX == 0 ? dxb + dvx * tdt : (AX == 1 ? dyb + dvy * tdt : dzb + dvz * tdt);
+    const acc cv = (acc)g.cv(i, j, k);
+    const acc t[3] = {dvx / dxb, dvy / dyb, dvz / dzb};
+    const acc two = A0 == 0 ? t[1] + t[2] : (A0 == 1 ? t[0] + t[2] : t[0] + t[1]);
+    vol0[c] = cv * ((acc)1.0 + (two + t[A0]) * tdt);
+    vol1[c] = cv * ((acc)1.0 + two * tdt);
+    vol2[c] = cv * ((acc)1.0 + t[A2] * tdt);
+    dx1[c] = dxb + dvx * tdt;
+    dy1[c] = dyb + dvy * tdt;
+    dz1[c] = dzb + dvz * tdt;
     lx = hx;
     ly = hy;
     lz = hz;

@@ -576,39 +576,41 @@ int sweep_predictor(double dt, bool first, bool last) {
   return 0;
 }
 
-// the geometry of a full sweep along AX; rest is the axis still to be swept
-// after it, 3 for the first sweep (two are) and -1 for the last.  From the
-// second sweep on, cv1 is the cv2 of the sweep before.
-template <int AX>
-int geom_full(int rest, double dt) {
+// The geometry of a full remap lives in Lagrangian work arrays, which nothing
+// reads between the corrector and the next step: the widths d?b1 of the three
+// axes, and the volumes before the first, second and last sweep (k_geom).
+real *remap_db1(int ax) { return ax == 0 ? S.al1 : (ax == 1 ? S.al2 : S.al3); }
+real *remap_vol(int q) { return q == 0 ? S.cv1 : (q == 1 ? S.cv2 : S.visc_heat); }
+int geom_full(int a0, int a1, double dt) {
   const Box cb = marched(cell_box());
-#define GEOM(R)                                                                                                      \
-  LAUNCH("geom", (k_geom<AX, R>), zchunk_grid(cb), box_block(), S.g, cb, S.vx1, S.vy1, S.vz1, S.cv1, S.cv2, S.db1, dt)
-  if (rest == 3) {
-    GEOM(3);
-    return 0;
+#define GEOM(P, Q)                                                                                                  \
+  if (a0 == P && a1 == Q) {                                                                                         \
+    LAUNCH("geom", (k_geom<P, Q>), zchunk_grid(cb), box_block(), S.g, cb, S.vx1, S.vy1, S.vz1, remap_vol(0),        \
+           remap_vol(1), remap_vol(2), remap_db1(0), remap_db1(1), remap_db1(2), dt);                               \
+    return 0;                                                                                                       \
   }
-  real *t = S.cv1;
-  S.cv1 = S.cv2;
-  S.cv2 = t;
-  if (rest < 0) GEOM(-1);
-  else if (rest == (AX + 1) % 3) GEOM((AX + 1) % 3);
-  else GEOM((AX + 2) % 3);
+  GEOM(0, 1)
+  GEOM(0, 2)
+  GEOM(1, 0)
+  GEOM(1, 2)
+  GEOM(2, 0)
+  GEOM(2, 1)
 #undef GEOM
-  return 0;
+  return fail(LARE_E_ARG, "remap axes %d, %d", a0, a1);
 }
 
-// one full sweep; first, last: its place in the remap, rest: see geom_full
+// the full sweep along AX, number q of the remap
 template <int AX>
-int sweep_full(double dt, bool first, bool last, int rest) {
+int sweep_full(double dt, int q) {
   const int N[3] = {nx(), ny(), nz()};
   const real *vel = AX == 0 ? S.vx1 : (AX == 1 ? S.vy1 : S.vz1);
-  int rc = geom_full<AX>(rest, dt);
-  if (rc) return rc;
+  const bool first = q == 0, last = q == 2;
+  const real *db1 = remap_db1(AX), *cv1 = remap_vol(q), *cv2 = last ? nullptr : remap_vol(q + 1);
+  int rc;
   {
     const double *const B[3] = {S.bx, S.by, S.bz};
     double *const spare[3] = {S.fxr, S.fyr, S.fzr};
-    rc = ct_sweep<AX>(B, spare, vel, S.db1, dt, first ? 1 : (last ? -1 : 0));
+    rc = ct_sweep<AX>(B, spare, vel, db1, dt, first ? 1 : (last ? -1 : 0));
     if (rc) return rc;
     swap_spare(S.bx, S.by, S.bz);
   }
@@ -624,15 +626,15 @@ int sweep_full(double dt, bool first, bool last, int rest) {
     const dim3 gx(wave_blocks((long)(mb.x1 - mb.x0 + 1) * (mb.y1 - mb.y0 + 1), REX_OUT), 1,
                   (unsigned)(mb.z1 - mb.z0 + 1));
 #define RHO_ENERGY(L)                                                                                               \
-  LAUNCH("rho_energy", k_mass_rho_energy_x<L>, gx, box_block(), S.g, mb, S.energy, S.rho, vel, S.db1, S.dm, S.cv1, \
-         S.cv2, S.rho_alt, S.Fe, dt, S.per[AX] ? 1 : 0)
+  LAUNCH("rho_energy", k_mass_rho_energy_x<L>, gx, box_block(), S.g, mb, S.energy, S.rho, vel, db1, S.dm, cv1, \
+         cv2, S.rho_alt, S.Fe, dt, S.per[AX] ? 1 : 0)
     if (last) RHO_ENERGY(true);
     else RHO_ENERGY(false);
 #undef RHO_ENERGY
   } else {
 #define RHO_ENERGY(L)                                                                                               \
   LAUNCH("rho_energy", (k_mass_rho_energy_m<AX, L>), zchunk_grid(march_box(mb, AX)), box_block(), S.g, mb, S.energy, \
-         S.rho, vel, S.db1, S.dm, S.cv1, S.cv2, S.rho_alt, S.Fe, dt, S.per[AX] ? 1 : 0)
+         S.rho, vel, db1, S.dm, cv1, cv2, S.rho_alt, S.Fe, dt, S.per[AX] ? 1 : 0)
     if (last) RHO_ENERGY(true);
     else RHO_ENERGY(false);
 #undef RHO_ENERGY
@@ -660,8 +662,8 @@ int sweep_full(double dt, bool first, bool last, int rest) {
       xb.zc = march_chunk(pb, xb.z1 - xb.z0 + 1);
       const dim3 gx(pb, 1, (unsigned)((xb.z1 - xb.z0 + xb.zc) / xb.zc));
 #define MOM_REMAP(R, L)                                                                                          \
-  LAUNCH("mom_remap", (k_mom_remap_x<R, L>), gx, box_block(), S.g, xb, S.vx, S.vy, S.vz, vel, S.db1, S.rho, S.cv1, \
-         S.cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk)
+  LAUNCH("mom_remap", (k_mom_remap_x<R, L>), gx, box_block(), S.g, xb, S.vx, S.vy, S.vz, vel, db1, S.rho, cv1, \
+         cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk)
       if (S.delta_ke && last) MOM_REMAP(true, true);
       else if (S.delta_ke) MOM_REMAP(true, false);
       else if (last) MOM_REMAP(false, true);
@@ -671,7 +673,7 @@ int sweep_full(double dt, bool first, bool last, int rest) {
       xb = marched(xb, AX);
 #define MOM_REMAP(R, L)                                                                                               \
   LAUNCH("mom_remap", (k_mom_remap_m<AX, R, L>), zchunk_grid(march_box(xb, AX)), box_block(), S.g, xb, S.vx, S.vy,  \
-         S.vz, vel, S.db1, S.rho, S.cv1, S.cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk)
+         S.vz, vel, db1, S.rho, cv1, cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk)
       if (S.delta_ke && last) MOM_REMAP(true, true);
       else if (S.delta_ke) MOM_REMAP(true, false);
       else if (last) MOM_REMAP(false, true);
@@ -716,12 +718,11 @@ int eulerian_remap(int step, bool predictor) {
   }
   // rke: delta_ke = 0 (remap.f90:38); only the interior is ever read
   if (S.delta_ke) LAUNCH_BOX("fill", k_fill, interior(), S.delta_ke, 0.0);
+  int rc = geom_full(kStrang[c][0], kStrang[c][1], dt);
+  if (rc) return rc;
   for (int q = 0; q < 3; ++q) {
     const int ax = kStrang[c][q];
-    const bool first = q == 0, last = q == 2;
-    const int rest = first ? 3 : (last ? -1 : kStrang[c][2]);
-    int rc = ax == 0 ? sweep_full<0>(dt, first, last, rest)
-                     : (ax == 1 ? sweep_full<1>(dt, first, last, rest) : sweep_full<2>(dt, first, last, rest));
+    rc = ax == 0 ? sweep_full<0>(dt, q) : (ax == 1 ? sweep_full<1>(dt, q) : sweep_full<2>(dt, q));
     if (rc) return rc;
   }
   return 0;

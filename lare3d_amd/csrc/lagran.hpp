@@ -1246,51 +1246,84 @@ struct FtnLayout {
 // partials of (en_b, en_ke, en_int, -|div B| dx) over nodes 0..n; the cell
 // terms on cells 1..n.  The layout L says where each staggering keeps
 // element (i, j, k); the arithmetic does not depend on it.
+//
+// Bound by its reads at large sizes, by the launch and the folds that follow
+// at small ones.  Marches in z: the masses of plane k+1 and bz of plane k
+// serve the next plane, and a block's partial covers its chunk, so at 64^3
+// one block folds the 561 partials (one per plane and tile would be 1105,
+// folded in two launches).
+template <class R>
+struct MassQuad {
+  R r;          // rho of (i, j)
+  double m[4];  // rho cv of the four cells of a node in one plane
+};
 template <class L, class R>
-__global__ __launch_bounds__(BX * BY) void k_energy(Geo g, L lay, const R *__restrict__ rho,
+__device__ __forceinline__ MassQuad<R> mass_quad(const L &lay, const R *__restrict__ rho, const double area[4], double dz,
+                                              int i, int j, int k) {
+  MassQuad<R> q;
+  const int di[4] = {0, 1, 0, 1}, dj[4] = {0, 0, 1, 1};
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const R r = rho[lay.cell(i + di[p], j + dj[p], k)];
+    if (p == 0) q.r = r;
+    q.m[p] = r * (area[p] * dz);
+  }
+  return q;
+}
+template <class L, class R>
+__global__ __launch_bounds__(BX * BY) void k_energy(Geo g, Box b, L lay, const R *__restrict__ rho,
                                                     const R *__restrict__ energy, const R *__restrict__ vx,
                                                     const R *__restrict__ vy, const R *__restrict__ vz,
                                                     const double *__restrict__ bx, const double *__restrict__ by,
                                                     const double *__restrict__ bz, double *__restrict__ partial) {
-  const Box b = {0, g.nx, 0, g.ny, 0, g.nz};
   PLANE_POS(b, i, j)
-  const int k = (int)blockIdx.z;
+  ZRANGE(b, k0, k1)
   double v[4] = {0.0, 0.0, 0.0, 0.0};
-  if (j <= g.ny && k <= g.nz) {
-    if (i >= 1 && j >= 1 && k >= 1) {
-      const double bx0 = bx[lay.fx(i, j, k)], bxm = bx[lay.fx(i - 1, j, k)];
-      const double by0 = by[lay.fy(i, j, k)], bym = by[lay.fy(i, j - 1, k)];
-      const double bz0 = bz[lay.fz(i, j, k)], bzm = bz[lay.fz(i, j, k - 1)];
-      double w1 = (bx0 * bx0 + bxm * bxm) * 0.5;
-      const double w2 = (by0 * by0 + bym * bym) * 0.5;
-      const double w3 = (bz0 * bz0 + bzm * bzm) * 0.5;
-      w1 = (w1 + w2 + w3) * 0.5;
-      const double cv = g.cv(i, j, k);
-      const int c = lay.cell(i, j, k);
-      v[0] = w1 * cv;
-      v[2] = energy[c] * rho[c] * cv;
-      const double dx = g.dxb[i], dy = g.dyb[j], dz = g.dzb[k];
-      const double d = (bx0 - bxm) / dx + (by0 - bym) / dy + (bz0 - bzm) / dz;
-      v[3] = -(fabs(d) * dmin(dmin(dx, dy), dz));
+  if (j <= g.ny) {
+    const bool cell = i >= 1 && j >= 1;
+    const double dx = g.dxb[i], dy = g.dyb[j], dx1 = g.dxb[i + 1], dy1 = g.dyb[j + 1];
+    const double area[4] = {dx * dy, dx1 * dy, dx * dy1, dx1 * dy1};
+    const Recip<double> rx = recip(dx), ry = recip(dy);
+    double wij = 1.0;  // halves on the boundary nodes
+    if (i == 0 || i == g.nx) wij = 0.5;
+    if (j == 0 || j == g.ny) wij = wij * 0.5;
+    double dz = g.dzb[k0];
+    MassQuad<R> lo = mass_quad(lay, rho, area, dz, i, j, k0);
+    double bzm = cell && k0 >= 1 ? bz[lay.fz(i, j, k0 - 1)] : 0.0;
+    for (int k = k0; k <= k1; ++k) {
+      const double dz1 = g.dzb[k + 1];
+      const MassQuad<R> hi = mass_quad(lay, rho, area, dz1, i, j, k + 1);
+      if (cell) {
+        const double bz0 = bz[lay.fz(i, j, k)];
+        if (k >= 1) {
+          const double bx0 = bx[lay.fx(i, j, k)], bxm = bx[lay.fx(i - 1, j, k)];
+          const double by0 = by[lay.fy(i, j, k)], bym = by[lay.fy(i, j - 1, k)];
+          double w1 = (bx0 * bx0 + bxm * bxm) * 0.5;
+          const double w2 = (by0 * by0 + bym * bym) * 0.5;
+          const double w3 = (bz0 * bz0 + bzm * bzm) * 0.5;
+          w1 = (w1 + w2 + w3) * 0.5;
+          const double cv = area[0] * dz;
+          v[0] = v[0] + w1 * cv;
+          v[2] = v[2] + energy[lay.cell(i, j, k)] * lo.r * cv;
+          const double d = (bx0 - bxm) / rx + (by0 - bym) / ry + (bz0 - bzm) / recip(dz);
+          v[3] = dmin(v[3], -(fabs(d) * dmin(dmin(dx, dy), dz)));
+        }
+        bzm = bz0;
+      }
+      double rv = lo.m[0];
+#pragma unroll
+      for (int q = 1; q < 8; ++q) rv = rv + (q < 4 ? lo.m[q] : hi.m[q - 4]);
+      double cvv = area[0] * dz;
+#pragma unroll
+      for (int q = 1; q < 8; ++q) cvv = cvv + (q < 4 ? area[q] * dz : area[q - 4] * dz1);
+      rv = rv / recip(cvv);
+      const int n = lay.node(i, j, k);
+      double w1 = rv * (cvv * 0.125) * (vx[n] * vx[n] + vy[n] * vy[n] + vz[n] * vz[n]) * wij;
+      if (k == 0 || k == g.nz) w1 = w1 * 0.5;
+      v[1] = v[1] + w1 * 0.5;
+      lo = hi;
+      dz = dz1;
     }
-    double cvs[8];
-    const int di[8] = {0, 1, 0, 1, 0, 1, 0, 1}, dj[8] = {0, 0, 1, 1, 0, 0, 1, 1}, dk[8] = {0, 0, 0, 0, 1, 1, 1, 1};
-#pragma unroll
-    for (int q = 0; q < 8; ++q) cvs[q] = g.cv(i + di[q], j + dj[q], k + dk[q]);
-    double rv = rho[lay.cell(i, j, k)] * cvs[0];
-#pragma unroll
-    for (int q = 1; q < 8; ++q) rv = rv + rho[lay.cell(i + di[q], j + dj[q], k + dk[q])] * cvs[q];
-    double cvv = cvs[0];
-#pragma unroll
-    for (int q = 1; q < 8; ++q) cvv = cvv + cvs[q];
-    rv = rv / cvv;
-    cvv = cvv * 0.125;
-    const int n = lay.node(i, j, k);
-    double w1 = rv * cvv * (vx[n] * vx[n] + vy[n] * vy[n] + vz[n] * vz[n]);
-    if (i == 0 || i == g.nx) w1 = w1 * 0.5;
-    if (j == 0 || j == g.ny) w1 = w1 * 0.5;
-    if (k == 0 || k == g.nz) w1 = w1 * 0.5;
-    v[1] = w1 * 0.5;
   }
   const int ops[4] = {1, 1, 1, 0};
   block_reduce_store<4>(v, ops, partial);

@@ -82,9 +82,9 @@ int api_energy_account_noalloc(const lare_grid *grid, const lare_fields *f, doub
       return fail(LARE_E_ARG, "energy_account_noalloc: grid size %d on axis %d outside 4..%d", n[a], a, NA_NMAX);
   const long nodes = (long)(n[0] + 5) * (n[1] + 5) * (n[2] + 5);
   if (nodes > 2147483647L) return fail(LARE_E_ARG, "energy_account_noalloc: grid too large for 32-bit indexing");
-  const fp64::Box b = fp64::mkbox(0, n[0], 0, n[1], 0, n[2]);
-  const dim3 gr = fp64::box_grid(b);
-  const long nb = (long)gr.x * gr.y * gr.z;
+  fp64::Box b = fp64::mkbox(0, n[0], 0, n[1], 0, n[2]);
+  const unsigned tiles = fp64::plane_blocks(b);
+  const long nb = (long)tiles * (n[2] + 1);
   if (nb > NA_MAX_BLOCKS)
     return fail(LARE_E_ARG,
                 "energy_account_noalloc: %ld reduction blocks exceed the scratch maximum of %d "
@@ -126,11 +126,13 @@ int api_energy_account_noalloc(const lare_grid *grid, const lare_fields *f, doub
   g.dyb = met + NA_LEN + 2;
   g.dzb = met + 2 * NA_LEN + 2;
   const fp64::FtnLayout lay = {n[0], n[1], n[2]};
-  hipLaunchKernelGGL((fp64::k_energy<fp64::FtnLayout, double>), gr, fp64::box_block(), 0, 0, g, lay, f->rho, f->energy,
+  b.zc = fp64::march_chunk(tiles, n[2] + 1);
+  const dim3 gr(tiles, 1, (unsigned)((n[2] + b.zc) / b.zc));
+  hipLaunchKernelGGL((fp64::k_energy<fp64::FtnLayout, double>), gr, fp64::box_block(), 0, 0, g, b, lay, f->rho, f->energy,
                      f->vx, f->vy, f->vz, f->bx, f->by, f->bz, partial);
   HIPCHK(hipGetLastError());
   // the fold of fp64::final_reduce, on the scratch array
-  const int nbi = (int)nb, nv = 4, minmask = 8;
+  const int nbi = (int)(gr.x * gr.z), nv = 4, minmask = 8;
   int rows;
   const int chunk = fp64::fold_chunk(nbi, &rows);
   if (chunk) {

@@ -335,12 +335,13 @@ CondArgs cond_args() {
 }
 
 int calc_s_stages() {
-  dim3 gr = grid_from0(nx(), ny(), nz());
+  const Box b = marched(nodes0n());
+  const dim3 gr = zchunk_grid(b);
   if (S.pi_eos)
-    LAUNCH("larsen", k_larsen<true>, gr, box_block(), S.g, S.energy, S.rho, S.larsen, S.partial, S.p.flux_limiter,
+    LAUNCH("larsen", k_larsen<true>, gr, box_block(), S.g, b, S.energy, S.rho, S.larsen, S.partial, S.p.flux_limiter,
            S.p.kappa_0, cond_args(), S.p.heat_flux_limiter);
   else
-    LAUNCH("larsen", k_larsen<false>, gr, box_block(), S.g, S.energy, S.rho, S.larsen, S.partial, S.p.flux_limiter,
+    LAUNCH("larsen", k_larsen<false>, gr, box_block(), S.g, b, S.energy, S.rho, S.larsen, S.partial, S.p.flux_limiter,
            S.p.kappa_0, cond_args(), S.p.heat_flux_limiter);
   int rc = final_reduce(gr, 1, 1, 0, 0);
   if (rc) return rc;
@@ -1515,13 +1516,19 @@ int api_get_neutral(double *xi_h, double *ep_h) {
   return rc;
 }
 
+// the four sums of k_energy to scalars 0..3
+int energy_sums() {
+  const Box b = marched(nodes0n());
+  const dim3 gr = zchunk_grid(b);
+  LAUNCH("energy", (k_energy<PadLayout, real>), gr, box_block(), S.g, b, PadLayout{S.g}, S.rho, S.energy, S.vx, S.vy,
+         S.vz, S.bx, S.by, S.bz, S.partial);
+  return final_reduce(gr, 4, 8, 0, 0);
+}
+
 int api_energy_account(double en[3], double *divb) {
   REQUIRE_LOADED();
   if (!en) return fail(LARE_E_ARG, "energy_account: NULL output");
-  dim3 gr = grid_from0(nx(), ny(), nz());
-  LAUNCH("energy", (k_energy<PadLayout, real>), gr, box_block(), S.g, PadLayout{S.g}, S.rho, S.energy, S.vx, S.vy,
-         S.vz, S.bx, S.by, S.bz, S.partial);
-  int rc = final_reduce(gr, 4, 8, 0, 0);
+  int rc = energy_sums();
   if (rc) return rc;
   double v[4];
   rc = read_scalars(0, 4, v);
@@ -2085,10 +2092,7 @@ int api_step_info(int32_t step, int32_t with_energy, lare_step_info *o) {
   int rc = api_step(step, &dt, &t);
   if (rc) return rc;
   if (with_energy) {
-    dim3 gr = grid_from0(nx(), ny(), nz());
-    LAUNCH("energy", (k_energy<PadLayout, real>), gr, box_block(), S.g, PadLayout{S.g}, S.rho, S.energy, S.vx, S.vy,
-           S.vz, S.bx, S.by, S.bz, S.partial);
-    rc = final_reduce(gr, 4, 8, 0, 0);
+    rc = energy_sums();
     if (rc) return rc;
   }
   double v[10];

@@ -470,6 +470,15 @@ __device__ __forceinline__ BPlane bplane(const double *__restrict__ bx, const do
   return p;
 }
 
+// bz at (i,j), (i+1,j), (i,j+1), (i+1,j+1) of one plane
+struct BzPlane {
+  double z0, zx, zy, zxy;
+};
+__device__ __forceinline__ BzPlane bzplane(const double *__restrict__ bz, int c, int Y) {
+  BzPlane p = {bz[c], bz[c + 1], bz[c + Y], bz[c + 1 + Y]};
+  return p;
+}
+
 // vertex current of lagran.F90:1479-1494 (also :358-373, :1424-1439) from
 // bx, by of planes k (lo) and k+1 (hi) and bz at (i,j), (i+1,j), (i,j+1),
 // (i+1,j+1) of plane k
@@ -590,8 +599,11 @@ struct EPlane {
 #define RS_ROWS 8
 #define RS_OUT_X 63
 #define RS_OUT_Y (RS_ROWS - 1)
-// FP32: held to five waves per SIMD (192^3: 484 us per step's substeps
-// against 546 with the compiler's choice; FP64 loses 4% by the same bound).
+// FP64 loads the face field a plane ahead and the cell's own values before
+// the barrier, which no load may cross (118 registers, still two blocks per
+// CU; a substep at 256^3 646 -> 602 us).  FP32 loads where it uses and keeps
+// the registers of three blocks (192^3: 240 us; loading ahead 250).
+#define RS_AHEAD (sizeof(acc) == sizeof(double))
 #define RS_WAVES (sizeof(acc) == sizeof(float) ? 5 : 1)
 template <bool COWL>
 __global__ __launch_bounds__(64 * RS_ROWS, RS_WAVES) void k_resist(Geo g, Box b, int tiles_x, const double *__restrict__ bx,
@@ -622,27 +634,59 @@ __global__ __launch_bounds__(64 * RS_ROWS, RS_WAVES) void k_resist(Geo g, Box b,
   double v = 0.0;
   EPlane m = {0, 0, 0, 0, 0, 0, 0};  // plane k-1
   acc mq[4] = {0, 0, 0, 0};          // curlb of plane k-1 at (i,j), (i-1,j), (i,j-1), (i-1,j-1)
-  BPlane lo = {0, 0, 0, 0};
-  bool have_lo = false;
+  // face bx, by of planes k (lo) and k+1 (hi), bz of plane k
+  BPlane lo = {0, 0, 0, 0}, hi = {0, 0, 0, 0};
+  BzPlane zb = {0, 0, 0, 0};
+  if (eij && k0 >= 0) lo = bplane(bx, by, g.idx(i, j, k0 - 1), Y);
+  if (RS_AHEAD && eij && k0 >= -1) {
+    hi = bplane(bx, by, g.idx(i, j, k0), Y);
+    if (k0 >= 0) zb = bzplane(bz, g.idx(i, j, k0 - 1), Y);
+  }
   for (int k = k0 - 1; k <= k1; ++k) {
     const int c = g.idx(i, j, k);
+    const bool ein = eij && k >= -1 && k <= g.nz + 1;
+    const bool own = out && k >= k0;
+    const bool cell = own && cij && k >= -1 && k <= g.nz + 2, hot = cell && hij && k >= 1 && k <= g.nz;
+    acc e_own = 0.0, od_own = 0.0, r_own = 1.0;
+    auto load_cell = [&] {
+      if (cell) e_own = energy[c];
+      if (hot) {
+        od_own = ohmic_dep[c];
+        r_own = rho[c];
+      }
+    };
+    BPlane next = {0, 0, 0, 0};
+    BzPlane zn = {0, 0, 0, 0};
+    if (RS_AHEAD) {
+      if (eij && k < k1 && k <= g.nz) {
+        next = bplane(bx, by, c + 2 * Z, Y);
+        if (k >= -2) zn = bzplane(bz, c + Z, Y);
+      }
+    } else if (eij && k >= -2 && k <= g.nz + 1) {
+      hi = bplane(bx, by, c + Z, Y);
+      if (k >= -1) zb = bzplane(bz, c, Y);
+    }
+    double nbx = lo.bx0, nby = lo.by0, nbz = zb.z0;
+    auto load_b = [&] {
+      nbx = bx[c];
+      nby = by[c];
+      nbz = bz[c];
+    };
+    if (RS_AHEAD) {
+      load_cell();
+      if (own && !ein) load_b();
+    }
     acc kx = 0.0, ky = 0.0, kz = 0.0, cbr = 0.0;
-    if (eij && k >= -1 && k <= g.nz + 1) {
-      if (!have_lo) lo = bplane(bx, by, c, Y);
-      const BPlane hi = bplane(bx, by, c + Z, Y);
+    if (ein) {
       acc jx, jy, jz;
-      vertex_current_acc(rx, ry, recip((acc)g.dzc[k]), lo, hi, bz[c], bz[c + 1], bz[c + Y], bz[c + 1 + Y], jx, jy,
-                         jz);
-      const BPlane plo = lo;
-      lo = hi;
-      have_lo = true;
+      vertex_current_acc(rx, ry, recip((acc)g.dzc[k]), lo, hi, zb.z0, zb.zx, zb.zy, zb.zxy, jx, jy, jz);
       const real es = sqrt(jx * jx + jy * jy + jz * jz) > (acc)j_max ? eta_bg + eta0 : eta_bg;
       if (out && k >= k0 && eta) eta[c] = es;
       if (kij && k >= 0 && k <= g.nz) {
         const acc e = es;
         acc cb;
         if constexpr (COWL) {
-          cowling_emf(plo, hi, bz[c], bz[c + 1], bz[c + Y], bz[c + 1 + Y], jx, jy, jz, e, (acc)eta_perp[c],
+          cowling_emf(lo, hi, zb.z0, zb.zx, zb.zy, zb.zxy, jx, jy, jz, e, (acc)eta_perp[c],
                       (acc)g.dxc[i], (acc)g.dyc[j], (acc)g.dzc[k], kx, ky, kz, cb);
         } else {
           kx = -jx * e * (acc)g.dxc[i] * (acc)0.5;
@@ -672,7 +716,7 @@ __global__ __launch_bounds__(64 * RS_ROWS, RS_WAVES) void k_resist(Geo g, Box b,
       const EPlane p = {kx, s[0][w][l - 1], ky, s[1][w - 1][l], kz, s[2][w - 1][l], s[2][w][l - 1]};
       if (k >= k0) {
         const bool upd = kij && k >= 0 && k <= g.nz;
-        double nbx = bx[c], nby = by[c], nbz = bz[c];
+        if (!RS_AHEAD) load_b();
         if (upd && j >= 1 && k >= 1) {
           const double area = g.dyb[j] * g.dzb[k];
           nbx = nbx + ((double)p.kz0 - p.kzm + m.kz0 - m.kzm - p.ky0 + m.ky0 - p.kym + m.kym) * dt / recip(area);
@@ -692,13 +736,14 @@ __global__ __launch_bounds__(64 * RS_ROWS, RS_WAVES) void k_resist(Geo g, Box b,
         bzo[c] = nbz;
       }
       const acc pq[4] = {cbr, s[3][w][l - 1], s[3][w - 1][l], s[3][w - 1][l - 1]};
-      if (k >= k0 && cij && k >= -1 && k <= g.nz + 2) {
-        acc e = energy[c];
-        if (hij && k >= 1 && k <= g.nz) {
+      if (!RS_AHEAD) load_cell();
+      if (cell) {
+        acc e = e_own;
+        if (hot) {
           // curlb(c) + (c-X) + (c-Y) + (c-X-Y) + (c-Z) + (c-X-Z) + (c-Y-Z) + (c-X-Y-Z)
           const acc sq = pq[0] + pq[1] + pq[2] + pq[3] + mq[0] + mq[1] + mq[2] + mq[3];
-          const acc lh = sq * (acc)dt / recip((acc)8.0 * rho[c]);
-          ohmic_dep[c] = ohmic_dep[c] + lh;
+          const acc lh = sq * (acc)dt / recip((acc)8.0 * r_own);
+          ohmic_dep[c] = od_own + lh;
           e = e + lh;
         }
         // with the cooling_term, k_cool_b takes the cooling off first and
@@ -708,6 +753,11 @@ __global__ __launch_bounds__(64 * RS_ROWS, RS_WAVES) void k_resist(Geo g, Box b,
 #pragma unroll
       for (int q = 0; q < 4; ++q) mq[q] = pq[q];
       m = p;
+    }
+    lo = hi;
+    if (RS_AHEAD) {
+      hi = next;
+      zb = zn;
     }
   }
   v = wave_sum(v);

@@ -18,6 +18,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <initializer_list>
 #include <string>
 #include <thread>
 #include <vector>

@@ -1139,12 +1139,14 @@ int lagrangian_step() {
 // ----------------------------------------------------------------------------
 #include "transfer.hpp"
 void sur_free();
+void slab_drop();
 void free_all() {
   sur_free();
   if (S.stream) (void)hipStreamSynchronize(S.stream);
   xfer_free();
   for (void *p : S.allocs) (void)hipFree(p);
   S.allocs.clear();
+  slab_drop();
   if (S.metric) (void)hipFree(S.metric);
   S.metric = nullptr;
   if (S.partial) (void)hipFree(S.partial);
@@ -1164,8 +1166,41 @@ void free_all() {
   S.ready = S.loaded = false;
 }
 
+// The arrays of the padded box come out of one allocation, made and cleared at
+// once: some 45 of their own took 1.5 ms to open and 3.4 ms to close at 32^3.
+// Where it is not to be had, or is used up, an array gets its own.
+#define SLAB_ALIGN 256
+struct Slab {
+  char *p = nullptr;
+  size_t cap = 0, used = 0;
+};
+Slab g_slab;
+void slab_drop() { g_slab = Slab(); }
+
+size_t slab_bytes(size_t n) { return (n + SLAB_ALIGN - 1) / SLAB_ALIGN * SLAB_ALIGN; }
+int slab_reserve(int reals, int doubles) {
+  g_slab = Slab();
+  const size_t n = reals * slab_bytes(sizeof(real) * S.ntot) + doubles * slab_bytes(sizeof(double) * S.ntot);
+  void *p = nullptr;
+  if (hipMalloc(&p, n) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  S.allocs.push_back(p);
+  g_slab.p = (char *)p;
+  g_slab.cap = n;
+  const hipError_t e = hipMemsetAsync(p, 0, n, S.stream);
+  return e == hipSuccess ? 0 : fail(-(int)e, "hipMemset failed");
+}
+
 template <class T>
 int dalloc(T **p) {
+  const size_t n = slab_bytes(sizeof(T) * S.ntot);
+  if (g_slab.cap - g_slab.used >= n) {
+    *p = (T *)(g_slab.p + g_slab.used);
+    g_slab.used += n;
+    return 0;
+  }
   hipError_t e = hipMalloc((void **)p, sizeof(T) * S.ntot);
   if (e != hipSuccess) return fail(LARE_E_NOMEM, "hipMalloc of %zu elements failed: %s", S.ntot, hipGetErrorString(e));
   S.allocs.push_back((void *)*p);
@@ -1302,11 +1337,23 @@ int api_init(const lare_grid *grid, const lare_params *params) {
                     &S.visc3, &S.visc_dep, &S.ohmic_dep, &S.rho_v, &S.cs_v, &S.al1, &S.al2, &S.al3,
                     &S.visc_heat, &S.p0, &S.pp, &S.cv1, &S.cv2, &S.db1, &S.Fe, &S.dm, &S.Fx, &S.Fy,
                     &S.Fz, &S.larsen, &S.Lc, &S.Yb[0], &S.Yb[1], &S.Yb[2]};
+  double **wide[] = {&S.bx, &S.by, &S.bz, &S.bpx, &S.bpy, &S.bpz, &S.fxr, &S.fyr, &S.fzr, &S.F, &S.F2};
+  {
+    // with the arrays of the options taken below
+    int reals = (int)(sizeof(bulk) / sizeof(bulk[0]));
+    if (params->fourth_order && params->resistive_mhd) reals += 8;
+    if (params->rke) reals += 4;
+    if (pi) reals += params->cowling_resistivity ? 2 : 1;
+    if (params->boris) reals += 1;
+    if (params->cooling_term) reals += params->resistive_mhd ? 3 : 2;
+    if (params->use_viscous_damping) reals += 3;
+    const int rc = slab_reserve(reals, (int)(sizeof(wide) / sizeof(wide[0])));
+    if (rc) return rc;
+  }
   for (real **pp : bulk) {
     int rc = dalloc(pp);
     if (rc) return rc;
   }
-  double **wide[] = {&S.bx, &S.by, &S.bz, &S.bpx, &S.bpy, &S.bpz, &S.fxr, &S.fyr, &S.fzr, &S.F, &S.F2};
   for (double **pp : wide) {
     int rc = dalloc(pp);
     if (rc) return rc;
@@ -1643,6 +1690,7 @@ int api_finalize(void) {
 
 
 struct Sur {
+  char *param_mem = nullptr, *field_mem = nullptr, *batch_mem = nullptr;  // the allocations of the groups below
   float *w = nullptr, *gr = nullptr, *m = nullptr, *v = nullptr;  // SUR_NPARAM each
   unsigned short *w1t = nullptr, *w2t = nullptr;                   // packed BF16 for inference
   bool have_params = false, have_norm = false;
@@ -1676,14 +1724,16 @@ void sfree(T *&p) {
 }
 
 void sur_free_batch() {
-  sfree(SU.Xb); sfree(SU.yb); sfree(SU.row); sfree(SU.H1); sfree(SU.H2); sfree(SU.yo);
-  sfree(SU.dy); sfree(SU.dZ2); sfree(SU.dZ1); sfree(SU.lossacc);
+  sfree(SU.batch_mem);
+  SU.Xb = SU.yb = SU.H1 = SU.H2 = SU.yo = SU.dy = SU.dZ2 = SU.dZ1 = nullptr;
+  SU.lossacc = nullptr;
+  SU.row = nullptr;
   SU.bcap = 0;
 }
 
 void sur_free() {
-  sfree(SU.w); sfree(SU.gr); sfree(SU.m); sfree(SU.v); sfree(SU.w1t); sfree(SU.w2t);
-  sfree(SU.feat); sfree(SU.E1); sfree(SU.trap); sfree(SU.E0save);
+  sfree(SU.param_mem);
+  sfree(SU.field_mem);
   sfree(SU.X); sfree(SU.y); sfree(SU.cells); sfree(SU.losshist);
   sur_free_batch();
   const int en = SU.enabled;
@@ -1701,14 +1751,30 @@ int salloc(T **p, size_t count) {
   return 0;
 }
 
+// the arrays of one group in one allocation
+struct SurPart {
+  void **p;
+  size_t bytes;
+  template <class T>
+  SurPart(T **q, size_t count) : p((void **)q), bytes(slab_bytes(sizeof(T) * count)) {}
+};
+int salloc_group(char **mem, std::initializer_list<SurPart> parts) {
+  size_t total = 0;
+  for (const SurPart &q : parts) total += q.bytes;
+  int rc = salloc(mem, total);
+  if (rc) return rc;
+  char *at = *mem;
+  for (const SurPart &q : parts) {
+    *q.p = at;
+    at += q.bytes;
+  }
+  return 0;
+}
+
 int sur_alloc_params() {
   if (SU.w) return 0;
-  int rc = salloc(&SU.w, SUR_NPARAM);
-  if (!rc) rc = salloc(&SU.gr, SUR_NPARAM);
-  if (!rc) rc = salloc(&SU.m, SUR_NPARAM);
-  if (!rc) rc = salloc(&SU.v, SUR_NPARAM);
-  if (!rc) rc = salloc(&SU.w1t, SUR_H * SUR_KP);
-  if (!rc) rc = salloc(&SU.w2t, SUR_H * SUR_HP);
+  int rc = salloc_group(&SU.param_mem, {{&SU.w, SUR_NPARAM}, {&SU.gr, SUR_NPARAM}, {&SU.m, SUR_NPARAM},
+                                        {&SU.v, SUR_NPARAM}, {&SU.w1t, SUR_H * SUR_KP}, {&SU.w2t, SUR_H * SUR_HP}});
   if (rc) return rc;
   HIPCHK(hipMemsetAsync(SU.m, 0, sizeof(float) * SUR_NPARAM, S.stream));
   HIPCHK(hipMemsetAsync(SU.v, 0, sizeof(float) * SUR_NPARAM, S.stream));
@@ -1717,10 +1783,8 @@ int sur_alloc_params() {
 
 int sur_alloc_fields() {
   if (SU.feat) return 0;
-  int rc = salloc(&SU.feat, S.ntot * SUR_CH);
-  if (!rc) rc = salloc(&SU.E1, S.ntot);
-  if (!rc) rc = salloc(&SU.trap, S.ntot);
-  if (!rc) rc = salloc(&SU.E0save, S.ntot);
+  int rc = salloc_group(&SU.field_mem,
+                        {{&SU.feat, S.ntot * SUR_CH}, {&SU.E1, S.ntot}, {&SU.trap, S.ntot}, {&SU.E0save, S.ntot}});
   if (rc) return rc;
   // cells never written by the feature kernel are never read by it either;
   // zero them once so no stale bits reach a gather
@@ -1732,16 +1796,9 @@ int sur_ensure_batch(int cols) {
   if (cols <= SU.bcap) return 0;
   sur_free_batch();
   const size_t c = (size_t)cols;
-  int rc = salloc(&SU.Xb, c * SUR_K);
-  if (!rc) rc = salloc(&SU.yb, c);
-  if (!rc) rc = salloc(&SU.row, c);
-  if (!rc) rc = salloc(&SU.H1, c * SUR_H);
-  if (!rc) rc = salloc(&SU.H2, c * SUR_H);
-  if (!rc) rc = salloc(&SU.yo, c);
-  if (!rc) rc = salloc(&SU.dy, c);
-  if (!rc) rc = salloc(&SU.dZ2, c * SUR_H);
-  if (!rc) rc = salloc(&SU.dZ1, c * SUR_H);
-  if (!rc) rc = salloc(&SU.lossacc, (c + 255) / 256);
+  int rc = salloc_group(&SU.batch_mem, {{&SU.Xb, c * SUR_K}, {&SU.yb, c}, {&SU.row, c}, {&SU.H1, c * SUR_H},
+                                        {&SU.H2, c * SUR_H}, {&SU.yo, c}, {&SU.dy, c}, {&SU.dZ2, c * SUR_H},
+                                        {&SU.dZ1, c * SUR_H}, {&SU.lossacc, (c + 255) / 256}});
   if (rc) return rc;
   SU.bcap = cols;
   return 0;

@@ -601,10 +601,11 @@ struct EPlane {
 #define RS_OUT_Y (RS_ROWS - 1)
 // FP64 loads the face field a plane ahead and the cell's own values before
 // the barrier, which no load may cross (118 registers, still two blocks per
-// CU; a substep at 256^3 646 -> 602 us).  FP32 loads where it uses and keeps
-// the registers of three blocks (192^3: 240 us; loading ahead 250).
+// CU; a substep at 256^3 646 -> 602 us).  FP32 loads where it uses and is held
+// to the registers of three blocks (192^3: 240 us; loading ahead 250, without
+// the bound 270).
 #define RS_AHEAD (sizeof(acc) == sizeof(double))
-#define RS_WAVES (sizeof(acc) == sizeof(float) ? 5 : 1)
+#define RS_WAVES (sizeof(acc) == sizeof(float) ? 6 : 1)
 template <bool COWL>
 __global__ __launch_bounds__(64 * RS_ROWS, RS_WAVES) void k_resist(Geo g, Box b, int tiles_x, const double *__restrict__ bx,
                                                          const double *__restrict__ by, const double *__restrict__ bz,

@@ -82,22 +82,32 @@ static inline Box mkbox(int x0, int x1, int y0, int y1, int z0, int z1) {
 }
 
 // Points a block marches over, for a launch of per_plane blocks on each of
-// `points` march positions: the longest chunk (each chunk re-reads the
-// planes before it) that still launches MARCH_BLOCKS blocks, two for each of
-// the 256 CUs.  Below that a launch is bound by the serial chain of loads of
-// its march, not by bandwidth: with chunks of 8 a marching kernel took 14 to
-// 25 us at 16^3 and at 64^3 alike, and with this rule 4 to 6 and 7 to 10 us.
-// Steps of the resistive sheet (FP64, ms) with chunks of 8 | targets of 256 |
-// 512 | 1024 | 2048 blocks:
-//   16^3 0.34 | 0.205 | 0.200 | 0.197 | 0.197    64^3 0.47 | 0.403 | 0.365 | 0.394 | 0.406
-//   96^3 0.79 | 0.774 | 0.729 | 0.739 | 0.823   128^3 1.55 | 1.545 | 1.545 | 1.548 | 1.528
-#ifndef MARCH_BLOCKS
-#define MARCH_BLOCKS 512
-#endif
+// `points` march positions.  A block of c points costs about c + 1 (the plane
+// before them), and a launch takes as many turns as the fullest of the 256 CUs
+// has blocks; below three blocks per CU a turn is bound by the serial chain of
+// loads of the march and a fuller CU takes no longer.  So: the c with the
+// least max(3, blocks per CU, rounded up) * (c + 1), the longer of two alike.
+// With chunks of 8 a marching kernel took 14 to 25 us at 16^3 and at 64^3
+// alike, and takes 4 to 6 and 7 to 10.  Against the longest of 8, 4, 2, 1 that
+// launches 512 blocks, which left 544 blocks of 4 planes to 64 x 64 x 128
+// (three on some CUs, two on most): 20 conduction super-steps there 9.9 -> 9.5
+// ms, 50 steps with conduction in FP32 28.5 -> 27.6, 50 steps at 97 x 61 x 130
+// 38.4 -> 37.7; 16^3, 64^3 and 192^3 and above unchanged.
+#define MARCH_CUS 256
+#define MARCH_TURNS 3
 static inline int march_chunk(unsigned per_plane, int points) {
-  int c = ZCHUNK;
-  while (c > 1 && (long)per_plane * ((points + c - 1) / c) < MARCH_BLOCKS) c >>= 1;
-  return c;
+  int best = 1;
+  long least = 0;
+  for (int c = 1; c <= ZCHUNK; ++c) {
+    long turns = ((long)per_plane * ((points + c - 1) / c) + MARCH_CUS - 1) / MARCH_CUS;
+    if (turns < MARCH_TURNS) turns = MARCH_TURNS;
+    const long cost = turns * (c + 1);
+    if (c == 1 || cost <= least) {
+      least = cost;
+      best = c;
+    }
+  }
+  return best;
 }
 
 __device__ __forceinline__ double dmin(double a, double b) { return a < b ? a : b; }

@@ -498,7 +498,7 @@ int ct_sweep(const double *const in[3], double *const out[3], const real *vel, c
     // x sweep: va1 = z and ga2 = z (see the flux table above); tiles of
     // CTX_W points in x by CTX_ROWS - 1 rows in y, marching in z
     const int ntx = (N[0] + 5 + CTX_W - 1) / CTX_W, nty = (N[1] + 5 + CTX_ROWS - 2) / (CTX_ROWS - 1);
-    const int mc = march_chunk((unsigned)(ntx * nty), N[2] + 5);
+    const int mc = cts_chunk((unsigned)(ntx * nty), N[2] + 5);
     const dim3 grid((unsigned)(ntx * nty), 1, (unsigned)((N[2] + 4 + mc) / mc));
     if (sc > 0)
       LAUNCH("ct_sweep", k_ct_sweep_x<1>, grid, blk, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX], vel,
@@ -514,7 +514,7 @@ int ct_sweep(const double *const in[3], double *const out[3], const real *vel, c
     // in x by CTM_ROWS - 1 rows along the other transverse axis
     const int P = AX == 2 ? 1 : 2;
     const int ntx = (N[0] + 5 + CTM_XW - 2) / (CTM_XW - 1), nty = (N[P] + 5 + CTM_ROWS - 2) / (CTM_ROWS - 1);
-    const int mc = march_chunk((unsigned)(ntx * nty), N[AX] + 5);
+    const int mc = cts_chunk((unsigned)(ntx * nty), N[AX] + 5);
     const dim3 grid((unsigned)(ntx * nty), 1, (unsigned)((N[AX] + 4 + mc) / mc));
     const dim3 blkm(CTM_THREADS, 1, 1);
     if (sc > 0)

@@ -41,6 +41,11 @@ struct Box {
 #define BX 64
 #define BY 4
 
+// The block and thread coordinates as parameters of a kernel's body that two
+// kernels share: they take the place of the built-in variables, so that the
+// index macros below read them.
+#define BLOCK_COORDS const dim3 blockIdx, const dim3 gridDim, const dim3 threadIdx
+
 // In-plane position (i, j) of a thread of a box launch.  The (x, y) extent
 // of the box is walked as one flattened index, BX*BY consecutive points per
 // block, so a box a few points wider than a multiple of 64 (n+1 .. n+4 for

@@ -343,14 +343,12 @@ __device__ __forceinline__ void ct_store(const Wid &wd, int c, int i, int j, int
 #endif
 #define CTM_ROWS (CTM_THREADS / CTM_XW)
 template <int M, int SC>
-__global__ __launch_bounds__(CTM_THREADS) void k_ct_sweep_m(Geo g, const double *__restrict__ t1i,
-                                                            const double *__restrict__ t2i,
-                                                            const double *__restrict__ ai, double *__restrict__ t1o,
-                                                            double *__restrict__ t2o, double *__restrict__ ao,
-                                                            const real *__restrict__ vel,
-                                                            const real *__restrict__ db1, int VS1, int GS1, int VS2,
-                                                            int GS2, double dt, int ntx, int mc, Box bt1, Box ba1, Box bt2,
-                                                            Box ba2) {
+__device__ __forceinline__ void ct_sweep_m(BLOCK_COORDS, Geo g, const double *__restrict__ t1i,
+                                           const double *__restrict__ t2i, const double *__restrict__ ai,
+                                           double *__restrict__ t1o, double *__restrict__ t2o,
+                                           double *__restrict__ ao, const real *__restrict__ vel,
+                                           const real *__restrict__ db1, int VS1, int GS1, int VS2, int GS2,
+                                           double dt, int ntx, int mc, Box bt1, Box ba1, Box bt2, Box ba2) {
   constexpr int T1 = CtComp<M>::T1, T2 = CtComp<M>::T2;
   constexpr int P = M == 2 ? 1 : 2;
   // fluxes F1, F2 of points m0-1 .. m1 (slot 0 = m0-1)
@@ -472,13 +470,12 @@ __global__ __launch_bounds__(CTM_THREADS) void k_ct_sweep_m(Geo g, const double 
 #endif
 #define CTX_ROWS (CTX_THREADS / 64)
 template <int SC>
-__global__ __launch_bounds__(CTX_THREADS) void k_ct_sweep_x(Geo g, const double *__restrict__ t1i,
-                                                            const double *__restrict__ t2i,
-                                                            const double *__restrict__ ai, double *__restrict__ t1o,
-                                                            double *__restrict__ t2o, double *__restrict__ ao,
-                                                            const real *__restrict__ vel,
-                                                            const real *__restrict__ db1, int GS1, int VS2, double dt,
-                                                            int ntx, int mc, Box bt1, Box ba1, Box bt2, Box ba2) {
+__device__ __forceinline__ void ct_sweep_x(BLOCK_COORDS, Geo g, const double *__restrict__ t1i,
+                                           const double *__restrict__ t2i, const double *__restrict__ ai,
+                                           double *__restrict__ t1o, double *__restrict__ t2o,
+                                           double *__restrict__ ao, const real *__restrict__ vel,
+                                           const real *__restrict__ db1, int GS1, int VS2, double dt, int ntx, int mc,
+                                           Box bt1, Box ba1, Box bt2, Box ba2) {
   constexpr int T1 = CtComp<0>::T1, T2 = CtComp<0>::T2;
   __shared__ real fl[CTS_CHUNK + 1][2][CTX_ROWS][64];
   const int lane = (int)threadIdx.x & 63, row = (int)threadIdx.x >> 6;
@@ -583,6 +580,33 @@ __global__ __launch_bounds__(CTX_THREADS) void k_ct_sweep_x(Geo g, const double 
                     fl[s][0][row - 1][lane], fl[s][1][row][lane], fl[s][1][row][lane - 1], fl[s - 1][1][row][lane],
                     bt1, ba1, bt2, ba2);
   }
+}
+
+// Arguments of a CT sweep: fields t1, t2 and along the axis, in and out, the
+// sweep velocity and width, the strides of the averages and the index boxes.
+struct CtArgs {
+  const double *t1i, *t2i, *ai;
+  double *t1o, *t2o, *ao;
+  const real *vel, *db1;
+  int vs1, gs1, vs2, gs2;
+  double dt;
+  int ntx, mc;
+  Box bt1, ba1, bt2, ba2;
+};
+// block b of the sweep along AX, of a grid gx blocks wide
+template <int AX, int SC>
+__device__ __forceinline__ void ct_block(const dim3 &b, const dim3 &gr, const dim3 &t, const Geo &g, const CtArgs &a) {
+  if constexpr (AX == 0)
+    ct_sweep_x<SC>(b, gr, t, g, a.t1i, a.t2i, a.ai, a.t1o, a.t2o, a.ao, a.vel, a.db1, a.gs1, a.vs2, a.dt, a.ntx, a.mc,
+                   a.bt1, a.ba1, a.bt2, a.ba2);
+  else
+    ct_sweep_m<AX, SC>(b, gr, t, g, a.t1i, a.t2i, a.ai, a.t1o, a.t2o, a.ao, a.vel, a.db1, a.vs1, a.gs1, a.vs2, a.gs2,
+                       a.dt, a.ntx, a.mc, a.bt1, a.ba1, a.bt2, a.ba2);
+}
+#define CT_THREADS(AX) ((AX) == 0 ? CTX_THREADS : CTM_THREADS)
+template <int AX, int SC>
+__global__ __launch_bounds__(CT_THREADS(AX)) void k_ct_sweep(Geo g, CtArgs a) {
+  ct_block<AX, SC>(dim3(blockIdx.x, 0, blockIdx.z), dim3(gridDim.x, 1, gridDim.z), dim3(threadIdx.x, 0, 0), g, a);
 }
 
 // Face-averaged sweep velocity of the mass/energy fluxes (xremap.f90:492-493)
@@ -1007,16 +1031,13 @@ __device__ __forceinline__ acc rke_edge(acc vs, acc vp, acc flm, acc fl, acc flp
 #define MOMX_OUT 62
 #define MOMX_OUT_RKE 61
 template <bool RKE, bool LASTSW>
-__global__ __launch_bounds__(BX * BY) void k_mom_remap_x(Geo g, Box b, const real *__restrict__ vx,
-                                                         const real *__restrict__ vy, const real *__restrict__ vz,
-                                                         const real *__restrict__ vel1,
-                                                         const real *__restrict__ db1,
-                                                         const real *__restrict__ rho1,
-                                                         const real *__restrict__ cv1,
-                                                         const real *__restrict__ cv2,
-                                                         const real *__restrict__ dm, real *__restrict__ vxo,
-                                                         real *__restrict__ vyo, real *__restrict__ vzo, double dt,
-                                                         RkeOut rk) {
+__device__ __forceinline__ void mom_remap_x(BLOCK_COORDS, Geo g, Box b,
+                                            const real *__restrict__ vx, const real *__restrict__ vy,
+                                            const real *__restrict__ vz, const real *__restrict__ vel1,
+                                            const real *__restrict__ db1, const real *__restrict__ rho1,
+                                            const real *__restrict__ cv1, const real *__restrict__ cv2,
+                                            const real *__restrict__ dm, real *__restrict__ vxo,
+                                            real *__restrict__ vyo, real *__restrict__ vzo, double dt, RkeOut rk) {
   const int lane = (int)threadIdx.x;  // BX = 64: threadIdx.y is the wave
   const int wq = b.x1 - b.x0 + 1;
   const int npts = wq * (b.y1 - b.y0 + 1);
@@ -1130,16 +1151,13 @@ __global__ __launch_bounds__(BX * BY) void k_mom_remap_x(Geo g, Box b, const rea
 // march: the term of the edge at m-1 needs the flux velocity at m, so a
 // chunk runs one point past its last node when that node's edge exists.
 template <int M, bool RKE, bool LASTSW>
-__global__ __launch_bounds__(BX * BY) void k_mom_remap_m(Geo g, Box b, const real *__restrict__ vx,
-                                                         const real *__restrict__ vy, const real *__restrict__ vz,
-                                                         const real *__restrict__ vel1,
-                                                         const real *__restrict__ db1,
-                                                         const real *__restrict__ rho1,
-                                                         const real *__restrict__ cv1,
-                                                         const real *__restrict__ cv2,
-                                                         const real *__restrict__ dm, real *__restrict__ vxo,
-                                                         real *__restrict__ vyo, real *__restrict__ vzo, double dt,
-                                                         RkeOut rk) {
+__device__ __forceinline__ void mom_remap_m(BLOCK_COORDS, Geo g, Box b,
+                                            const real *__restrict__ vx, const real *__restrict__ vy,
+                                            const real *__restrict__ vz, const real *__restrict__ vel1,
+                                            const real *__restrict__ db1, const real *__restrict__ rho1,
+                                            const real *__restrict__ cv1, const real *__restrict__ cv2,
+                                            const real *__restrict__ dm, real *__restrict__ vxo,
+                                            real *__restrict__ vyo, real *__restrict__ vzo, double dt, RkeOut rk) {
   MCOLUMN(M, b, i, p, m0, m1)
   const int MS = M == 2 ? g.sz : g.sy;
   const int nM = g.n(M), nP = g.n(M == 2 ? 1 : 2);
@@ -1253,6 +1271,59 @@ __global__ __launch_bounds__(BX * BY) void k_mom_remap_m(Geo g, Box b, const rea
       dpp = dp;
     }
     dp = dm_;
+  }
+}
+
+// Arguments of a momentum remap over box b.
+struct MomArgs {
+  Box b;
+  const real *vx, *vy, *vz, *vel1, *db1, *rho1, *cv1, *cv2, *dm;
+  real *vxo, *vyo, *vzo;
+  double dt;
+  RkeOut rk;
+};
+template <int AX, bool RKE, bool LASTSW>
+__device__ __forceinline__ void mom_block(const dim3 &b, const dim3 &gr, const dim3 &t, const Geo &g,
+                                          const MomArgs &a) {
+  if constexpr (AX == 0)
+    mom_remap_x<RKE, LASTSW>(b, gr, t, g, a.b, a.vx, a.vy, a.vz, a.vel1, a.db1, a.rho1, a.cv1, a.cv2, a.dm, a.vxo,
+                             a.vyo, a.vzo, a.dt, a.rk);
+  else
+    mom_remap_m<AX, RKE, LASTSW>(b, gr, t, g, a.b, a.vx, a.vy, a.vz, a.vel1, a.db1, a.rho1, a.cv1, a.cv2, a.dm, a.vxo,
+                                 a.vyo, a.vzo, a.dt, a.rk);
+}
+template <int AX, bool RKE, bool LASTSW>
+__global__ __launch_bounds__(BX * BY) void k_mom_remap(Geo g, MomArgs a) {
+  mom_block<AX, RKE, LASTSW>(dim3(blockIdx.x, 0, blockIdx.z), dim3(gridDim.x, 1, gridDim.z),
+                             dim3(threadIdx.x, threadIdx.y, 0), g, a);
+}
+
+// The momentum remap and the CT sweep of one sweep in one launch: neither
+// reads what the other writes, and on small grids each leaves most of the chip
+// idle behind its chains of loads.  The first blocks take the momentum remap
+// (an x sweep's block two of its tiles), the rest the CT sweep.
+//
+// Runs with the two apart and together: 64^3 30.3 -> 29.0 ms (100 steps),
+// 97 x 61 x 130 37.9 -> 36.9 (50), 64 x 64 x 128 FP32 27.5 -> 26.6 (50),
+// 45 x 37 x 41 9.9 -> 9.4 (30).  Where both fill the chip FP32 still gains, by the
+// tail of one under the head of the other (192^3 339.4 -> 337.4 ms), and FP64,
+// at the bandwidth of a copy in both, does not (256^3 1003.8 -> 1006.8).
+#define MOM_CT_BLOCKS 4096
+static inline bool mom_ct_together(unsigned blocks) {
+  return sizeof(acc) == sizeof(float) || blocks <= MOM_CT_BLOCKS;
+}
+template <int AX, int SC>
+__global__ __launch_bounds__(CT_THREADS(AX)) void k_mom_ct(Geo g, MomArgs m, dim3 mg, CtArgs c, dim3 cg) {
+  constexpr unsigned PER = CT_THREADS(AX) / (BX * BY);  // momentum tiles per block
+  const unsigned mb = (mg.x * mg.z + PER - 1) / PER;
+  const unsigned t = threadIdx.x;
+  if (blockIdx.x < mb) {
+    const unsigned q = blockIdx.x * PER + t / (BX * BY);
+    if (q >= mg.x * mg.z) return;
+    mom_block<AX, false, (SC < 0)>(dim3(q % mg.x, 0, q / mg.x), mg, dim3(t % BX, t / BX % BY, 0), g, m);
+  } else {
+    const unsigned q = blockIdx.x - mb;
+    ct_block<AX, SC>(dim3(q % cg.x, 0, q / cg.x), cg, dim3(t, 0, 0), g, c);
   }
 }
 

@@ -474,7 +474,8 @@ int strides(int ax) { return ax == 0 ? 1 : (ax == 1 ? S.sy : S.sz); }
 // remap.f90:44-67 folded in).  sc = -1 (last predictor sweep): out gets B
 // back (remap.f90:102-125 folded in).
 template <int AX>
-int ct_sweep(const double *const in[3], double *const out[3], const real *vel, const real *db1, double dt, int sc) {
+CtArgs ct_args(const double *const in[3], double *const out[3], const real *vel, const real *db1, double dt,
+               dim3 *grid) {
   const int N[3] = {nx(), ny(), nz()};
   const Box ub = mkbox(0, N[0] + 1, 0, N[1] + 1, 0, N[2] + 1);
   // (transverse field t, velocity-average axis, geometry-average axis, box_t, box_a) x 2
@@ -493,41 +494,33 @@ int ct_sweep(const double *const in[3], double *const out[3], const real *vel, c
     t1 = 0; va1 = 1; ga1 = 0;  // vz_bx_flux
     t2 = 1; va2 = 0; ga2 = 1;  // vz_by_flux
   }
-  const dim3 blk(CTX_THREADS, 1, 1);
-  if constexpr (AX == 0) {
-    // x sweep: va1 = z and ga2 = z (see the flux table above); tiles of
-    // CTX_W points in x by CTX_ROWS - 1 rows in y, marching in z
-    const int ntx = (N[0] + 5 + CTX_W - 1) / CTX_W, nty = (N[1] + 5 + CTX_ROWS - 2) / (CTX_ROWS - 1);
-    const int mc = cts_chunk((unsigned)(ntx * nty), N[2] + 5);
-    const dim3 grid((unsigned)(ntx * nty), 1, (unsigned)((N[2] + 4 + mc) / mc));
-    if (sc > 0)
-      LAUNCH("ct_sweep", k_ct_sweep_x<1>, grid, blk, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX], vel,
-             db1, strides(ga1), strides(va2), dt, ntx, mc, bt1, ba1, bt2, ba2);
-    else if (sc < 0)
-      LAUNCH("ct_sweep", k_ct_sweep_x<-1>, grid, blk, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX], vel,
-             db1, strides(ga1), strides(va2), dt, ntx, mc, bt1, ba1, bt2, ba2);
-    else
-      LAUNCH("ct_sweep", k_ct_sweep_x<0>, grid, blk, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX], vel,
-             db1, strides(ga1), strides(va2), dt, ntx, mc, bt1, ba1, bt2, ba2);
-  } else {
-    // y and z sweeps march along the sweep axis; tiles of CTM_XW - 1 points
-    // in x by CTM_ROWS - 1 rows along the other transverse axis
-    const int P = AX == 2 ? 1 : 2;
-    const int ntx = (N[0] + 5 + CTM_XW - 2) / (CTM_XW - 1), nty = (N[P] + 5 + CTM_ROWS - 2) / (CTM_ROWS - 1);
-    const int mc = cts_chunk((unsigned)(ntx * nty), N[AX] + 5);
-    const dim3 grid((unsigned)(ntx * nty), 1, (unsigned)((N[AX] + 4 + mc) / mc));
-    const dim3 blkm(CTM_THREADS, 1, 1);
-    if (sc > 0)
-      LAUNCH("ct_sweep", (k_ct_sweep_m<AX, 1>), grid, blkm, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX],
-             vel, db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, mc, bt1, ba1, bt2, ba2);
-    else if (sc < 0)
-      LAUNCH("ct_sweep", (k_ct_sweep_m<AX, -1>), grid, blkm, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX],
-             vel, db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, mc, bt1, ba1, bt2, ba2);
-    else
-      LAUNCH("ct_sweep", (k_ct_sweep_m<AX, 0>), grid, blkm, S.g, in[t1], in[t2], in[AX], out[t1], out[t2], out[AX],
-             vel, db1, strides(va1), strides(ga1), strides(va2), strides(ga2), dt, ntx, mc, bt1, ba1, bt2, ba2);
-  }
+  // x sweep: va1 = z and ga2 = z (see the flux table above); tiles of CTX_W
+  // points in x by CTX_ROWS - 1 rows in y, marching in z.  y and z sweeps march
+  // along the sweep axis; tiles of CTM_XW - 1 points in x by CTM_ROWS - 1 rows
+  // along the other transverse axis.
+  const int P = AX == 0 ? 1 : 3 - AX, march = AX == 0 ? 2 : AX;
+  const int w = AX == 0 ? CTX_W : CTM_XW - 1, rows = (AX == 0 ? CTX_ROWS : CTM_ROWS) - 1;
+  const int ntx = (N[0] + 5 + w - 1) / w, nty = (N[P] + 5 + rows - 1) / rows;
+  const int mc = cts_chunk((unsigned)(ntx * nty), N[march] + 5);
+  *grid = dim3((unsigned)(ntx * nty), 1, (unsigned)((N[march] + 4 + mc) / mc));
+  return CtArgs{in[t1],       in[t2],       in[AX],       out[t1],      out[t2], out[AX], vel, db1, strides(va1),
+                strides(ga1), strides(va2), strides(ga2), dt,           ntx,     mc,      bt1, ba1, bt2,
+                ba2};
+}
+// sc: 1 the first sweep of a remap, -1 the last, 0 between
+template <int AX>
+int ct_launch(const CtArgs &a, dim3 grid, int sc) {
+  const dim3 blk(CT_THREADS(AX), 1, 1);
+  if (sc > 0) LAUNCH("ct_sweep", (k_ct_sweep<AX, 1>), grid, blk, S.g, a);
+  else if (sc < 0) LAUNCH("ct_sweep", (k_ct_sweep<AX, -1>), grid, blk, S.g, a);
+  else LAUNCH("ct_sweep", (k_ct_sweep<AX, 0>), grid, blk, S.g, a);
   return 0;
+}
+template <int AX>
+int ct_sweep(const double *const in[3], double *const out[3], const real *vel, const real *db1, double dt, int sc) {
+  dim3 grid;
+  const CtArgs a = ct_args<AX>(in, out, vel, db1, dt, &grid);
+  return ct_launch<AX>(a, grid, sc);
 }
 
 // the face arrays a and the spare EMF arrays swap roles (the CT output went
@@ -608,13 +601,11 @@ int sweep_full(double dt, int q) {
   const bool first = q == 0, last = q == 2;
   const real *db1 = remap_db1(AX), *cv1 = remap_vol(q), *cv2 = last ? nullptr : remap_vol(q + 1);
   int rc;
-  {
-    const double *const B[3] = {S.bx, S.by, S.bz};
-    double *const spare[3] = {S.fxr, S.fyr, S.fzr};
-    rc = ct_sweep<AX>(B, spare, vel, db1, dt, first ? 1 : (last ? -1 : 0));
-    if (rc) return rc;
-    swap_spare(S.bx, S.by, S.bz);
-  }
+  const int sc = first ? 1 : (last ? -1 : 0);
+  const double *const B[3] = {S.bx, S.by, S.bz};
+  double *const spare[3] = {S.fxr, S.fyr, S.fzr};
+  dim3 cg;
+  const CtArgs ct = ct_args<AX>(B, spare, vel, db1, dt, &cg);
   int hi[3] = {N[0] + 1, N[1] + 1, N[2] + 1};
   hi[AX] = N[AX];
   Box mb = mkbox(0, hi[0], 0, hi[1], 0, hi[2]);
@@ -657,30 +648,38 @@ int sweep_full(double dt, int q) {
     // rho_alt); the new velocities land in the flux arrays, which then swap
     // roles with the velocity arrays
     Box xb = full_box();
+    dim3 mg;
     if constexpr (AX == 0) {
       const unsigned pb = wave_blocks((long)(xb.x1 - xb.x0 + 1) * (xb.y1 - xb.y0 + 1),
                                       S.delta_ke ? MOMX_OUT_RKE : MOMX_OUT);
       xb.zc = march_chunk(pb, xb.z1 - xb.z0 + 1);
-      const dim3 gx(pb, 1, (unsigned)((xb.z1 - xb.z0 + xb.zc) / xb.zc));
-#define MOM_REMAP(R, L)                                                                                          \
-  LAUNCH("mom_remap", (k_mom_remap_x<R, L>), gx, box_block(), S.g, xb, S.vx, S.vy, S.vz, vel, db1, S.rho, cv1, \
-         cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk)
-      if (S.delta_ke && last) MOM_REMAP(true, true);
-      else if (S.delta_ke) MOM_REMAP(true, false);
-      else if (last) MOM_REMAP(false, true);
-      else MOM_REMAP(false, false);
-#undef MOM_REMAP
+      mg = dim3(pb, 1, (unsigned)((xb.z1 - xb.z0 + xb.zc) / xb.zc));
     } else {
       xb = marched(xb, AX);
-#define MOM_REMAP(R, L)                                                                                               \
-  LAUNCH("mom_remap", (k_mom_remap_m<AX, R, L>), zchunk_grid(march_box(xb, AX)), box_block(), S.g, xb, S.vx, S.vy,  \
-         S.vz, vel, db1, S.rho, cv1, cv2, S.dm, S.Fx, S.Fy, S.Fz, dt, S.rk)
+      mg = zchunk_grid(march_box(xb, AX));
+    }
+    const MomArgs mo = {xb,   S.vx, S.vy, S.vz, vel, db1,  S.rho, cv1, cv2,
+                        S.dm, S.Fx, S.Fy, S.Fz, dt,  S.rk};
+    // together with the CT sweep, whose turn may come anywhere between the
+    // geometry and the boundary fill
+    const unsigned per = CT_THREADS(AX) / (BX * BY), nm = (mg.x * mg.z + per - 1) / per, nc = cg.x * cg.z;
+    if (!S.delta_ke && mom_ct_together(nm + nc)) {
+#define MOM_CT(SC) LAUNCH("mom_ct", (k_mom_ct<AX, SC>), dim3(nm + nc), dim3(CT_THREADS(AX)), S.g, mo, mg, ct, cg)
+      if (sc > 0) MOM_CT(1);
+      else if (sc < 0) MOM_CT(-1);
+      else MOM_CT(0);
+#undef MOM_CT
+    } else {
+#define MOM_REMAP(R, L) LAUNCH("mom_remap", (k_mom_remap<AX, R, L>), mg, box_block(), S.g, mo)
       if (S.delta_ke && last) MOM_REMAP(true, true);
       else if (S.delta_ke) MOM_REMAP(true, false);
       else if (last) MOM_REMAP(false, true);
       else MOM_REMAP(false, false);
 #undef MOM_REMAP
+      rc = ct_launch<AX>(ct, cg, sc);
+      if (rc) return rc;
     }
+    swap_spare(S.bx, S.by, S.bz);
     // rke: this sweep's edge terms into delta_ke
     if (S.delta_ke) LAUNCH_BOX("rke_gather", k_rke_gather<AX>, interior(), S.rk, S.delta_ke);
     real *tv;

@@ -847,13 +847,20 @@ int open_bcs() {
 
 // the reference STOPs on an inverted temperature bracket (neutral.f90:172-175):
 // report it once the work queued so far has run, and clear the flag
-int check_neutral_fault(const char *where) {
+// (the flag is a word of the pinned mirror).  folded: a fold was queued after
+// the last neutral_fraction, and its ticket says that it has run; a 45 x 37 x 41
+// step waited some 15 us for the end of the remap instead.
+int check_neutral_fault(const char *where, bool folded) {
   if (!S.nf_flag) return 0;
-  int h = 0;
-  HIPCHK(hipMemcpyAsync(&h, S.nf_flag, sizeof(int), hipMemcpyDeviceToHost, S.stream));
-  HIPCHK(hipStreamSynchronize(S.stream));
-  if (!h) return 0;
-  HIPCHK(hipMemsetAsync(S.nf_flag, 0, sizeof(int), S.stream));
+  if (folded) {
+    const int rc = read_scalars(0, 0, nullptr);
+    if (rc) return rc;
+  } else {
+    HIPCHK(hipStreamSynchronize(S.stream));
+  }
+  volatile int *flag = S.nf_flag;
+  if (!*flag) return 0;
+  *flag = 0;
   return fail(LARE_F_TBOUNDS, "%s: neutral_fraction temperature bracket inverted (energy <= 0 in some cell)", where);
 }
 
@@ -921,7 +928,9 @@ int resist_rk4_substep() {
   return final_reduce(gr, 1, 0, 9, 1);
 }
 
-int lagrangian_step() {
+// xi_known: xi_n is that of the density and energy on entry, which the first
+// resistive substep finds unchanged
+int lagrangian_step(bool xi_known) {
   const int N0 = nx(), N1 = ny(), N2 = nz();
   LagArgs a = lag_args();  // dt = previous step's dt (Q1)
   {
@@ -995,7 +1004,7 @@ int lagrangian_step() {
     for (int sc = 1; sc <= substeps; ++sc) {
       // eta_calc runs inside the substep kernels; neutral_fraction and
       // perpendicular_resistivity read nothing it writes (lagran.F90:146-149)
-      if (S.pi_eos) {
+      if (S.pi_eos && !(sc == 1 && xi_known)) {
         rc = neutral_fraction(S.energy, TMODE_DIRECT);
         if (rc) return rc;
       }
@@ -1388,9 +1397,6 @@ int api_init(const lare_grid *grid, const lare_params *params) {
     int rc = dalloc(&S.xi);
     if (!rc && params->cowling_resistivity) rc = dalloc(&S.eta_perp);
     if (rc) return rc;
-    HIPCHK(hipMalloc((void **)&S.nf_flag, sizeof(int)));
-    S.allocs.push_back(S.nf_flag);
-    HIPCHK(hipMemsetAsync(S.nf_flag, 0, sizeof(int), S.stream));
   }
   if (params->boris) {
     int rc = dalloc(&S.gamma_boris);
@@ -1423,8 +1429,9 @@ int api_init(const lare_grid *grid, const lare_params *params) {
   HIPCHK(hipMalloc((void **)&S.partial, sizeof(double) * (S.partial_cap + RED_ROWS * RED_MAXV)));
   HIPCHK(hipMalloc((void **)&S.dscal, sizeof(double) * 16));
   HIPCHK(hipMemset(S.dscal, 0, sizeof(double) * 16));
-  HIPCHK(hipHostMalloc((void **)&S.hscal, sizeof(double) * 17));
-  memset(S.hscal, 0, sizeof(double) * 17);
+  HIPCHK(hipHostMalloc((void **)&S.hscal, sizeof(double) * 18));
+  memset(S.hscal, 0, sizeof(double) * 18);
+  if (pi) S.nf_flag = (int *)(S.hscal + 17);
   S.ticket = 0;
   HIPCHK(hipStreamSynchronize(S.stream));
   S.dt = S.dt2 = S.dtr = S.time = 0.0;
@@ -1496,9 +1503,9 @@ int api_set_scalars(const lare_scalars *in) {
 
 int api_lagrangian_step(void) {
   REQUIRE_LOADED();
-  int rc = lagrangian_step();
+  int rc = lagrangian_step(false);
   if (rc) return rc;
-  return check_neutral_fault("lagrangian_step");
+  return check_neutral_fault("lagrangian_step", false);
 }
 
 int api_eulerian_remap(int32_t step) {
@@ -1518,7 +1525,7 @@ int api_conduct_heat(void) {
   if (rc) return rc;
   rc = heat_conduct_sts2(0);
   if (rc) return rc;
-  return check_neutral_fault("conduct_heat");
+  return check_neutral_fault("conduct_heat", false);
 }
 
 int api_boundary_conditions(void) {
@@ -1531,7 +1538,7 @@ int api_neutral_fraction(void) {
   if (!S.pi_eos) return fail(LARE_E_STATE, "neutral_fraction needs eos_number EOS_ION or EOS_PI");
   int rc = neutral_fraction(S.energy, TMODE_DIRECT);
   if (rc) return rc;
-  return check_neutral_fault("neutral_fraction");
+  return check_neutral_fault("neutral_fraction", false);
 }
 
 int api_perpendicular_resistivity(void) {
@@ -1608,7 +1615,7 @@ int api_step(int32_t step, double *dt, double *time) {
     rc = neutral_fraction(S.energy, TMODE_DIRECT);
     if (rc) return rc;
   }
-  rc = lagrangian_step();
+  rc = lagrangian_step(true);
   if (rc) return rc;
   rc = eulerian_remap(step, false);
   if (rc) return rc;
@@ -1618,7 +1625,9 @@ int api_step(int32_t step, double *dt, double *time) {
   }
   rc = eta_calc();
   if (rc) return rc;
-  rc = check_neutral_fault("step");
+  // the fold of the corrector's heating total comes after the step's last
+  // neutral_fraction
+  rc = check_neutral_fault("step", true);
   if (rc) return rc;
   if (!isfinite(S.dt) || (S.dt <= 0.0 && !S.p.restart))
     return fail(LARE_F_NONFINITE, "step %d: invalid dt %g", step, S.dt);

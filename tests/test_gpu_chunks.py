@@ -1,6 +1,7 @@
 """Full steps against the CPU restatement on grids for which the marching
 kernels take chunks of 3 points and of 6 to 8 (1, 2, 4 and 5: test_gpu_march.py),
-with a short last chunk: every element of every state array."""
+with a short last chunk, and on one on which every sweep's momentum remap and CT
+sweep are launches of their own: every element of every state array."""
 import numpy as np
 import pytest
 
@@ -23,6 +24,26 @@ def test_steps_at_the_other_chunks(n):
         d.boundary_conditions()
         d.eta_calc()
     assert dev.step(1) == orc.step(1)
+    fd, fo = dev.fields(), orc.fields()
+    for name in STATE:
+        assert np.array_equal(getattr(fd, name), getattr(fo, name)), name
+    dev.close()
+    orc.close()
+
+
+def test_sweeps_of_large_grids():
+    from lare3d_amd.device import Device
+    from oracle.oracle import Oracle
+    grid, params, f = configs.harris(192, ny=190, nz=190)
+    dev, orc = Device(grid, params, f), Oracle(grid, params, f)
+    print("\n[case] sweeps apart 192x190x190", flush=True)
+    for d in (dev, orc):
+        d.boundary_conditions()
+        d.eta_calc()
+    dev.profile(True)
+    assert dev.step(1) == orc.step(1)
+    names = dev.kernel_stats()
+    assert "mom_remap" in names and "ct_sweep" in names and "mom_ct" not in names
     fd, fo = dev.fields(), orc.fields()
     for name in STATE:
         assert np.array_equal(getattr(fd, name), getattr(fo, name)), name

@@ -11,8 +11,8 @@
 //   k_resist          resistive sub-cycle (:1176-1635): eta_calc, rkstep,
 //                     bstep and the ohmic heating in one pass
 //   k_eta             eta_calc after the remap (lare3d.f90:87)
-//   predictor energy/pressure (:234-249): in the predictor remap's last
-//                     geometry pass (k_geom<AX, 1>, remap.hpp)
+//   predictor energy/pressure (:234-249): in the predictor remap's
+//                     geometry pass (k_geom_pred, remap.hpp)
 //   k_force           f_visc (:745-789) + grad p + J x B (half-step B)
 //                     + gravity -> v1 at nodes 0..n (:251-387)
 //   k_shock_corr      shock_heating (:861-937) fused with the corrector

@@ -1303,6 +1303,8 @@ struct FtnLayout {
 // serve the next plane, and a block's partial covers its chunk, so at 64^3
 // one block folds the 561 partials (one per plane and tile would be 1105,
 // folded in two launches).
+// Plain divisions: a quotient by Recip that should be infinite is NaN, which
+// the largest |div B| would drop.
 template <class R>
 struct MassQuad {
   R r;          // rho of (i, j)
@@ -1334,7 +1336,6 @@ __global__ __launch_bounds__(BX * BY) void k_energy(Geo g, Box b, L lay, const R
     const bool cell = i >= 1 && j >= 1;
     const double dx = g.dxb[i], dy = g.dyb[j], dx1 = g.dxb[i + 1], dy1 = g.dyb[j + 1];
     const double area[4] = {dx * dy, dx1 * dy, dx * dy1, dx1 * dy1};
-    const Recip<double> rx = recip(dx), ry = recip(dy);
     double wij = 1.0;  // halves on the boundary nodes
     if (i == 0 || i == g.nx) wij = 0.5;
     if (j == 0 || j == g.ny) wij = wij * 0.5;
@@ -1356,7 +1357,7 @@ __global__ __launch_bounds__(BX * BY) void k_energy(Geo g, Box b, L lay, const R
           const double cv = area[0] * dz;
           v[0] = v[0] + w1 * cv;
           v[2] = v[2] + energy[lay.cell(i, j, k)] * lo.r * cv;
-          const double d = (bx0 - bxm) / rx + (by0 - bym) / ry + (bz0 - bzm) / recip(dz);
+          const double d = (bx0 - bxm) / dx + (by0 - bym) / dy + (bz0 - bzm) / dz;
           v[3] = dmin(v[3], -(fabs(d) * dmin(dmin(dx, dy), dz)));
         }
         bzm = bz0;
@@ -1367,7 +1368,7 @@ __global__ __launch_bounds__(BX * BY) void k_energy(Geo g, Box b, L lay, const R
       double cvv = area[0] * dz;
 #pragma unroll
       for (int q = 1; q < 8; ++q) cvv = cvv + (q < 4 ? area[q] * dz : area[q - 4] * dz1);
-      rv = rv / recip(cvv);
+      rv = rv / cvv;
       const int n = lay.node(i, j, k);
       double w1 = rv * (cvv * 0.125) * (vx[n] * vx[n] + vy[n] * vy[n] + vz[n] * vz[n]) * wij;
       if (k == 0 || k == g.nz) w1 = w1 * 0.5;

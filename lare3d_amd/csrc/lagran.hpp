@@ -132,13 +132,14 @@ __global__ __launch_bounds__(BX * BY) void k_vertex_prep(Geo g, Box b, const rea
     acc sc = cvs[0];
 #pragma unroll
     for (int q = 1; q < 8; ++q) sc = sc + cvs[q];
-    const Recip<acc> rsc = recip(sc);
-    rho_v[c] = s / rsc;
+    rho_v[c] = s / recip(sc);
     acc scs = lo.cs[0] * cvs[0];
 #pragma unroll
     for (int q = 1; q < 8; ++q) scs = scs + (q < 4 ? lo.cs[q] : hi.cs[q - 4]) * cvs[q];
-    // (scs / 8) / (sc / 8): the eighths are exact and cancel
-    cs_v[c] = scs / rsc;
+    // (scs / 8) / (sc / 8): the eighths are exact and cancel.  A plain
+    // division: an edge takes the smaller speed of its nodes, whatever the
+    // other one is, unless that is NaN
+    cs_v[c] = scs / sc;
     lo = hi;
   }
 }
@@ -394,9 +395,10 @@ __global__ __launch_bounds__(BX * BY) void k_visc_dt(Geo g, Box bx0, const real 
           if (a.write_gb) gbo[c] = (real)g_b;
           g_b = (real)g_b;
         }
-        const Recip<double> rr = recip(rho0);
-        const double cs2 = (a.gamma * (double)p + g_b * w1) / rr;
-        const double c_visc2 = (double)pv / rr;
+        // plain divisions: an infinite speed makes dt 0, where the NaN of a
+        // Recip would be dropped by the minimum
+        const double cs2 = (a.gamma * (double)p + g_b * w1) / rho0;
+        const double c_visc2 = pv / rho0;
         const double dxb = g.dxb[i], dyb = g.dyb[j], dzb = g.dzb[k];
         const double length = dmin(dmin(dxb, dyb), dzb);
         const double dt1 = length / (root(c_visc2) + root(cs2 + c_visc2));

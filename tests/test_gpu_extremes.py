@@ -1,10 +1,11 @@
 """Infinities given to the diagnostics and quantities that leave the range of the
-type, against the CPU restatement.  What is compared is whether a value is
-infinite, so equality is exact."""
+type, against the CPU restatement.  What is compared is a time step, or
+whether a value is finite, so equality is exact."""
 import numpy as np
 import pytest
 
 from lare3d_amd import configs
+from lare3d_amd.abi import DeviceError
 from tests.test_zz_no_alloc import _noalloc
 
 pytestmark = pytest.mark.gpu
@@ -30,3 +31,49 @@ def test_infinite_diagnostics(field, value):
         assert [np.isinf(x) for x in got[0]] == [np.isinf(x) for x in want]
         assert not np.isnan(got[0]).any()
         assert np.isinf(got[1]) == np.isinf(wdiv)
+
+
+def _pair(cfg):
+    from lare3d_amd.device import Device
+    from oracle.oracle import Oracle
+    dev, orc = Device(*cfg), Oracle(*cfg)
+    for d in (dev, orc):
+        d.set_scalars(dt=1.0e-2)  # of the step before, which the edge viscosity looks at
+        d.boundary_conditions()
+        d.eta_calc()
+    return dev, orc
+
+
+def _thin_cell(b, visc):
+    """Density 1e-300 in one cell, a field b on one of its faces alone."""
+    grid, params, f = configs.orszag_tang(12)
+    params.visc1, params.visc2 = visc
+    f.rho[7, 7, 7] = 1e-300
+    f.by[...] = f.bz[...] = 0.0
+    f.bx[8, 7, 7] = b
+    return grid, params, f
+
+
+def test_infinite_speed_stops_the_step():
+    # b^2 / rho = 4e308 in set_dt, 1e308 with the face average of the cell
+    print("\n[case] infinite speed in set_dt", flush=True)
+    dev, orc = _pair(_thin_cell(2.0e4, (0.0, 0.0)))
+    assert orc.step(1)[0] == 0.0
+    with pytest.raises(DeviceError, match="invalid dt 0"):
+        dev.step(1)
+    dev.close()
+    orc.close()
+
+
+def test_infinite_speed_of_a_cell_stays_on_its_nodes():
+    # the cell's own speed is infinite: its edges to other nodes take theirs
+    print("\n[case] infinite speed of a cell", flush=True)
+    dev, orc = _pair(_thin_cell(1.0e5, (0.1, 0.5)))
+    for d in (dev, orc):
+        d.lagrangian_step()
+    assert dev.scalars().dt == orc.scalars().dt
+    for name in ("rho", "energy", "vx", "vy", "vz"):
+        a, b = dev.fields().interior(name), orc.fields().interior(name)
+        assert np.array_equal(np.isfinite(a), np.isfinite(b)), name
+    dev.close()
+    orc.close()

@@ -334,7 +334,9 @@ __device__ __forceinline__ acc edge_heat_v(acc dxb, acc dyb, acc dzb, acc cv, co
   h = h - (acc)0.25 * dxb * dyb * a3x * aa[9];
   h = h - (acc)0.25 * dxb * dyb * a3xy * aa[10];
   h = h - (acc)0.25 * dxb * dyb * a3y * aa[11];
-  return h / recip(cv);
+  // plain: the MAX(., 0) of the corrector makes the NaN of a Recip that
+  // overflows no heating at all
+  return h / cv;
 }
 
 // p_visc + visc_heat over cells 0..n+1; pressure p0 of lagran.F90:93 stored
@@ -745,7 +747,8 @@ __global__ __launch_bounds__(64 * RS_ROWS, RS_WAVES) void k_resist(Geo g, Box b,
         if (hot) {
           // curlb(c) + (c-X) + (c-Y) + (c-X-Y) + (c-Z) + (c-X-Z) + (c-Y-Z) + (c-X-Y-Z)
           const acc sq = pq[0] + pq[1] + pq[2] + pq[3] + mq[0] + mq[1] + mq[2] + mq[3];
-          const acc lh = sq * (acc)dt / recip((acc)8.0 * r_own);
+          // plain: the MAX(., 0) below would make a NaN zero
+          const acc lh = sq * (acc)dt / ((acc)8.0 * r_own);
           ohmic_dep[c] = od_own + lh;
           e = e + lh;
         }
@@ -1056,7 +1059,11 @@ __device__ __forceinline__ void store_node3(const Geo &g, int c, int i, int j, i
 // predictor momentum (lagran.F90:251-387) with fx/fy/fz_visc (:745-789)
 // recomputed here from alpha and v.  Without CAUCHY, B is the half-step
 // (predictor-remapped) face field; with CAUCHY, J and B come from the
-// cell-centred B1 cv1 (b1x..b1z) and cv1 of k_cauchy_b.
+// cell-centred B1 cv1 (b1x..b1z) and cv1 of k_cauchy_b.  Plain divisions but
+// for the current: an infinite velocity has to stay one (its cell ends with the
+// density 0 that the next step's state check names), and Recip's gained nothing
+// here or in k_shock_corr (100 steps at 256^3 997.9 ms with and without, 192^3
+// in FP32 336.1 and 337.3).
 template <bool CAUCHY>
 __global__ __launch_bounds__(BX * BY) void k_force(Geo g, Box b, const real *__restrict__ vx, const real *__restrict__ vy,
                         const real *__restrict__ vz, const real *__restrict__ pp,
@@ -1107,7 +1114,7 @@ __global__ __launch_bounds__(BX * BY) void k_force(Geo g, Box b, const real *__r
     const acc a4 = al2[c + Y + Z] * dxc * dzc;
     const acc a5 = a3lo * dxc * dyc;
     const acc a6 = a3hi * dxc * dyc;
-    const Recip<acc> cvv = recip((acc)0.125 * (acc)cv_sum8(g, i, j, k));
+    const acc cvv = (acc)0.125 * (acc)cv_sum8(g, i, j, k);
     acc fv[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
@@ -1122,13 +1129,13 @@ __global__ __launch_bounds__(BX * BY) void k_force(Geo g, Box b, const real *__r
     const acc ppxy = plo.pxy, ppxz = phi.px, ppyz = phi.py, ppxyz = phi.pxy;
     acc w1 = (p + ppy + ppz + ppyz) * q4;
     acc w2 = (ppx + ppxy + ppxz + ppxyz) * q4;
-    acc fx = -(w2 - w1) / rx;
+    acc fx = -(w2 - w1) / dxc;
     w1 = (p + ppx + ppz + ppxz) * q4;
     w2 = (ppy + ppxy + ppyz + ppxyz) * q4;
-    acc fy = -(w2 - w1) / ry;
+    acc fy = -(w2 - w1) / dyc;
     w1 = (p + ppx + ppy + ppxy) * q4;
     w2 = (ppz + ppxz + ppyz + ppxyz) * q4;
-    acc fz = -(w2 - w1) / rz;
+    acc fz = -(w2 - w1) / dzc;
     acc bxv, byv, bzv, jx, jy, jz;
     if (CAUCHY) {
       cauchy_jb(dxc, dyc, dzc, clo, chi, jx, jy, jz, bxv, byv, bzv);
@@ -1148,9 +1155,8 @@ __global__ __launch_bounds__(BX * BY) void k_force(Geo g, Box b, const real *__r
     const acc rv = rho_v[c];
     fz = fz - rv * (acc)g.grav[k];
     const acc h = (acc)dt2;
-    const Recip<acc> rrv = recip(rv);
-    const real w1x = u0[0] + h * (fv[0] + fx) / rrv, w1y = u0[1] + h * (fv[1] + fy) / rrv,
-               w1z = u0[2] + h * (fv[2] + fz) / rrv;
+    const real w1x = u0[0] + h * (fv[0] + fx) / rv, w1y = u0[1] + h * (fv[1] + fy) / rv,
+               w1z = u0[2] + h * (fv[2] + fz) / rv;
     if (wall) {
       store_node3(g, c, i, j, k, w1x, w1y, w1z, vx1, vy1, vz1);
     } else {
@@ -1195,7 +1201,7 @@ __global__ __launch_bounds__(BX * BY) void k_shock_corr(Geo g, Box b, const real
   if (j <= b.y1) {
     const int Y = g.sy, Z = g.sz;
     const bool column = i >= 1 && j >= 1;
-    const Recip<acc> rx = recip((acc)g.dxb[i]), ry = recip((acc)g.dyb[j]);
+    const acc dxb = (acc)g.dxb[i], dyb = (acc)g.dyb[j];
     const int cb = g.idx(i, j, k0) - Z;
     Node4 lx = node4(vx, cb, Y), ly = node4(vy, cb, Y), lz = node4(vz, cb, Y);
     Node4 lx1 = node4(vx1, cb, Y), ly1 = node4(vy1, cb, Y), lz1 = node4(vz1, cb, Y);
@@ -1214,7 +1220,7 @@ __global__ __launch_bounds__(BX * BY) void k_shock_corr(Geo g, Box b, const real
         EDGES(AAS)
 #undef AAS
         const acc a30 = al3[c], a3x = al3[c - 1], a3xy = al3[c - 1 - Y], a3y = al3[c - Y];
-        const acc vh = max0(edge_heat_v((acc)g.dxb[i], (acc)g.dyb[j], (acc)g.dzb[k], (acc)g.cv(i, j, k), alo, ahi, a30,
+        const acc vh = max0(edge_heat_v(dxb, dyb, (acc)g.dzb[k], (acc)g.cv(i, j, k), alo, ahi, a30,
                                         a3x, a3xy, a3y, aa));
         // face-averaged v1 (quad sums in the order c, c-Y, c-Z, c-Y-Z etc.;
         // node C = c, B = c-Y, D = c-X, A = c-X-Y)
@@ -1227,12 +1233,12 @@ __global__ __launch_bounds__(BX * BY) void k_shock_corr(Geo g, Box b, const real
         const acc vzbm = (lz1.c + lz1.d + lz1.b + lz1.a) * q4;
         const acc dta = (acc)dt;
         const acc dv =
-            ((vxb - vxbm) / rx + (vyb - vybm) / ry + (vzb - vzbm) / recip((acc)g.dzb[k])) * dta;
+            ((vxb - vxbm) / dxb + (vyb - vybm) / dyb + (vzb - vzbm) / (acc)g.dzb[k]) * dta;
         const acc r = rho[c];
         const acc e0 = clamp ? max0((acc)energy[c]) : (acc)energy[c];
-        const real e1 = e0 + (dta * vh - dv * pp[c]) / recip(r);
+        const real e1 = e0 + (dta * vh - dv * pp[c]) / r;
         visc_dep[c] = visc_dep[c] + dta * vh;
-        const real rn = r / recip((acc)1.0 + dv);
+        const real rn = r / ((acc)1.0 + dv);
         rho[c] = rn;
         if (COOL) {
           // a running average of the viscous heating is removed again, and

@@ -77,3 +77,39 @@ def test_infinite_speed_of_a_cell_stays_on_its_nodes():
         assert np.array_equal(np.isfinite(a), np.isfinite(b)), name
     dev.close()
     orc.close()
+
+
+def test_viscous_heating_beyond_the_range():
+    print("\n[case] viscous heating overflow", flush=True)
+    grid, params, f = configs.orszag_tang(12)
+    params.visc1, params.visc2 = 0.1, 0.5
+    f.vx[6, 6, 6] = 1.0e104  # density x (velocity difference)^3 overflows, its square does not
+    dev, orc = _pair((grid, params, f))
+    for d in (dev, orc):
+        d.lagrangian_step()
+    for name in ("rho", "energy", "vx", "vy", "vz", "visc_dep"):
+        a, b = dev.fields().interior(name), orc.fields().interior(name)
+        assert np.array_equal(np.isfinite(a), np.isfinite(b)), name
+    assert np.isinf(orc.fields().interior("energy")).any()
+    dev.close()
+    orc.close()
+
+
+def test_ohmic_heating_beyond_the_range():
+    print("\n[case] ohmic heating overflow", flush=True)
+    grid, params, f = configs.harris(12)
+    params.eta_background, params.eta0, params.visc1, params.visc2 = 1.0e7, 0.0, 0.0, 0.0
+    # a thin cell without a field of its own, in the current of its neighbours'
+    f.rho[6, 6, 6] = 1e-300
+    f.bx[...] = 1.0e10
+    f.bx[6:8, 6, 6] = f.by[6, 6:8, 6] = f.bz[6, 6, 6:8] = 0.0
+    dev, orc = _pair((grid, params, f))
+    for d in (dev, orc):
+        d.lagrangian_step()
+    assert dev.scalars().last_substeps == orc.scalars().last_substeps == 1
+    lost = ~np.isfinite(orc.fields().interior("ohmic_dep"))
+    assert lost.any()
+    for name in ("ohmic_dep", "energy"):
+        assert not np.isfinite(dev.fields().interior(name)[lost]).any(), name
+    dev.close()
+    orc.close()

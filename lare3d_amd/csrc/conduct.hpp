@@ -144,7 +144,7 @@ __global__ __launch_bounds__(BX * BY) void k_larsen(Geo g, Box b, const real *__
       if (i >= 1 && j >= 1 && k >= 1) {
         const double kappa1 = kappa_0 * L;
         const double n = dmin(r * (dx * dx), dmin(r * (dy * dy), r * (dz * dz)));
-        v[0] = dmin(v[0], n / (2.0 * kappa1 * temp));
+        v[0] = dmin(n / (2.0 * kappa1 * temp), v[0]);  // a NaN leaves v[0]
       }
       Tm = T;
       T = Tp;

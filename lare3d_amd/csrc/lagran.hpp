@@ -1366,7 +1366,7 @@ __global__ __launch_bounds__(BX * BY) void k_energy(Geo g, Box b, L lay, const R
           v[0] = v[0] + w1 * cv;
           v[2] = v[2] + energy[lay.cell(i, j, k)] * lo.r * cv;
           const double d = (bx0 - bxm) / dx + (by0 - bym) / dy + (bz0 - bzm) / dz;
-          v[3] = dmin(v[3], -(fabs(d) * dmin(dmin(dx, dy), dz)));
+          v[3] = dmin(-(fabs(d) * dmin(dmin(dx, dy), dz)), v[3]);  // a NaN leaves v[3]
         }
         bzm = bz0;
       }

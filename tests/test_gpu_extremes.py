@@ -113,3 +113,38 @@ def test_ohmic_heating_beyond_the_range():
         assert not np.isfinite(dev.fields().interior(name)[lost]).any(), name
     dev.close()
     orc.close()
+
+
+@pytest.mark.parametrize("k", range(8, 16))
+def test_negative_temperature_beside_the_step_limit(k):
+    """One plane above the cell that sets the conduction step limit (229 stages;
+    9 without it), a cell whose own limit is NaN."""
+    print(f"\n[case] conduction step limit beside NaN, k={k}", flush=True)
+    from lare3d_amd.device import Device
+    grid, params, f, dt = configs.arcade_conduction(64, 64, 64, s_target=9)
+    f.energy[20, 7, k] = 20.0 * f.energy.max()
+    f.energy[20, 7, k + 1] = -1.0
+    dev = Device(grid, params, f)
+    dev.set_scalars(dt=dt)
+    dev.boundary_conditions()
+    dev.conduct_heat()
+    assert dev.scalars().n_s_stages == 229
+    dev.close()
+
+
+@pytest.mark.parametrize("k", range(8, 16))
+def test_nan_beside_the_largest_divergence(k):
+    """One and two planes above the two cells with the largest |div B|, cells whose
+    own is NaN."""
+    print(f"\n[case] div B beside NaN, k={k}", flush=True)
+    from lare3d_amd.device import Device
+    grid, params, f = configs.orszag_tang(64)
+    f.bx[20, 7, k] += 100.0
+    want = []
+    for nan in (False, True):
+        if nan:
+            f.bz[19:21, 7, k + 2] = np.nan
+        dev = Device(grid, params, f)
+        want.append(dev.divb())
+        dev.close()
+    assert want[0] == want[1] > 1.0

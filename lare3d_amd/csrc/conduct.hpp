@@ -123,7 +123,6 @@ __global__ __launch_bounds__(BX * BY) void k_larsen(Geo g, Box b, const real *__
       else return tfac * energy[q];
     };
     const double dx = g.dxb[i], dy = g.dyb[j];
-    const Recip<double> rx = recip(dx), ry = recip(dy);
     const int c0 = g.idx(i, j, k0), Z = g.sz;
     double Tm = T_at(c0 - Z), T = T_at(c0);
     for (int k = k0; k <= k1; ++k) {
@@ -132,11 +131,12 @@ __global__ __launch_bounds__(BX * BY) void k_larsen(Geo g, Box b, const real *__
       const double temp = pow25(T);
       double L = 1.0;
       if (limiter_on) {
+        // plain divisions: a flux beyond the range makes the factor 0, not NaN
         const double q_fs = flux_limiter * 42.85 * r * pow15(T);
         const double q_fs2 = q_fs * q_fs;
-        const double q_spx = -kappa_0 * temp * (T_at(c + 1) - T_at(c - 1)) * 0.5 / rx;
-        const double q_spy = -kappa_0 * temp * (T_at(c + g.sy) - T_at(c - g.sy)) * 0.5 / ry;
-        const double q_spz = -kappa_0 * temp * (Tp - Tm) * 0.5 / recip(dz);
+        const double q_spx = -kappa_0 * temp * (T_at(c + 1) - T_at(c - 1)) * 0.5 / dx;
+        const double q_spy = -kappa_0 * temp * (T_at(c + g.sy) - T_at(c - g.sy)) * 0.5 / dy;
+        const double q_spz = -kappa_0 * temp * (Tp - Tm) * 0.5 / dz;
         const double q_sp2 = q_spx * q_spx + q_spy * q_spy + q_spz * q_spz;
         L = q_fs / sqrt(q_fs2 + q_sp2);
       }

@@ -148,3 +148,25 @@ def test_nan_beside_the_largest_divergence(k):
         want.append(dev.divb())
         dev.close()
     assert want[0] == want[1] > 1.0
+
+
+@pytest.mark.parametrize("e", [1.0e91, 1.0e100])
+def test_limited_flux_beyond_the_range(e):
+    """A conduction whose unlimited flux overflows in two cells: the flux limiter's
+    factor is zero there."""
+    print("\n[case] conduction flux overflow", flush=True)
+    from lare3d_amd.device import Device
+    from oracle.oracle import Oracle
+    grid, params, f, dt = configs.harris_conduction(12, seed=1)
+    params.heat_flux_limiter, params.flux_limiter = 1, 0.1
+    f.energy[6:8, 6, 6] = e
+    out = []
+    for cls in (Device, Oracle):
+        sim = cls(grid, params, f)
+        sim.set_scalars(dt=0.01 * dt)
+        sim.boundary_conditions()
+        sim.conduct_heat()
+        out.append((sim.scalars().n_s_stages, sim.fields().interior("energy")))
+        sim.close()
+    assert out[0][0] == out[1][0] == 3
+    assert np.array_equal(out[0][1], out[1][1], equal_nan=True)

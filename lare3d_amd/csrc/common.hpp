@@ -158,6 +158,13 @@ __device__ __forceinline__ float operator/(float a, const Recip<float> &b) {
   q = fmaf(fmaf(-b.d, q, a), b.y, q);
   return fmaf(fmaf(-b.d, q, a), b.y, q);
 }
+// The same quotient with the zero, infinite and NaN operands of a / b as well.
+__device__ __forceinline__ double over(double a, const Recip<double> &b) {
+  return __builtin_amdgcn_div_fixup(a / b, b.d, a);
+}
+__device__ __forceinline__ float over(float a, const Recip<float> &b) {
+  return __builtin_amdgcn_div_fixupf(a / b, b.d, a);
+}
 // Square root of a positive normal number: the steps of the compiler's
 // correctly rounded root (Goldschmidt's iteration with fused remainders) less
 // its scaling and its cases for zero and infinity.

@@ -166,7 +166,7 @@ __device__ __forceinline__ acc face_flux(const FaceB &b, acc n, acc t1, acc t2, 
                                          acc L, acc kappa_0) {
   const acc modb = b.x * b.x + b.y * b.y + b.z * b.z + (acc)MIN_B;
   tb = dmax(tb, (acc)0.0);
-  return -L * kappa_0 * pow25(tb) * (n * (tg * n + a1 * t1 + a2 * t2) + tg * (acc)MIN_B) / recip(modb);
+  return over(-L * kappa_0 * pow25(tb) * (n * (tg * n + a1 * t1 + a2 * t2) + tg * (acc)MIN_B), recip(modb));
 }
 // average of four values of the FP64 face field, in the reference's order
 __device__ __forceinline__ acc mean4(double a, double b, double c, double d) { return (acc)(0.25 * (a + b + c + d)); }
@@ -248,6 +248,10 @@ __device__ __forceinline__ void map_coord(int c, int n, int user, int olo, int o
 // two, and FP32 four, by themselves).  A stage at 256^3 in FP64: 560 us, with
 // the reciprocals 501, with three waves 457; FP32 373, 363, and with the
 // carried field 294; 64 x 64 x 128 FP64 30.2 -> 26.3.
+// The fluxes, their divergence and 1 / rho keep their infinities (over): the
+// MAX(energy, 0) at the end of a step's conduction makes a NaN zero.  It costs
+// nothing measurable; in the gradients too, whose numerators are differences of
+// temperatures, it would take 9.5 ms for 20 super-steps there to 10.0.
 #define RKL_OUT 63
 #define RKL_WAVES(PI, OPEN) (sizeof(acc) == sizeof(double) && !(PI) && !(OPEN) ? 3 : 1)
 template <int MODE, int FIRST, bool PI, bool OPEN>
@@ -334,20 +338,20 @@ __global__ __launch_bounds__(BX * BY, RKL_WAVES(PI, OPEN)) void k_rkl2_z(Geo g, 
     bzlY = bzY;
     bzlP = bzP;
     if (out) {
-      acc fl = (acc)0.0 + fz_in / recip((acc)g.dzb[k - 1]);
-      fl = fl + fy_in / recip((acc)g.dyb[j - 1]);
-      fl = fl + fx_in / recip((acc)g.dxb[i - 1]);
-      fl = fl - fx_out / recip((acc)g.dxb[i]);
-      fl = fl - fy_out / recip((acc)g.dyb[j]);
-      fl = fl - fz_out / recip((acc)g.dzb[k]);
+      acc fl = (acc)0.0 + over(fz_in, recip((acc)g.dzb[k - 1]));
+      fl = fl + over(fy_in, recip((acc)g.dyb[j - 1]));
+      fl = fl + over(fx_in, recip((acc)g.dxb[i - 1]));
+      fl = fl - over(fx_out, recip((acc)g.dxb[i]));
+      fl = fl - over(fy_out, recip((acc)g.dyb[j]));
+      fl = fl - over(fz_out, recip((acc)g.dzb[k]));
       if (FIRST) {
-        const acc lc = ((acc)1.0 / recip((acc)rho[c0])) * fl;
+        const acc lc = over((acc)1.0, recip((acc)rho[c0])) * fl;
         Lc[c0] = lc;
         const acc cc = (acc)mu_t * tdt * lc;
         Yout[c0] = E0[c0] + cc;
       } else {
         const acc cc0 = (acc)gam_t * tdt * Lc[c0];
-        const acc lj = ((acc)1.0 / recip((acc)rho[c0])) * fl;
+        const acc lj = over((acc)1.0, recip((acc)rho[c0])) * fl;
         const acc cc1 = (acc)mu_t * tdt * lj;
         acc y3;
         if constexpr (sizeof(acc) == sizeof(double)) {

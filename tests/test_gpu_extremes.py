@@ -170,3 +170,24 @@ def test_limited_flux_beyond_the_range(e):
         sim.close()
     assert out[0][0] == out[1][0] == 3
     assert np.array_equal(out[0][1], out[1][1], equal_nan=True)
+
+
+@pytest.mark.parametrize("field,value", [("bx", 1.0e155), ("rho", 1.0e-100)])
+def test_flux_over_an_infinite_field(field, value):
+    """B^2 beyond the range in two cells (no flux), and a density whose energy
+    grows beyond it."""
+    print(f"\n[case] conduction with {field} = {value}", flush=True)
+    from lare3d_amd.device import Device
+    from oracle.oracle import Oracle
+    grid, params, f, dt = configs.harris_conduction(12, seed=1)
+    getattr(f, field)[6:8, 6, 6] = value
+    out = []
+    for cls in (Device, Oracle):
+        sim = cls(grid, params, f)
+        sim.set_scalars(dt=1.0e-4 if field == "bx" else 1.0e-6)
+        sim.boundary_conditions()
+        sim.conduct_heat()
+        out.append((sim.scalars().n_s_stages, sim.fields().interior("energy")))
+        sim.close()
+    assert out[0][0] == out[1][0]
+    assert np.array_equal(out[0][1], out[1][1], equal_nan=True)

@@ -65,7 +65,8 @@ __device__ __forceinline__ double saha_neutral(const NeutralArgs &a, double t_v,
 // the ghosts of Y through the boundary map (an RKL2 stage value whose
 // ghosts were never filled, conduct.f90:400-404; E0 on a BC_OPEN side),
 // rho as stored.  An inverted bracket (the reference's STOP, :172-175)
-// sets *flag.
+// sets *flag, in pinned memory, past the caches: the host looks at it after a
+// later kernel's ticket, when no end of stream has written them back.
 template <int MODE>
 __global__ __launch_bounds__(BX * BY) void k_neutral(Geo g, Box b, const real *__restrict__ Y,
                                                      const real *__restrict__ E0, const real *__restrict__ rho,
@@ -75,7 +76,7 @@ __global__ __launch_bounds__(BX * BY) void k_neutral(Geo g, Box b, const real *_
   const double rho0 = rho[c];
   const double e0 = ghost_read(g, Y, E0, i, j, k, MODE);
   const double ta1 = a.gm1 * dmax((e0 - a.ip) / 2.0, NONE_ZERO), ta2 = a.gm1 * e0;
-  if (ta1 > ta2) *flag = 1;
+  if (ta1 > ta2) __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   double dx = ta2 - ta1, t = ta1, xi_a = 0.0;
   for (int loop = 1; loop <= 100; ++loop) {
     dx = dx / 2.0;

@@ -57,13 +57,12 @@ struct Dev {
   // lagrangian scratch
   real *rho_v, *cs_v, *al1, *al2, *al3, *visc_heat, *p0, *pp;
   double *bpx, *bpy, *bpz;       // predictor B
-  double *fxr, *fyr, *fzr;       // resistive EMFs (CT update of B)
+  double *fxr, *fyr, *fzr;       // spare face arrays: a CT sweep's or resistive substep's new B
   real *qx, *qy, *qz;
-  // remap scratch: F, F2 the CT face fluxes (FP64-sized arrays, holding
-  // the fluxes in the storage type; the potential field's FP64 scratch),
-  // Fe the energy flux
+  // remap scratch: volumes and width (with some Lagrangian arrays: remap_db1,
+  // remap_vol), the mass flux, and where the new energy and velocities go
   real *cv1, *cv2, *db1, *Fe, *dm, *Fx, *Fy, *Fz;
-  double *F, *F2;
+  double *F, *F2;  // the potential field's potential and flux patch
   // conduction scratch
   real *larsen, *Lc, *Yb[3];
   // options: gamma_boris (boris), cool_term_v / cool_term_b and the stored

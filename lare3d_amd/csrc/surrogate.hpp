@@ -199,8 +199,8 @@ struct SurBatch {
 // hash(seed, b) % draw and keeps it in row[]; otherwise row b, and the
 // padding columns zeros.
 // All weights but layer 1's are loaded ahead of the products that need them.
-#define SUR_FB_K 21  // K steps of layer 1 whose loads are issued together
-static_assert((SUR_K / 16) % SUR_FB_K == 0, "layer 1 in whole batches of K steps");
+// The loads of layer 1's SUR_FB_K steps are issued together.
+#define SUR_FB_K (SUR_K / 16)
 __global__ __launch_bounds__(256) void k_sur_fb(SurBatch s, const float *__restrict__ w, int draw,
                                                 unsigned long long seed) {
   __shared__ bf16x4 frag[2][4][64];
@@ -232,21 +232,19 @@ __global__ __launch_bounds__(256) void k_sur_fb(SurBatch s, const float *__restr
   const float tgt = s.y && real_row ? s.y[r] : 0.0f;
   // layer 1
   f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int st = 0; st < SUR_K / 16; st += SUR_FB_K) {
-    float wa[SUR_FB_K][4];
-    float4 xb[SUR_FB_K];
+  float wa[SUR_FB_K][4];
+  float4 xb[SUR_FB_K];
 #pragma unroll
-    for (int q = 0; q < SUR_FB_K; ++q) {
-      const int kb = (st + q) * 16 + kq;
+  for (int q = 0; q < SUR_FB_K; ++q) {
+    const int kb = q * 16 + kq;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) wa[q][t] = w[SUR_OFF_W1 + (kb + t) * SUR_H + f0 + col];
-      xb[q] = real_row ? *(const float4 *)(s.X + (size_t)r * SUR_K + kb) : float4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-#pragma unroll
-    for (int q = 0; q < SUR_FB_K; ++q)
-      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pack4(wa[q][0], wa[q][1], wa[q][2], wa[q][3]),
-                                                      pack4(xb[q].x, xb[q].y, xb[q].z, xb[q].w), acc, 0, 0, 0);
+    for (int t = 0; t < 4; ++t) wa[q][t] = w[SUR_OFF_W1 + (kb + t) * SUR_H + f0 + col];
+    xb[q] = real_row ? *(const float4 *)(s.X + (size_t)r * SUR_K + kb) : float4{0.0f, 0.0f, 0.0f, 0.0f};
   }
+#pragma unroll
+  for (int q = 0; q < SUR_FB_K; ++q)
+    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pack4(wa[q][0], wa[q][1], wa[q][2], wa[q][3]),
+                                                    pack4(xb[q].x, xb[q].y, xb[q].z, xb[q].w), acc, 0, 0, 0);
   float z1[4], h[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {

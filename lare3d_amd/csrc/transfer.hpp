@@ -30,9 +30,6 @@ struct XferSet {
   unsigned long total;
 };
 
-#ifndef XFER_CHUNK
-#define XFER_CHUNK (512 * 1024)  // elements, 4 MiB of pinned memory
-#endif
 // Pinned memory costs about 0.2 ms per MiB to allocate and a thread about
 // 20 us to start, so a small transfer takes small chunks and few threads: a
 // 32nd of the run within XFER_CHUNK_MIN..MAX elements (1/2 and 4 MiB; the

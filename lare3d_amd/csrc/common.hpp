@@ -137,8 +137,8 @@ __device__ __forceinline__ float max0(float x) { return x > 0.0f ? x : 0.0f; }
 // infinite is NaN.  So it divides only where an infinity and a NaN end alike, in
 // a value that the state check of the next step finds: where a minimum, a
 // MAX(., 0) or a comparison would drop a NaN, the division is the plain one or
-// goes through over().  A quotient is 3 (FP32: 5) operations on its critical path
-// instead of 11.  Everywhere with the fix-up of over() and its overflow, 2 more:
+// goes through over() or over_all().  A quotient is 3 (FP32: 5) operations on its
+// critical path instead of 11, and 4 or 5 by these.  over_all() everywhere took
 // 100 steps at 192^3 in FP32 337 -> 350 ms, 256^3 in FP64 996 -> 1009, 20
 // conduction super-steps at 64 x 64 x 128 9.5 -> 10.0.
 template <class A>
@@ -165,13 +165,21 @@ __device__ __forceinline__ float operator/(float a, const Recip<float> &b) {
   q = fmaf(fmaf(-b.d, q, a), b.y, q);
   return fmaf(fmaf(-b.d, q, a), b.y, q);
 }
-// The same quotient with the zero, infinite and NaN operands of a / b as well:
-// the hardware's fix-up, one operation more.
+// The same quotient with the zero, infinite and NaN operands of a / b as well, by
+// the hardware's fix-up, which also sets the sign.
 __device__ __forceinline__ double over(double a, const Recip<double> &b) {
   return __builtin_amdgcn_div_fixup(a / b, b.d, a);
 }
 __device__ __forceinline__ float over(float a, const Recip<float> &b) {
   return __builtin_amdgcn_div_fixupf(a / b, b.d, a);
+}
+// And with the infinity of a quotient beyond the range: the maximum takes the
+// NaN for one, whose sign the fix-up sets.
+__device__ __forceinline__ double over_all(double a, const Recip<double> &b) {
+  return __builtin_amdgcn_div_fixup(__builtin_fmax(a / b, -__builtin_inf()), b.d, a);
+}
+__device__ __forceinline__ float over_all(float a, const Recip<float> &b) {
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaxf(a / b, -__builtin_inff()), b.d, a);
 }
 // Square root of a positive normal number: the steps of the compiler's
 // correctly rounded root (Goldschmidt's iteration with fused remainders) less

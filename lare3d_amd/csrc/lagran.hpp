@@ -502,16 +502,17 @@ __device__ __forceinline__ void vertex_current_vals(double dxc, double dyc, doub
 
 // The same vertex current in the arithmetic type: the differences of the
 // FP64 face field are taken in FP64 and divided by the widths (as reciprocals
-// of dxc, dyc, dzc) in it; for FP64, the quotients of vertex_current_vals.
+// of dxc, dyc, dzc) in it; for FP64, the quotients of vertex_current_vals, with
+// their infinities (over_all), since eta compares the current.
 __device__ __forceinline__ void vertex_current_acc(const Recip<acc> &ax, const Recip<acc> &ay, const Recip<acc> &az,
                                                    const BPlane &lo, const BPlane &hi, double bz0, double bzx,
                                                    double bzy, double bzxy, acc &jx, acc &jy, acc &jz) {
-  const acc jx1 = (acc)(bzy - bz0) / ay - (acc)(hi.by0 - lo.by0) / az;
-  const acc jx2 = (acc)(bzxy - bzx) / ay - (acc)(hi.byx - lo.byx) / az;
-  const acc jy1 = (acc)(hi.bx0 - lo.bx0) / az - (acc)(bzx - bz0) / ax;
-  const acc jy2 = (acc)(hi.bxy - lo.bxy) / az - (acc)(bzxy - bzy) / ax;
-  const acc jz1 = (acc)(lo.byx - lo.by0) / ax - (acc)(lo.bxy - lo.bx0) / ay;
-  const acc jz2 = (acc)(hi.byx - hi.by0) / ax - (acc)(hi.bxy - hi.bx0) / ay;
+  const acc jx1 = over_all((acc)(bzy - bz0), ay) - over_all((acc)(hi.by0 - lo.by0), az);
+  const acc jx2 = over_all((acc)(bzxy - bzx), ay) - over_all((acc)(hi.byx - lo.byx), az);
+  const acc jy1 = over_all((acc)(hi.bx0 - lo.bx0), az) - over_all((acc)(bzx - bz0), ax);
+  const acc jy2 = over_all((acc)(hi.bxy - lo.bxy), az) - over_all((acc)(bzxy - bzy), ax);
+  const acc jz1 = over_all((acc)(lo.byx - lo.by0), ax) - over_all((acc)(lo.bxy - lo.bx0), ay);
+  const acc jz2 = over_all((acc)(hi.byx - hi.by0), ax) - over_all((acc)(hi.bxy - hi.bx0), ay);
   jx = (jx1 + jx2) * (acc)0.5;
   jy = (jy1 + jy2) * (acc)0.5;
   jz = (jz1 + jz2) * (acc)0.5;

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from lare3d_amd import configs
-from lare3d_amd.abi import DeviceError
+from lare3d_amd.abi import DeviceError, PREC_FP32
 from tests.test_zz_no_alloc import _noalloc
 
 pytestmark = pytest.mark.gpu
@@ -191,3 +191,27 @@ def test_flux_over_an_infinite_field(field, value):
         sim.close()
     assert out[0][0] == out[1][0]
     assert np.array_equal(out[0][1], out[1][1], equal_nan=True)
+
+
+@pytest.mark.parametrize("precision,b", [(0, 1.7e308), (PREC_FP32, 1.0e39)])
+def test_infinite_current_is_above_the_threshold(precision, b):
+    """Currents beyond the range (the difference or its quotient) are above j_max:
+    eta is eta_background + eta0 at their nodes, as the restatement has it."""
+    print(f"\n[case] infinite current precision={precision}", flush=True)
+    from lare3d_amd.device import Device
+    from oracle.oracle import Oracle
+    grid, params, f = configs.harris(12)
+    params.eta_background, params.eta0 = 1.0 / 1024, 1.0 / 64  # values that FP32 holds
+    params.j_max = 1.0e30
+    f.bx[6, 6, 6] = b  # over the 2/3 of a cell in y
+    orc = Oracle(grid, params, f)
+    params.precision = precision
+    dev = Device(grid, params, f)
+    eta = []
+    for sim in (dev, orc):
+        sim.boundary_conditions()
+        sim.eta_calc()
+        eta.append(sim.fields().eta)
+        sim.close()
+    assert np.array_equal(eta[0], eta[1], equal_nan=True)
+    assert (eta[1] > 1.0 / 64).any() and (eta[1] < 1.0 / 64).any()

@@ -1301,13 +1301,19 @@ __global__ __launch_bounds__(BX * BY) void k_mom_remap(Geo g, MomArgs a) {
 // The momentum remap and the CT sweep of one sweep in one launch: neither
 // reads what the other writes, and on small grids each leaves most of the chip
 // idle behind its chains of loads.  The first blocks take the momentum remap
-// (an x sweep's block two of its tiles), the rest the CT sweep.
+// (an x sweep's block two of its tiles, so that there the order of xcd_tile
+// alternates between two XCDs), the rest the CT sweep.
 //
 // Runs with the two apart and together: 64^3 30.3 -> 29.0 ms (100 steps),
 // 97 x 61 x 130 37.9 -> 36.9 (50), 64 x 64 x 128 FP32 27.5 -> 26.6 (50),
 // 45 x 37 x 41 9.9 -> 9.4 (30).  Where both fill the chip FP32 still gains, by the
 // tail of one under the head of the other (192^3 339.4 -> 337.4 ms), and FP64,
-// at the bandwidth of a copy in both, does not (256^3 1003.8 -> 1006.8).
+// at the bandwidth of a copy in both, does not (256^3 1003.8 -> 1006.8).  The
+// sheet's step on cubes in FP64, apart and together, in ms: 96^3 0.640 and 0.623,
+// 128^3 1.357 and 1.318, 150^3 2.157 and 2.126, 176^3 3.305 and 3.283, 192^3 4.231
+// and 4.218, 208^3 5.159 and 5.159, 256^3 9.129 and 9.162 (three runs each agree to
+// 0.1%).  So the two are alike at 208^3; the line is crossed at 145 (y and z sweeps)
+// to 178 (x) cells a side, where apart costs 1.4 to 0.7%.
 #define MOM_CT_BLOCKS 4096
 static inline bool mom_ct_together(unsigned blocks) {
   return sizeof(acc) == sizeof(float) || blocks <= MOM_CT_BLOCKS;

@@ -608,7 +608,8 @@ int sweep_full(double dt, int q) {
   // the momentum remap's box and grid; it goes together with the CT sweep, whose
   // turn may come anywhere between the geometry and the boundary fill.  Apart,
   // the CT sweep comes first, so that the mass kernel finds the velocity and
-  // the width in the cache (100 steps at 256^3 995 -> 992 ms).
+  // the width in the cache (100 steps at 256^3 995 -> 992 ms, hardly more than
+  // such runs differ by).
   Box xb = full_box();
   dim3 mg;
   if constexpr (AX == 0) {
@@ -1090,7 +1091,7 @@ int lagrangian_step(bool xi_known) {
     S.dt = dt_full;
     if (rc) return rc;
     // the predictor energy and pressure were formed in the predictor
-    // remap's last geometry pass
+    // remap's geometry pass
     LAUNCH("force", k_force<false>, zchunk_grid(nb), box_block(), S.g, nb, S.vx, S.vy, S.vz, S.pp,
            S.bpx, S.bpy, S.bpz, S.rho_v, S.al1, S.al2, S.al3, S.gamma_boris, S.vx1, S.vy1, S.vz1, S.dt2, S.cv1,
            nullptr, nullptr, nullptr, wall);

@@ -4,12 +4,12 @@
 // For callers that cannot call hipMalloc (code under HIP graph capture,
 // tight serving loops, harnesses that forbid it).  The kernels are those of
 // lare_dev_energy_account (k_energy with the Fortran layout, then the same
-// two-level fold of the per-block partials), so the results are the same
+// fold of the per-block partials, in one level or two), so the results are the same
 // bits for the same field values.  Instead of the partial buffer that
 // lare_dev_init allocates, they use `scratch`, a fixed array in device
 // memory that each GPU holds from the library's load to the end of the
 // process:
-//   [0, NA_MET)            dxb, dyb, dzb copied from the host grid
+//   [0, NA_MET)            dxb, dyb, dzb of the host grid
 //   [NA_MET, +NA_PART)     per-block partial sums, 4 doubles per block
 //   [.., +NA_LEVEL1)       level-1 results of the fold
 //   [.., +NA_OUT)          the four final sums

@@ -1497,6 +1497,8 @@ int api_set_scalars(const lare_scalars *in) {
   S.first_set_dt = in->first_set_dt;
   S.step = in->step;
   double acc[2] = {in->total_visc_heating, in->total_ohmic_heating};
+  // a step returns before its last folds have run, and they write the mirror too
+  HIPCHK(hipStreamSynchronize(S.stream));
   HIPCHK(hipMemcpy(S.dscal + 8, acc, sizeof(acc), hipMemcpyHostToDevice));
   S.hscal[8] = acc[0];
   S.hscal[9] = acc[1];
